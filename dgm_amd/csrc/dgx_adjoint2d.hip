@@ -217,8 +217,8 @@ __global__ void __launch_bounds__(64) k_adjtraces2(AdjArgs a) {
   }
   __syncthreads();
   double *Le = a.Lt + (size_t)e * 4 * NF * QF;
-  contract<NF, L, L, 2, 2, NT>(CT<P>::Bend(), A, Kb, tid);   // [NF][L][2]: edges 0 / 2
-  contract<NF, L, L, 1, 2, NT>(CT<P>::Bend(), A, Ka, tid);   // [NF][2][L]: edges 3 / 1
+  contract<NF, L, L, 2, 2, NT>(EO<P>::Bend(), A, Kb, tid);   // [NF][L][2]: edges 0 / 2
+  contract<NF, L, L, 1, 2, NT>(EO<P>::Bend(), A, Ka, tid);   // [NF][2][L]: edges 3 / 1
   __syncthreads();
   contract<NF, L, 2, 1, QF, NT>(AT<P>::PWt(), Kb, O, tid);   // [NF][QF][2]
   __syncthreads();
@@ -253,9 +253,9 @@ __global__ void __launch_bounds__(64) k_vjp2(AdjArgs a) {
     M[i] = a.U[((size_t)v * ne + e) * L2 + (i - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 1, Q, NT>(CT<P>::BT(), M, X, tid);   // [NF][Q][L]
+  contract<NF, L, L, 1, Q, NT>(EO<P>::BT(), M, X, tid);   // [NF][Q][L]
   __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(CT<P>::BT(), X, N1, tid);  // [NF][Q][Q]
+  contract<NF, Q, L, 2, Q, NT>(EO<P>::BT(), X, N1, tid);  // [NF][Q][Q]
   __syncthreads();
   double un[NPT][NF];
 #pragma unroll

@@ -253,6 +253,24 @@ int upload_all_tables() {
       std::copy(t->begin(), t->end(), packed.begin() + off);
       off += t->size();
     }
+    // halves of the symmetric matrices (dgx_device.hpp: EOx)
+    auto rows = [&](const std::vector<double> &M, int nr, int ni, int odd) {   // points -> modes
+      for (int l = 0; l < nr; ++l) {
+        const double s = (l + odd) % 2 ? -1.0 : 1.0;
+        for (int i = 0; i < dgx::half_up(ni); ++i)
+          packed[off++] = 0.5 * (M[l * ni + i] + s * M[l * ni + ni - 1 - i]);
+      }
+    };
+    auto square = [&](const std::vector<double> &M, int no, int ni) {          // points -> points
+      for (int o = 0; o < dgx::half_up(no); ++o) {
+        for (int i = 0; i < dgx::half_up(ni); ++i)
+          packed[off++] = 2 * i + 1 == ni ? M[o * ni + i] : 0.5 * (M[o * ni + i] + M[o * ni + ni - 1 - i]);
+        for (int i = 0; i < ni / 2; ++i) packed[off++] = 0.5 * (M[o * ni + i] - M[o * ni + ni - 1 - i]);
+      }
+    };
+    const int L = b.L, Q = b.Q, QF = b.QF;
+    rows(b.BW, L, Q, 0); rows(b.QD, L, Q, 1); rows(b.PI, L, Q, 0); rows(b.BL, L, Q, 0); rows(b.PW, L, QF, 0);
+    square(b.Ig, QF, Q); square(b.GL, Q, QF); square(b.D, Q, Q); square(b.NP1, Q, Q); square(b.NPD, Q, Q);
     if (off != (size_t)dgx::tab_offset(p) + dgx::tab_size(p)) return fail(DGX_ERR_ARGUMENT, "table layout");
   }
   hipError_t e;

@@ -40,9 +40,9 @@ k_cfl2(CflArgs a) {
   }
   __syncthreads();
   // modal -> GLL nodes, all fields at once: [NF][L][L] -> [NF][Q][L] -> [NF][Q][Q]
-  contract<NF, L, L, 1, Q, NT>(CT<P>::BT(), A, X, tid);
+  contract<NF, L, L, 1, Q, NT>(EO<P>::BT(), A, X, tid);
   __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(CT<P>::BT(), X, O, tid);
+  contract<NF, Q, L, 2, Q, NT>(EO<P>::BT(), X, O, tid);
   __syncthreads();
   const double g = a.gamma;
   double m = 0.0;

@@ -1,7 +1,7 @@
 // FP64 sum-factorization contractions over LDS tensors, shared by the fused
-// hex kernels.  One thread owns one pencil at a time and computes a chunk of
-// outputs from its inputs; chunks are outermost so that only a chunk of
-// coefficient rows (constant memory, scalar registers) is live at a time.
+// hex kernels.  One thread owns one pencil at a time and computes all of its
+// outputs with the even-odd form of the matrix (dgx_device.hpp), whose
+// coefficients come from constant memory as scalar operands.
 #pragma once
 #include "dgx_device.hpp"
 
@@ -19,66 +19,45 @@ template <int V> struct IC { static constexpr int value = V; };
 constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
 
-// Coefficient rows per pass (about 40 doubles live in scalar registers).
-template <int NI> constexpr int out_chunk() { return NI * 3 <= 40 ? 3 : 2; }
-
-// [A][N][B][C] (last-dim pitch PI) -> [A][NO][B][C] (pitch PO), contracting N.
-// When every thread owns at most one pencil (NP <= NT), the pencil's inputs
-// are read from LDS once and all output chunks are computed from registers;
-// otherwise the chunks are outermost (inputs re-read per chunk) so that only
-// one chunk of coefficient rows is live in scalar registers across the
-// pencil loop.  Both orders give bitwise the same sums.
-template <int A, int N, int B, int C, int NO, int PI, int PO, int NT, bool ACC = false>
-__device__ __forceinline__ void con_mid(const double *__restrict__ M, const double *in,
-                                        double *out, int tid) {
-  constexpr int NP = A * B * C, OC = out_chunk<N>();
-  auto pencil = [&](int pc, int o0, int o1) {
+// [A][N][B][C] (last-dim pitch PI) -> [A][NO][B][C] (pitch PO), contracting N
+// with an even-odd matrix; one thread computes all outputs of a pencil.
+template <int A, int N, int B, int C, int NO, int PI, int PO, int NT, bool ACC = false, int K>
+__device__ __forceinline__ void con_mid(EoMat<K, double> M, const double *in, double *out, int tid) {
+  constexpr int NP = A * B * C;
+  auto pencil = [&](int pc) {
     const int c = pc % C, t = pc / C, b = t % B, a = t / B;
-    double x[N];
+    double x[N], y[NO];
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = in[((a * N + i) * B + b) * PI + c];
+    eo_apply<K, N, NO>(M.h, x, y);
 #pragma unroll
-    for (int o = o0; o < o1; ++o) {
-      double s = 0.0;
-#pragma unroll
-      for (int i = 0; i < N; ++i) s = fma(M[o * N + i], x[i], s);
+    for (int o = 0; o < NO; ++o) {
       double *dst = out + ((a * NO + o) * B + b) * PO + c;
-      if (ACC) *dst += s; else *dst = s;
+      if (ACC) *dst += y[o]; else *dst = y[o];
     }
   };
   if constexpr (NP <= NT) {
-    if (tid < NP) pencil(tid, 0, NO);
+    if (tid < NP) pencil(tid);
   } else {
-#pragma unroll
-    for (int o0 = 0; o0 < NO; o0 += OC)
-      for (int pc = tid; pc < NP; pc += NT) pencil(pc, o0, o0 + OC < NO ? o0 + OC : NO);
+    for (int pc = tid; pc < NP; pc += NT) pencil(pc);
   }
 }
 
-// [R][NI] (pitch PI) -> [R][NO] (pitch PO), contracting the last dimension
-// (loop order as in con_mid).
-template <int R, int NI, int NO, int PI, int PO, int NT>
-__device__ __forceinline__ void con_last(const double *__restrict__ M, const double *in, double *out,
-                                         int tid) {
-  constexpr int OC = out_chunk<NI>();
-  auto pencil = [&](int r, int o0, int o1) {
-    double x[NI];
+// [R][NI] (pitch PI) -> [R][NO] (pitch PO), contracting the last dimension.
+template <int R, int NI, int NO, int PI, int PO, int NT, int K>
+__device__ __forceinline__ void con_last(EoMat<K, double> M, const double *in, double *out, int tid) {
+  auto pencil = [&](int r) {
+    double x[NI], y[NO];
 #pragma unroll
     for (int i = 0; i < NI; ++i) x[i] = in[r * PI + i];
+    eo_apply<K, NI, NO>(M.h, x, y);
 #pragma unroll
-    for (int o = o0; o < o1; ++o) {
-      double s = 0.0;
-#pragma unroll
-      for (int i = 0; i < NI; ++i) s = fma(M[o * NI + i], x[i], s);
-      out[r * PO + o] = s;
-    }
+    for (int o = 0; o < NO; ++o) out[r * PO + o] = y[o];
   };
   if constexpr (R <= NT) {
-    if (tid < R) pencil(tid, 0, NO);
+    if (tid < R) pencil(tid);
   } else {
-#pragma unroll
-    for (int o0 = 0; o0 < NO; o0 += OC)
-      for (int r = tid; r < R; r += NT) pencil(r, o0, o0 + OC < NO ? o0 + OC : NO);
+    for (int r = tid; r < R; r += NT) pencil(r);
   }
 }
 

@@ -72,9 +72,9 @@ __device__ void curved_project2(double *Fw, double *S1, double *S2, double *AP, 
   constexpr int L = P + 1, Q = P + 2, L2 = L * L, Q2 = Q * Q;
   constexpr int NW = NT / 64, NML = (NF * L2 + NT - 1) / NT;
   // b = B^T (wJ f): into AP (compact [NF][L2])
-  contract<NF, Q, Q, 1, L, NT>(CT<P>::BL(), Fw, S1, tid);   // [NF][L][Q]
+  contract<NF, Q, Q, 1, L, NT>(EO<P>::BL(), Fw, S1, tid);   // [NF][L][Q]
   __syncthreads();
-  contract<NF, L, Q, 2, L, NT>(CT<P>::BL(), S1, AP, tid);   // [NF][L][L]
+  contract<NF, L, Q, 2, L, NT>(EO<P>::BL(), S1, AP, tid);   // [NF][L][L]
   __syncthreads();
   if (cf) {
     // M x = b with the element's Cholesky factor M = C C^T (rows of C packed),
@@ -132,15 +132,15 @@ __device__ void curved_project2(double *Fw, double *S1, double *S2, double *AP, 
   }
   field_dots2<NF, NW>(part, red, bb, tid);
   auto mass = [&]() {   // AP = B^T diag(wJ) B Pv
-    contract<NF, L, L, 1, Q, NT>(CT<P>::BT(), Pv, S1, tid);   // [NF][Q][L]
+    contract<NF, L, L, 1, Q, NT>(EO<P>::BT(), Pv, S1, tid);   // [NF][Q][L]
     __syncthreads();
-    contract<NF, Q, L, 2, Q, NT>(CT<P>::BT(), S1, S2, tid);   // [NF][Q][Q]
+    contract<NF, Q, L, 2, Q, NT>(EO<P>::BT(), S1, S2, tid);   // [NF][Q][Q]
     __syncthreads();
     for (int i = tid; i < NF * Q2; i += NT) S2[i] *= ge[4 * Q2 + (i % Q2)];
     __syncthreads();
-    contract<NF, Q, Q, 1, L, NT>(CT<P>::BL(), S2, S1, tid);   // [NF][L][Q]
+    contract<NF, Q, Q, 1, L, NT>(EO<P>::BL(), S2, S1, tid);   // [NF][L][Q]
     __syncthreads();
-    contract<NF, L, Q, 2, L, NT>(CT<P>::BL(), S1, AP, tid);   // [NF][L][L]
+    contract<NF, L, Q, 2, L, NT>(EO<P>::BL(), S1, AP, tid);   // [NF][L][L]
     __syncthreads();
   };
   mass();
@@ -228,7 +228,7 @@ __device__ void curved_project2(double *Fw, double *S1, double *S2, double *AP, 
 template <int P, int NF, int NT>
 __device__ __forceinline__ void lift_edges2(const double *gF, double *S1, double *Fw, const double *ge, int tid) {
   constexpr int Q = P + 2, Q2 = Q * Q, QF = P + 1, NPT = (Q2 + NT - 1) / NT;
-  contract<4 * NF, QF, 1, 1, Q, NT>(CT<P>::GL(), gF, S1, tid);   // [NF 4][Q]
+  contract<4 * NF, QF, 1, 1, Q, NT>(EO<P>::GL(), gF, S1, tid);   // [NF 4][Q]
   __syncthreads();
   const double wend = CT<P>::BW()[0] / CT<P>::BT()[0];   // GLL end weight: phi_0 w_0 / phi_0
 #pragma unroll
@@ -256,9 +256,9 @@ __device__ __forceinline__ void lift_edges2(const double *gF, double *S1, double
 template <int P, int NF, int NT>
 __device__ __forceinline__ void nodal2(const double *M, double *S, double *Out, int tid) {
   constexpr int L = P + 1, Q = P + 2;
-  contract<NF, L, L, 1, Q, NT>(CT<P>::BT(), M, S, tid);   // [NF][Q][L]
+  contract<NF, L, L, 1, Q, NT>(EO<P>::BT(), M, S, tid);   // [NF][Q][L]
   __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(CT<P>::BT(), S, Out, tid);   // [NF][Q][Q]
+  contract<NF, Q, L, 2, Q, NT>(EO<P>::BT(), S, Out, tid);   // [NF][Q][Q]
   __syncthreads();
 }
 
@@ -324,9 +324,9 @@ k_rhs2c(CurvedArgs a) {
     S1[i] = a.U[((size_t)v * ne + e) * L2 + (i - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 1, Q, NT>(CT<P>::BT(), S1, S2, tid);   // [NF][Q][L]
+  contract<NF, L, L, 1, Q, NT>(EO<P>::BT(), S1, S2, tid);   // [NF][Q][L]
   __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(CT<P>::BT(), S2, Un, tid);   // [NF][Q][Q]
+  contract<NF, Q, L, 2, Q, NT>(EO<P>::BT(), S2, Un, tid);   // [NF][Q][Q]
 
   // edge corrections g = (J_side/J_vol)(Fhat - F(U-).n) at the Gauss points
   bool bad = false;
@@ -580,7 +580,7 @@ k_visc2c(CurvedArgs a) {
     for (int c = 0; c < 6; ++c) Lay[(s * 6 + c) * Q + j] = Fv[c * Q2 + k];
   }
   __syncthreads();
-  contract<1, 24, Q, 2, QF, NT>(CT<P>::Ig(), Lay, Wf, tid);
+  contract<1, 24, Q, 2, QF, NT>(EO<P>::Ig(), Lay, Wf, tid);
   __syncthreads();
   for (int i = tid; i < 4 * 3 * QF; i += NT) {
     const int s = i / (3 * QF), r = i - s * 3 * QF, c = r / QF, q = r - c * QF;

@@ -25,15 +25,17 @@ namespace dgx {
 
 // Float copies of the basis tables for the mixed residual (FP32 contractions
 // and derivatives; FP64 metrics, fluxes, state and the mass solve), filled
-// beside c_tab at upload.  TB3<R, P> gives the tables of arithmetic type R.
+// beside c_tab at upload.  TE3<R, P> and TB3<R, P> give the tables of
+// arithmetic type R.
 static __constant__ float c_tabf3[kTabTotal];
+struct EoBaseF3 {
+  using R = float;
+  __device__ static __forceinline__ const float *base() { return c_tabf3; }
+};
+template <typename R, int P> using TE3 = EOx<std::conditional_t<std::is_same<R, double>::value, EoBaseD, EoBaseF3>, P>;
 template <typename R, int P> struct TB3;
 template <int P> struct TB3<double, P> : CT<P> {};
 template <int P> struct TB3<float, P> {
-  static constexpr int L = P + 1, Q = P + 2, QF = P + 1, b = tab_offset(P);
-  __device__ static __forceinline__ const float *BT() { return c_tabf3 + b; }
-  __device__ static __forceinline__ const float *BL() { return c_tabf3 + (CT<P>::BL() - c_tab); }
-  __device__ static __forceinline__ const float *GL() { return c_tabf3 + (CT<P>::GL() - c_tab); }
   __device__ static __forceinline__ const float *DN() { return c_tabf3 + (CT<P>::DN() - c_tab); }
 };
 
@@ -59,8 +61,8 @@ template <int P> struct C3 {
 };
 
 // [NF][N]^3 blocks (compact) through matrix M [NO][N] along all three dimensions
-template <int NF, int N, int NO, int NT, typename T>
-__device__ __forceinline__ void chain3(const T *M, const T *in, T *s1, T *s2, T *out, int tid) {
+template <int NF, int N, int NO, int NT, int K, typename T>
+__device__ __forceinline__ void chain3(EoMat<K, T> M, const T *in, T *s1, T *s2, T *out, int tid) {
   contract<NF, N, N * N, 1, NO, NT>(M, in, s1, tid);             // [NF][NO][N N]
   __syncthreads();
   contract<NF * NO, N, N, 1, NO, NT>(M, s1, s2, tid);            // [NF NO][NO][N]
@@ -97,19 +99,19 @@ template <int P, int NT, int NF>
 __device__ __forceinline__ void mass_apply(const double *Pv, double *AP, double *S1, double *S2, const double *ge,
                                            int tid) {
   constexpr int L = P + 1, Q = P + 2, Q3 = Q * Q * Q;
-  contract<NF, L, L * L, 1, Q, NT>(CT<P>::BT(), Pv, S1, tid);        // [NF][Q][L L]
+  contract<NF, L, L * L, 1, Q, NT>(EO<P>::BT(), Pv, S1, tid);        // [NF][Q][L L]
   __syncthreads();
-  contract<NF * Q, L, L, 1, Q, NT>(CT<P>::BT(), S1, S2, tid);        // [NF Q][Q][L]
+  contract<NF * Q, L, L, 1, Q, NT>(EO<P>::BT(), S1, S2, tid);        // [NF Q][Q][L]
   __syncthreads();
-  contract<NF * Q * Q, L, 1, 1, Q, NT>(CT<P>::BT(), S2, S1, tid);    // nodal [NF][Q3]
+  contract<NF * Q * Q, L, 1, 1, Q, NT>(EO<P>::BT(), S2, S1, tid);    // nodal [NF][Q3]
   __syncthreads();
   for (int i = tid; i < NF * Q3; i += NT) S1[i] *= ge[9 * Q3 + (i % Q3)];
   __syncthreads();
-  contract<NF, Q, Q * Q, 1, L, NT>(CT<P>::BL(), S1, S2, tid);        // [NF][L][Q Q]
+  contract<NF, Q, Q * Q, 1, L, NT>(EO<P>::BL(), S1, S2, tid);        // [NF][L][Q Q]
   __syncthreads();
-  contract<NF * L, Q, Q, 1, L, NT>(CT<P>::BL(), S2, S1, tid);        // [NF L][L][Q]
+  contract<NF * L, Q, Q, 1, L, NT>(EO<P>::BL(), S2, S1, tid);        // [NF L][L][Q]
   __syncthreads();
-  contract<NF * L * L, Q, 1, 1, L, NT>(CT<P>::BL(), S1, AP, tid);    // [NF][L3]
+  contract<NF * L * L, Q, 1, 1, L, NT>(EO<P>::BL(), S1, AP, tid);    // [NF][L3]
   __syncthreads();
 }
 
@@ -346,7 +348,7 @@ k_rhs3c(CurvedArgs a) {
     if (i < 5 * L3) S1r[i] = (R)um[k];
   }
   __syncthreads();
-  chain3<5, L, Q, NT>(TB3<R, P>::BT(), S1r, Fr, S1r, S2r, tid);
+  chain3<5, L, Q, NT>(TE3<R, P>::BT(), S1r, Fr, S1r, S2r, tid);
   const R *Un = S2r;
 
   // volume: wJ * sum_x sum_d (dxi_d/dx_x) D_d F_x at every node, field by
@@ -404,9 +406,9 @@ k_rhs3c(CurvedArgs a) {
   }
   __syncthreads();
   // faces: Gauss -> GLL face nodes for 30 blocks, then wJ / w_end at the face nodes
-  contract<30, QF, QF, 1, Q, NT>(TB3<R, P>::GL(), gF, S1r, tid);   // [30][Q][QF]
+  contract<30, QF, QF, 1, Q, NT>(TE3<R, P>::GL(), gF, S1r, tid);   // [30][Q][QF]
   __syncthreads();
-  contract<30, Q, QF, 2, Q, NT>(TB3<R, P>::GL(), S1r, S2r, tid);    // [30][Q][Q]
+  contract<30, Q, QF, 2, Q, NT>(TE3<R, P>::GL(), S1r, S2r, tid);    // [30][Q][Q]
   __syncthreads();
   {
     const double wend = CT<P>::BW()[0] / CT<P>::BT()[0];   // GLL end weight: phi_0 w_0 / phi_0
@@ -435,7 +437,7 @@ k_rhs3c(CurvedArgs a) {
   __syncthreads();
   }   // !PROJ
   // b = B^T (wJ f): into Bv (compact [5][L3], the face-term region, free now)
-  chain3<5, Q, L, NT>(TB3<R, P>::BL(), Fr, S1r, S2r, Bvr, tid);
+  chain3<5, Q, L, NT>(TE3<R, P>::BL(), Fr, S1r, S2r, Bvr, tid);
   // the mass solve: Pv (compact [5][L3]) reuses Fw; totals after the reductions.
   // The update's RK register is loaded first: the solve's barriers cover it.
   double x[NML], utin[NML];
@@ -574,7 +576,7 @@ k_grad3c(CurvedArgs a) {
     S1[i] = a.U[((size_t)v * ne + e) * L3 + (i - v * L3)];
   }
   __syncthreads();
-  chain3<5, L, Q, NT>(CT<P>::BT(), S1, S2, S1, Pq, tid);
+  chain3<5, L, Q, NT>(EO<P>::BT(), S1, S2, S1, Pq, tid);
   double mg[NPT][9];
 #pragma unroll
   for (int rr = 0; rr < NPT; ++rr) {
@@ -620,9 +622,9 @@ k_grad3c(CurvedArgs a) {
       S2[i] = a.fgeo[(((size_t)e * 6 + s) * QF2 + q) * 4 + x] * Jq[(c * 6 + s) * QF2 + q];
     }
     __syncthreads();
-    contract<6 * NG, QF, QF, 1, Q, NT>(CT<P>::GL(), S2, S1, tid);   // [6 NG][Q][QF]
+    contract<6 * NG, QF, QF, 1, Q, NT>(EO<P>::GL(), S2, S1, tid);   // [6 NG][Q][QF]
     __syncthreads();
-    contract<6 * NG, Q, QF, 2, Q, NT>(CT<P>::GL(), S1, S2, tid);    // [6 NG][Q][Q]
+    contract<6 * NG, Q, QF, 2, Q, NT>(EO<P>::GL(), S1, S2, tid);    // [6 NG][Q][Q]
     __syncthreads();
 #pragma unroll
     for (int rr = 0; rr < NPT; ++rr) {
@@ -645,7 +647,7 @@ k_grad3c(CurvedArgs a) {
     }
     __syncthreads();
     // b = B^T (wJ g), then M x = b
-    chain3<NG, Q, L, NT>(CT<P>::BL(), Fw, S1, S2, Bv, tid);
+    chain3<NG, Q, L, NT>(EO<P>::BL(), Fw, S1, S2, Bv, tid);
     double bvec[ML], x[ML];
 #pragma unroll
     for (int k = 0; k < ML; ++k) {
@@ -684,13 +686,13 @@ k_visc3c(CurvedArgs a) {
     S1[i] = a.U[((size_t)v * ne + e) * L3 + (i - v * L3)];
   }
   __syncthreads();
-  chain3<5, L, Q, NT>(CT<P>::BT(), S1, S2, S1, Un, tid);
+  chain3<5, L, Q, NT>(EO<P>::BT(), S1, S2, S1, Un, tid);
   // the 12 gradient components at this thread's nodes
   double gq[NPT][12];
   for (int c = 0; c < 4; ++c) {
     for (int i = tid; i < 3 * L3; i += NT) S1[i] = a.G[((size_t)e * 12 + 3 * c) * L3 + i];
     __syncthreads();
-    chain3<3, L, Q, NT>(CT<P>::BT(), S1, S2, S1, Fc, tid);
+    chain3<3, L, Q, NT>(EO<P>::BT(), S1, S2, S1, Fc, tid);
 #pragma unroll
     for (int rr = 0; rr < NPT; ++rr) {
       const int n = tid + rr * NT;
@@ -776,9 +778,9 @@ k_visc3c(CurvedArgs a) {
       S1[i] = Fc[x * Q3 + n];
     }
     __syncthreads();
-    contract<18, Q, Q, 1, QF, NT>(CT<P>::Ig(), S1, S2, tid);    // [18][QF][Q]
+    contract<18, Q, Q, 1, QF, NT>(EO<P>::Ig(), S1, S2, tid);    // [18][QF][Q]
     __syncthreads();
-    contract<18, QF, Q, 2, QF, NT>(CT<P>::Ig(), S2, S1, tid);   // [18][QF][QF]
+    contract<18, QF, Q, 2, QF, NT>(EO<P>::Ig(), S2, S1, tid);   // [18][QF][QF]
     __syncthreads();
     for (int i = tid; i < 6 * QF2; i += NT) {
       const int s = i / QF2, q = i - s * QF2;

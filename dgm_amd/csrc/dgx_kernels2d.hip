@@ -11,6 +11,7 @@
 #include <hip/hip_cooperative_groups.h>
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 #include "dgx_kernels.hpp"
@@ -34,6 +35,12 @@ template <int P> struct TB<float, P> {
   __device__ static __forceinline__ const float *PW() { return c_tabf + b + 3 * Q * L + QF * L + 2 * L; }
 };
 
+struct EoBaseF {
+  using R = float;
+  __device__ static __forceinline__ const float *base() { return c_tabf; }
+};
+template <typename R, int P> using TE = EOx<std::conditional_t<std::is_same<R, double>::value, EoBaseD, EoBaseF>, P>;
+
 template <int P> struct H2 {
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1;
   static constexpr int L2 = L * L, Q2 = Q * Q;
@@ -44,9 +51,9 @@ template <int P>
 __device__ __forceinline__ void backward2(const Tab &tb, const double *m, double *s1, double *out,
                                           int tid) {
   constexpr int L = H2<P>::L, Q = H2<P>::Q, NT = H2<P>::NT;
-  contract<1, L, L, 1, Q, NT>(CT<P>::BT(), m, s1, tid);
+  contract<1, L, L, 1, Q, NT>(EO<P>::BT(), m, s1, tid);
   __syncthreads();
-  contract<1, Q, L, 2, Q, NT>(CT<P>::BT(), s1, out, tid);
+  contract<1, Q, L, 2, Q, NT>(EO<P>::BT(), s1, out, tid);
   __syncthreads();
 }
 
@@ -69,8 +76,8 @@ __device__ __forceinline__ void traces2_core(const double *__restrict__ U, doubl
     A[i] = (R)U[((size_t)v * ne + e) * L2 + (i - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 2, 2, NT>(TB<R, P>::Bend(), A, Kb, tid);   // [NF][L][2]
-  contract<NF, L, L, 1, 2, NT>(TB<R, P>::Bend(), A, Ka, tid);   // [NF][2][L]
+  contract<NF, L, L, 2, 2, NT>(TE<R, P>::Bend(), A, Kb, tid);   // [NF][L][2]
+  contract<NF, L, L, 1, 2, NT>(TE<R, P>::Bend(), A, Ka, tid);   // [NF][2][L]
   __syncthreads();
   contract<NF, L, 2, 1, QF, NT>(TB<R, P>::Bg(), Kb, O, tid);    // [NF][QF][2]: edges 0 / 2
   __syncthreads();
@@ -132,9 +139,9 @@ __device__ __forceinline__ void load_nodal2(const double *__restrict__ U, int ne
     M[i] = (R)U[((size_t)v * ne + e) * L2 + (i - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 1, Q, NT>(TB<R, P>::BT(), M, X, tid);   // [NF][Q][L]
+  contract<NF, L, L, 1, Q, NT>(TE<R, P>::BT(), M, X, tid);   // [NF][Q][L]
   __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(TB<R, P>::BT(), X, N, tid);   // [NF][Q][Q]
+  contract<NF, Q, L, 2, Q, NT>(TE<R, P>::BT(), X, N, tid);   // [NF][Q][Q]
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < NPT; ++r) {
@@ -150,13 +157,13 @@ template <int P, int NF, typename R = double>
 __device__ __forceinline__ void divergence2(R *M, R *X1, R *X2, R *N1, R *N2, const R *gF, R *H, int tid) {
   using F = H2F<P, NF>;
   constexpr int L = F::L, Q = F::Q, QF = F::QF, NT = 64;
-  contract<NF, Q, Q, 2, L, NT>(TB<R, P>::BW(), N1, X1, tid);
-  contract<NF, Q, Q, 2, L, NT>(TB<R, P>::QD(), N2, X2, tid);
+  contract<NF, Q, Q, 2, L, NT>(TE<R, P>::BW(), N1, X1, tid);
+  contract<NF, Q, Q, 2, L, NT>(TE<R, P>::QD(), N2, X2, tid);
   contract<NF, 4, QF, 2, L, NT>(TB<R, P>::PW(), gF, H, tid);
   __syncthreads();
-  contract<NF, Q, L, 1, L, NT>(TB<R, P>::QD(), X1, M, tid);
+  contract<NF, Q, L, 1, L, NT>(TE<R, P>::QD(), X1, M, tid);
   __syncthreads();
-  contract<NF, Q, L, 1, L, NT, true>(TB<R, P>::BW(), X2, M, tid);
+  contract<NF, Q, L, 1, L, NT, true>(TE<R, P>::BW(), X2, M, tid);
   __syncthreads();
 }
 
@@ -427,12 +434,12 @@ k_grad2(const double *__restrict__ U, const double *__restrict__ T, double *__re
       Fb[k] = val;
     }
     __syncthreads();
-    contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), Fb, Xa, tid);
-    contract<1, Q, Q, 2, L, NT>(CT<P>::QD(), Fb, Xc, tid);
+    contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), Fb, Xa, tid);
+    contract<1, Q, Q, 2, L, NT>(EO<P>::QD(), Fb, Xc, tid);
     contract<1, 4, QF, 2, L, NT>(CT<P>::PW(), Jq + q * 4 * QF, H, tid);
     __syncthreads();
-    contract<1, Q, L, 1, L, NT>(CT<P>::QD(), Xa, D2, tid);
-    contract<1, Q, L, 1, L, NT>(CT<P>::BW(), Xc, D2 + L2, tid);
+    contract<1, Q, L, 1, L, NT>(EO<P>::QD(), Xa, D2, tid);
+    contract<1, Q, L, 1, L, NT>(EO<P>::BW(), Xc, D2 + L2, tid);
     __syncthreads();
     for (int k = tid; k < L2; k += NT) {
       const int l = k / L, m = k - l * L;
@@ -494,7 +501,7 @@ k_visc2(const double *__restrict__ U, const double *__restrict__ G, double *__re
     for (int q = 0; q < 3; ++q) Lay[(s * 3 + q) * Q + j] = f[q][0] * nn[0] + f[q][1] * nn[1];
   }
   __syncthreads();
-  contract<1, 12, Q, 2, QF, NT>(CT<P>::Ig(), Lay, Wf, tid);
+  contract<1, 12, Q, 2, QF, NT>(EO<P>::Ig(), Lay, Wf, tid);
   __syncthreads();
   copy_block<NT>(Wf, TV + (size_t)e * 12 * QF, 12 * QF, tid);
   const double *mt = geo.metric + 9 * (size_t)e;
@@ -509,12 +516,12 @@ k_visc2(const double *__restrict__ U, const double *__restrict__ G, double *__re
   }
   __syncthreads();
   for (int q = 0; q < 3; ++q) {
-    contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), Gn + 2 * q * Q2, X1, tid);
-    contract<1, Q, Q, 2, L, NT>(CT<P>::QD(), Gn + (2 * q + 1) * Q2, X2, tid);
+    contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), Gn + 2 * q * Q2, X1, tid);
+    contract<1, Q, Q, 2, L, NT>(EO<P>::QD(), Gn + (2 * q + 1) * Q2, X2, tid);
     __syncthreads();
-    contract<1, Q, L, 1, L, NT>(CT<P>::QD(), X1, Vo, tid);
+    contract<1, Q, L, 1, L, NT>(EO<P>::QD(), X1, Vo, tid);
     __syncthreads();
-    contract<1, Q, L, 1, L, NT, true>(CT<P>::BW(), X2, Vo, tid);
+    contract<1, Q, L, 1, L, NT, true>(EO<P>::BW(), X2, Vo, tid);
     __syncthreads();
     copy_block<NT>(Vo, V + ((size_t)e * 3 + q) * L2, L2, tid);
     __syncthreads();
@@ -530,9 +537,9 @@ k_forward2(const double *__restrict__ Fn, double *__restrict__ Fm, Tab tb, int n
   const int e = blockIdx.x % ne, v = blockIdx.x / ne, tid = threadIdx.x;
   copy_block<NT>(Fn + ((size_t)v * ne + e) * Q2, A, Q2, tid);
   __syncthreads();
-  contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), A, X, tid);
+  contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), A, X, tid);
   __syncthreads();
-  contract<1, Q, L, 1, L, NT>(CT<P>::BW(), X, O, tid);
+  contract<1, Q, L, 1, L, NT>(EO<P>::BW(), X, O, tid);
   __syncthreads();
   copy_block<NT>(O, Fm + ((size_t)v * ne + e) * L2, L2, tid);
 }

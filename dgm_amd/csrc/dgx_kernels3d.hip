@@ -30,11 +30,11 @@ __device__ __forceinline__ void backward3(const Tab &tb, const double *m, double
                                           double *out, int tid) {
   using S = H3<P>;
   constexpr int L = S::L, Q = S::Q, NT = S::NT;
-  contract<L, L, L, 0, Q, NT>(CT<P>::BT(), m, s1, tid);
+  contract<L, L, L, 0, Q, NT>(EO<P>::BT(), m, s1, tid);
   __syncthreads();
-  contract<Q, L, L, 1, Q, NT>(CT<P>::BT(), s1, s2, tid);
+  contract<Q, L, L, 1, Q, NT>(EO<P>::BT(), s1, s2, tid);
   __syncthreads();
-  contract<Q, Q, L, 2, Q, NT>(CT<P>::BT(), s2, out, tid);
+  contract<Q, Q, L, 2, Q, NT>(EO<P>::BT(), s2, out, tid);
   __syncthreads();
 }
 
@@ -47,23 +47,23 @@ __device__ __forceinline__ void divergence3(const Tab &tb, double *Fb, double *X
   constexpr int L = S::L, Q = S::Q, NT = S::NT;
   fill(0, Fb);
   __syncthreads();
-  contract<Q, Q, Q, 2, L, NT>(CT<P>::BW(), Fb, X, tid);
+  contract<Q, Q, Q, 2, L, NT>(EO<P>::BW(), Fb, X, tid);
   __syncthreads();
-  contract<Q, Q, L, 1, L, NT>(CT<P>::BW(), X, Y1, tid);
+  contract<Q, Q, L, 1, L, NT>(EO<P>::BW(), X, Y1, tid);
   fill(1, Fb);
   __syncthreads();
-  contract<Q, Q, Q, 2, L, NT>(CT<P>::BW(), Fb, X, tid);
+  contract<Q, Q, Q, 2, L, NT>(EO<P>::BW(), Fb, X, tid);
   __syncthreads();
-  contract<Q, Q, L, 1, L, NT>(CT<P>::QD(), X, Y2, tid);
+  contract<Q, Q, L, 1, L, NT>(EO<P>::QD(), X, Y2, tid);
   fill(2, Fb);
   __syncthreads();
-  contract<Q, Q, Q, 2, L, NT>(CT<P>::QD(), Fb, X, tid);
+  contract<Q, Q, Q, 2, L, NT>(EO<P>::QD(), Fb, X, tid);
   __syncthreads();
-  contract<Q, Q, L, 1, L, NT, true>(CT<P>::BW(), X, Y2, tid);
+  contract<Q, Q, L, 1, L, NT, true>(EO<P>::BW(), X, Y2, tid);
   __syncthreads();
-  contract<Q, L, L, 0, L, NT>(CT<P>::QD(), Y1, out, tid);
+  contract<Q, L, L, 0, L, NT>(EO<P>::QD(), Y1, out, tid);
   __syncthreads();
-  contract<Q, L, L, 0, L, NT, true>(CT<P>::BW(), Y2, out, tid);
+  contract<Q, L, L, 0, L, NT, true>(EO<P>::BW(), Y2, out, tid);
   __syncthreads();
 }
 
@@ -74,9 +74,9 @@ __device__ __forceinline__ void face_project3(const Tab &tb, const double *g, do
                                               int tid) {
   using S = H3<P>;
   constexpr int L = S::L, QF = S::QF, NT = S::NT;
-  contract<6, QF, QF, 1, L, NT>(CT<P>::PW(), g, W, tid);
+  contract<6, QF, QF, 1, L, NT>(EO<P>::PW(), g, W, tid);
   __syncthreads();
-  contract<6, L, QF, 2, L, NT>(CT<P>::PW(), W, H, tid);
+  contract<6, L, QF, 2, L, NT>(EO<P>::PW(), W, H, tid);
   __syncthreads();
 }
 
@@ -95,15 +95,15 @@ k_traces3(const double *__restrict__ U, double *__restrict__ T, Tab tb, int ne, 
   for (int v = 0; v < nf; ++v) {
     copy_block<NT>(U + ((size_t)v * ne + e) * L3, A, L3, tid);
     __syncthreads();
-    contract<L, L, L, 0, 2, NT>(CT<P>::Bend(), A, K0, tid);
-    contract<L, L, L, 1, 2, NT>(CT<P>::Bend(), A, K1, tid);
-    contract<L, L, L, 2, 2, NT>(CT<P>::Bend(), A, K2, tid);
+    contract<L, L, L, 0, 2, NT>(EO<P>::Bend(), A, K0, tid);
+    contract<L, L, L, 1, 2, NT>(EO<P>::Bend(), A, K1, tid);
+    contract<L, L, L, 2, 2, NT>(EO<P>::Bend(), A, K2, tid);
     __syncthreads();
     double *Te = T + (size_t)e * 6 * nf * QF2;
     // faces 4 (xi=-1) and 2 (xi=+1): [2][QF(b)][QF(c)]
-    contract<2, L, L, 1, QF, NT>(CT<P>::Bg(), K0, W, tid);
+    contract<2, L, L, 1, QF, NT>(EO<P>::Bg(), K0, W, tid);
     __syncthreads();
-    contract<2, QF, L, 2, QF, NT>(CT<P>::Bg(), W, O, tid);
+    contract<2, QF, L, 2, QF, NT>(EO<P>::Bg(), W, O, tid);
     __syncthreads();
     for (int i = tid; i < 2 * QF2; i += NT) {
       const int end = i / QF2, a = i - end * QF2;
@@ -111,9 +111,9 @@ k_traces3(const double *__restrict__ U, double *__restrict__ T, Tab tb, int ne, 
     }
     __syncthreads();
     // faces 1 (eta=-1) and 3 (eta=+1): [QF(a)][2][QF(c)]
-    contract<L, 2, L, 0, QF, NT>(CT<P>::Bg(), K1, W, tid);
+    contract<L, 2, L, 0, QF, NT>(EO<P>::Bg(), K1, W, tid);
     __syncthreads();
-    contract<QF, 2, L, 2, QF, NT>(CT<P>::Bg(), W, O, tid);
+    contract<QF, 2, L, 2, QF, NT>(EO<P>::Bg(), W, O, tid);
     __syncthreads();
     for (int i = tid; i < 2 * QF2; i += NT) {
       const int ia = i / (2 * QF), r = i - ia * 2 * QF, end = r / QF, ic = r - end * QF;
@@ -121,9 +121,9 @@ k_traces3(const double *__restrict__ U, double *__restrict__ T, Tab tb, int ne, 
     }
     __syncthreads();
     // faces 0 (zeta=-1) and 5 (zeta=+1): [QF(a)][QF(b)][2]
-    contract<L, L, 2, 0, QF, NT>(CT<P>::Bg(), K2, W, tid);
+    contract<L, L, 2, 0, QF, NT>(EO<P>::Bg(), K2, W, tid);
     __syncthreads();
-    contract<QF, L, 2, 1, QF, NT>(CT<P>::Bg(), W, O, tid);
+    contract<QF, L, 2, 1, QF, NT>(EO<P>::Bg(), W, O, tid);
     __syncthreads();
     for (int i = tid; i < 2 * QF2; i += NT) {
       const int ab = i >> 1, end = i & 1;
@@ -305,16 +305,16 @@ k_grad3(const double *__restrict__ U, const double *__restrict__ T, double *__re
       Fb[k] = val;
     }
     __syncthreads();
-    contract<Q, Q, Q, 2, L, NT>(CT<P>::BW(), Fb, Xa, tid);
-    contract<Q, Q, Q, 2, L, NT>(CT<P>::QD(), Fb, Xc, tid);
+    contract<Q, Q, Q, 2, L, NT>(EO<P>::BW(), Fb, Xa, tid);
+    contract<Q, Q, Q, 2, L, NT>(EO<P>::QD(), Fb, Xc, tid);
     __syncthreads();
-    contract<Q, Q, L, 1, L, NT>(CT<P>::BW(), Xa, Ya, tid);
-    contract<Q, Q, L, 1, L, NT>(CT<P>::QD(), Xa, Yb, tid);
-    contract<Q, Q, L, 1, L, NT>(CT<P>::BW(), Xc, Yc, tid);
+    contract<Q, Q, L, 1, L, NT>(EO<P>::BW(), Xa, Ya, tid);
+    contract<Q, Q, L, 1, L, NT>(EO<P>::QD(), Xa, Yb, tid);
+    contract<Q, Q, L, 1, L, NT>(EO<P>::BW(), Xc, Yc, tid);
     __syncthreads();
-    contract<Q, L, L, 0, L, NT>(CT<P>::QD(), Ya, D3, tid);
-    contract<Q, L, L, 0, L, NT>(CT<P>::BW(), Yb, D3 + L3, tid);
-    contract<Q, L, L, 0, L, NT>(CT<P>::BW(), Yc, D3 + 2 * L3, tid);
+    contract<Q, L, L, 0, L, NT>(EO<P>::QD(), Ya, D3, tid);
+    contract<Q, L, L, 0, L, NT>(EO<P>::BW(), Yb, D3 + L3, tid);
+    contract<Q, L, L, 0, L, NT>(EO<P>::BW(), Yc, D3 + 2 * L3, tid);
     face_project3<P>(tb, Jq + q * 6 * QF2, Xa, Ya, tid);   // H -> Ya ([6][L][L])
     for (int k = tid; k < L3; k += NT) {
       const int l = k / L2, m = (k / L) % L, n = k % L;
@@ -358,11 +358,11 @@ k_visc3(const double *__restrict__ U, const double *__restrict__ G, double *__re
     double *dst = v < 5 ? Un + v * Q3 : Gn + (v - 5) * Q3;
     copy_block<NT>(src, m0, L3, tid);
     __syncthreads();
-    contract<L, L, L, 0, Q, NT>(CT<P>::BT(), m0, s1, tid);
+    contract<L, L, L, 0, Q, NT>(EO<P>::BT(), m0, s1, tid);
     __syncthreads();
-    contract<Q, L, L, 1, Q, NT>(CT<P>::BT(), s1, s2, tid);
+    contract<Q, L, L, 1, Q, NT>(EO<P>::BT(), s1, s2, tid);
     __syncthreads();
-    contract<Q, Q, L, 2, Q, NT>(CT<P>::BT(), s2, dst, tid);
+    contract<Q, Q, L, 2, Q, NT>(EO<P>::BT(), s2, dst, tid);
     __syncthreads();
   }
   const double mu = ph.vis, kap = ph.vis * ph.gamma / ph.Pr;
@@ -406,9 +406,9 @@ k_visc3(const double *__restrict__ U, const double *__restrict__ G, double *__re
       Lay[(s * 4 + q) * Q2 + ij] = f[q][0] * nn[0] + f[q][1] * nn[1] + f[q][2] * nn[2];
   }
   __syncthreads();
-  contract<24, Q, Q, 1, QF, NT>(CT<P>::Ig(), Lay, Wf, tid);
+  contract<24, Q, Q, 1, QF, NT>(EO<P>::Ig(), Lay, Wf, tid);
   __syncthreads();
-  contract<24, QF, Q, 2, QF, NT>(CT<P>::Ig(), Wf, Lay, tid);   // [24][QF][QF] == [6][4][QF2]
+  contract<24, QF, Q, 2, QF, NT>(EO<P>::Ig(), Wf, Lay, tid);   // [24][QF][QF] == [6][4][QF2]
   __syncthreads();
   copy_block<NT>(Lay, TV + (size_t)e * 24 * QF2, 24 * QF2, tid);
   __syncthreads();
@@ -427,21 +427,21 @@ k_visc3(const double *__restrict__ U, const double *__restrict__ G, double *__re
   double *X = Sc, *Y1 = Sc + Q2 * L, *Y2 = Y1 + Q * L2, *Vo = Y2 + Q * L2;
   for (int q = 0; q < 4; ++q) {
     const double *Fr = Gn + 3 * q * Q3, *Fs = Fr + Q3, *Ft = Fs + Q3;
-    contract<Q, Q, Q, 2, L, NT>(CT<P>::BW(), Fr, X, tid);
+    contract<Q, Q, Q, 2, L, NT>(EO<P>::BW(), Fr, X, tid);
     __syncthreads();
-    contract<Q, Q, L, 1, L, NT>(CT<P>::BW(), X, Y1, tid);
+    contract<Q, Q, L, 1, L, NT>(EO<P>::BW(), X, Y1, tid);
     __syncthreads();
-    contract<Q, Q, Q, 2, L, NT>(CT<P>::BW(), Fs, X, tid);
+    contract<Q, Q, Q, 2, L, NT>(EO<P>::BW(), Fs, X, tid);
     __syncthreads();
-    contract<Q, Q, L, 1, L, NT>(CT<P>::QD(), X, Y2, tid);
+    contract<Q, Q, L, 1, L, NT>(EO<P>::QD(), X, Y2, tid);
     __syncthreads();
-    contract<Q, Q, Q, 2, L, NT>(CT<P>::QD(), Ft, X, tid);
+    contract<Q, Q, Q, 2, L, NT>(EO<P>::QD(), Ft, X, tid);
     __syncthreads();
-    contract<Q, Q, L, 1, L, NT, true>(CT<P>::BW(), X, Y2, tid);
+    contract<Q, Q, L, 1, L, NT, true>(EO<P>::BW(), X, Y2, tid);
     __syncthreads();
-    contract<Q, L, L, 0, L, NT>(CT<P>::QD(), Y1, Vo, tid);
+    contract<Q, L, L, 0, L, NT>(EO<P>::QD(), Y1, Vo, tid);
     __syncthreads();
-    contract<Q, L, L, 0, L, NT, true>(CT<P>::BW(), Y2, Vo, tid);
+    contract<Q, L, L, 0, L, NT, true>(EO<P>::BW(), Y2, Vo, tid);
     __syncthreads();
     copy_block<NT>(Vo, V + ((size_t)e * 4 + q) * L3, L3, tid);
     __syncthreads();
@@ -461,11 +461,11 @@ k_forward3(const double *__restrict__ Fn, double *__restrict__ Fm, Tab tb, int n
   const int e = blockIdx.x % ne, v = blockIdx.x / ne, tid = threadIdx.x;
   copy_block<NT>(Fn + ((size_t)v * ne + e) * Q3, A, Q3, tid);
   __syncthreads();
-  contract<Q, Q, Q, 2, L, NT>(CT<P>::BW(), A, X, tid);
+  contract<Q, Q, Q, 2, L, NT>(EO<P>::BW(), A, X, tid);
   __syncthreads();
-  contract<Q, Q, L, 1, L, NT>(CT<P>::BW(), X, Y, tid);
+  contract<Q, Q, L, 1, L, NT>(EO<P>::BW(), X, Y, tid);
   __syncthreads();
-  contract<Q, L, L, 0, L, NT>(CT<P>::BW(), Y, O, tid);
+  contract<Q, L, L, 0, L, NT>(EO<P>::BW(), Y, O, tid);
   __syncthreads();
   copy_block<NT>(O, Fm + ((size_t)v * ne + e) * L3, L3, tid);
 }

@@ -599,16 +599,16 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
     }
     __syncthreads();
     constexpr int KP = S::KP;
-    con_mid<F, L, L, L, 2, LP, LP, NT>(CT<P>::Bend(), Md, K0, tid);       // [F][2][L][L]
-    con_mid<F * L, L, 1, L, 2, LP, LP, NT>(CT<P>::Bend(), Md, K1, tid);   // [F][L][2][L]
-    con_last<F * L2, L, 2, LP, KP, NT>(CT<P>::Bend(), Md, K2, tid);       // [F][L][L][2]
+    con_mid<F, L, L, L, 2, LP, LP, NT>(EO<P>::Bend(), Md, K0, tid);       // [F][2][L][L]
+    con_mid<F * L, L, 1, L, 2, LP, LP, NT>(EO<P>::Bend(), Md, K1, tid);   // [F][L][2][L]
+    con_last<F * L2, L, 2, LP, KP, NT>(EO<P>::Bend(), Md, K2, tid);       // [F][L][L][2]
     __syncthreads();
     double *W = Md, *O = Md + F * S::TW;
     double *Te = a.Tn + (size_t)e * 6 * 5 * QF2;
     // faces 4 / 2: [F][2][QF][QF]
-    con_mid<2 * F, L, 1, L, QF, LP, LP, NT>(CT<P>::Bg(), K0, W, tid);     // [2F][QF][L]
+    con_mid<2 * F, L, 1, L, QF, LP, LP, NT>(EO<P>::Bg(), K0, W, tid);     // [2F][QF][L]
     __syncthreads();
-    con_last<2 * F * QF, L, QF, LP, FP, NT>(CT<P>::Bg(), W, O, tid);      // [2F][QF][QF]
+    con_last<2 * F * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);      // [2F][QF][QF]
     __syncthreads();
     for (int i = tid; i < 2 * F * QF2; i += NT) {
       const int ve = i / QF2, q = i - ve * QF2, v = ve >> 1, end = ve & 1;
@@ -616,9 +616,9 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
     }
     __syncthreads();
     // faces 1 / 3: [F][QF][2][QF]
-    con_mid<F, L, 2, L, QF, LP, LP, NT>(CT<P>::Bg(), K1, W, tid);         // [F][QF][2][L]
+    con_mid<F, L, 2, L, QF, LP, LP, NT>(EO<P>::Bg(), K1, W, tid);         // [F][QF][2][L]
     __syncthreads();
-    con_last<2 * F * QF, L, QF, LP, FP, NT>(CT<P>::Bg(), W, O, tid);      // [F][QF][2][QF]
+    con_last<2 * F * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);      // [F][QF][2][QF]
     __syncthreads();
     for (int i = tid; i < 2 * F * QF2; i += NT) {
       const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
@@ -627,9 +627,9 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
     }
     __syncthreads();
     // faces 0 / 5: [F][QF][QF][2]
-    con_mid<F, L, L, 2, QF, KP, KP, NT>(CT<P>::Bg(), K2, W, tid);         // [F][QF][L][2]
+    con_mid<F, L, L, 2, QF, KP, KP, NT>(EO<P>::Bg(), K2, W, tid);         // [F][QF][L][2]
     __syncthreads();
-    con_mid<F * QF, L, 1, 2, QF, KP, KP, NT>(CT<P>::Bg(), W, O, tid);     // [F][QF][QF][2]
+    con_mid<F * QF, L, 1, 2, QF, KP, KP, NT>(EO<P>::Bg(), W, O, tid);     // [F][QF][QF][2]
     __syncthreads();
     for (int i = tid; i < 2 * F * QF2; i += NT) {
       const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;

@@ -55,8 +55,8 @@ template <int P, int NTH = kStageThreads> struct S3 {
 // acc[k][l] += sum_i M[l][i] in[f][i][m][n] for the thread's pencils
 // G = tid + k*NT = f*L2 + m*L + n.
 template <int P, int NF, int NS, int NTH = kStageThreads>
-__device__ __forceinline__ void chain_to_regs(const double *__restrict__ M, const double *in,
-                                              double (&acc)[NS][P + 1], int tid) {
+__device__ __forceinline__ void chain_to_regs(EoMat<EO_NM, double> M, const double *in, double (&acc)[NS][P + 1],
+                                              int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, L2 = S::L2, LP = S::LP, NT = S::NT;
 #pragma unroll
@@ -67,13 +67,10 @@ __device__ __forceinline__ void chain_to_regs(const double *__restrict__ M, cons
       double x[Q];
 #pragma unroll
       for (int i = 0; i < Q; ++i) x[i] = in[((f * Q + i) * L + m) * LP + n];
+      double y[L];
+      eo_apply<EO_NM, Q, L>(M.h, x, y);
 #pragma unroll
-      for (int l = 0; l < L; ++l) {
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < Q; ++i) s = fma(M[l * Q + i], x[i], s);
-        acc[k][l] += s;
-      }
+      for (int l = 0; l < L; ++l) acc[k][l] += y[l];
     }
   }
 }
@@ -88,9 +85,9 @@ __device__ __forceinline__ void nodal_deriv(const double *A, double *B, int tid)
   using S = S3<P, NTH>;
   constexpr int Q = S::Q, QP = S::QP, NT = S::NT;
   static_assert(D != 2 || !ACC, "the c derivative comes first and writes B");
-  if constexpr (D == 2) con_last<NF * Q * Q, Q, Q, QP, QP, NT>(CT<P>::DN(), A, B, tid);
-  else if constexpr (D == 1) con_mid<NF * Q, Q, 1, Q, Q, QP, QP, NT, ACC>(CT<P>::DN(), A, B, tid);
-  else con_mid<NF, Q, Q, Q, Q, QP, QP, NT, ACC>(CT<P>::DN(), A, B, tid);
+  if constexpr (D == 2) con_last<NF * Q * Q, Q, Q, QP, QP, NT>(EO<P>::DN(), A, B, tid);
+  else if constexpr (D == 1) con_mid<NF * Q, Q, 1, Q, Q, QP, QP, NT, ACC>(EO<P>::DN(), A, B, tid);
+  else con_mid<NF, Q, Q, Q, Q, QP, QP, NT, ACC>(EO<P>::DN(), A, B, tid);
 }
 
 // Projection BW (x) BW (x) BW of NF nodal fields in B, accumulated into the
@@ -99,11 +96,11 @@ template <int P, int NF, int NS, int NTH = kStageThreads>
 __device__ __forceinline__ void proj_to_regs(double *A, double *B, double (&acc)[NS][P + 1], int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT;
-  con_last<NF * Q * Q, Q, L, QP, LP, NT>(CT<P>::BW(), B, A, tid);   // [NF Q Q][L]
+  con_last<NF * Q * Q, Q, L, QP, LP, NT>(EO<P>::BW(), B, A, tid);   // [NF Q Q][L]
   __syncthreads();
-  con_mid<NF * Q, Q, 1, L, L, LP, LP, NT>(CT<P>::BW(), A, B, tid);  // [NF Q][L][L]
+  con_mid<NF * Q, Q, 1, L, L, LP, LP, NT>(EO<P>::BW(), A, B, tid);  // [NF Q][L][L]
   __syncthreads();
-  chain_to_regs<P, NF, NS, NTH>(CT<P>::BW(), B, acc, tid);           // [NF][L][L][L]
+  chain_to_regs<P, NF, NS, NTH>(EO<P>::BW(), B, acc, tid);           // [NF][L][L][L]
   __syncthreads();
 }
 
@@ -112,11 +109,11 @@ template <int P, int NF, int NTH = kStageThreads>
 __device__ __forceinline__ void backward_batch(double *A, double *B, int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT;
-  con_mid<NF, L, L, L, Q, LP, LP, NT>(CT<P>::BT(), A, B, tid);   // [NF][Q][L][L]
+  con_mid<NF, L, L, L, Q, LP, LP, NT>(EO<P>::BT(), A, B, tid);   // [NF][Q][L][L]
   __syncthreads();
-  con_mid<NF * Q, L, 1, L, Q, LP, LP, NT>(CT<P>::BT(), B, A, tid);   // [NF Q][Q][L]
+  con_mid<NF * Q, L, 1, L, Q, LP, LP, NT>(EO<P>::BT(), B, A, tid);   // [NF Q][Q][L]
   __syncthreads();
-  con_last<NF * Q * Q, L, Q, LP, QP, NT>(CT<P>::BT(), A, B, tid);   // [NF Q Q][Q]
+  con_last<NF * Q * Q, L, Q, LP, QP, NT>(EO<P>::BT(), A, B, tid);   // [NF Q Q][Q]
   __syncthreads();
 }
 
@@ -125,9 +122,9 @@ template <int P, int NFB, int NTH = kStageThreads>
 __device__ __forceinline__ void face_project(const double *g, double *A, double *B, int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, QF = S::QF, LP = S::LP, FP = S::FP, NT = S::NT;
-  con_mid<NFB, QF, 1, QF, L, FP, FP, NT>(CT<P>::PW(), g, A, tid);     // [NFB][L][QF]
+  con_mid<NFB, QF, 1, QF, L, FP, FP, NT>(EO<P>::PW(), g, A, tid);     // [NFB][L][QF]
   __syncthreads();
-  con_last<NFB * L, QF, L, FP, LP, NT>(CT<P>::PW(), A, B, tid);     // [NFB][L][L]
+  con_last<NFB * L, QF, L, FP, LP, NT>(EO<P>::PW(), A, B, tid);     // [NFB][L][L]
   __syncthreads();
 }
 
@@ -349,16 +346,16 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
   __syncthreads();
   constexpr int KP = 3;   // pitch of the [..][2] collapse
   double *K0 = B, *K1 = B + 10 * L * LP, *K2 = B + 20 * L * LP;
-  con_mid<5, L, L, L, 2, LP, LP, NT>(CT<P>::Bend(), A, K0, tid);       // [5][2][L][L]
-  con_mid<5 * L, L, 1, L, 2, LP, LP, NT>(CT<P>::Bend(), A, K1, tid);   // [5][L][2][L]
-  con_last<5 * L2, L, 2, LP, KP, NT>(CT<P>::Bend(), A, K2, tid);       // [5][L][L][2]
+  con_mid<5, L, L, L, 2, LP, LP, NT>(EO<P>::Bend(), A, K0, tid);       // [5][2][L][L]
+  con_mid<5 * L, L, 1, L, 2, LP, LP, NT>(EO<P>::Bend(), A, K1, tid);   // [5][L][2][L]
+  con_last<5 * L2, L, 2, LP, KP, NT>(EO<P>::Bend(), A, K2, tid);       // [5][L][L][2]
   __syncthreads();
   double *W = A, *O = A + 10 * QF * cmax(LP, KP * L);
   double *Te = a.Tn + (size_t)e * 6 * 5 * QF2;
   // faces 4 / 2: [5][2][QF][QF]
-  con_mid<10, L, 1, L, QF, LP, LP, NT>(CT<P>::Bg(), K0, W, tid);      // [10][QF][L]
+  con_mid<10, L, 1, L, QF, LP, LP, NT>(EO<P>::Bg(), K0, W, tid);      // [10][QF][L]
   __syncthreads();
-  con_last<10 * QF, L, QF, LP, FP, NT>(CT<P>::Bg(), W, O, tid);       // [10][QF][QF]
+  con_last<10 * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);       // [10][QF][QF]
   __syncthreads();
   for (int i = tid; i < 10 * QF2; i += NT) {
     const int ve = i / QF2, q = i - ve * QF2, v = ve >> 1, end = ve & 1;
@@ -366,9 +363,9 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
   }
   __syncthreads();
   // faces 1 / 3: [5][QF][2][QF]
-  con_mid<5, L, 2, L, QF, LP, LP, NT>(CT<P>::Bg(), K1, W, tid);       // [5][QF][2][L]
+  con_mid<5, L, 2, L, QF, LP, LP, NT>(EO<P>::Bg(), K1, W, tid);       // [5][QF][2][L]
   __syncthreads();
-  con_last<10 * QF, L, QF, LP, FP, NT>(CT<P>::Bg(), W, O, tid);       // [5][QF][2][QF]
+  con_last<10 * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);       // [5][QF][2][QF]
   __syncthreads();
   for (int i = tid; i < 10 * QF2; i += NT) {
     const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
@@ -377,9 +374,9 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
   }
   __syncthreads();
   // faces 0 / 5: [5][QF][QF][2]
-  con_mid<5, L, L, 2, QF, KP, KP, NT>(CT<P>::Bg(), K2, W, tid);       // [5][QF][L][2]
+  con_mid<5, L, L, 2, QF, KP, KP, NT>(EO<P>::Bg(), K2, W, tid);       // [5][QF][L][2]
   __syncthreads();
-  con_mid<5 * QF, L, 1, 2, QF, KP, KP, NT>(CT<P>::Bg(), W, O, tid);   // [5][QF][QF][2]
+  con_mid<5 * QF, L, 1, 2, QF, KP, KP, NT>(EO<P>::Bg(), W, O, tid);   // [5][QF][QF][2]
   __syncthreads();
   for (int i = tid; i < 10 * QF2; i += NT) {
     const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
@@ -396,7 +393,7 @@ __device__ __forceinline__ void lifted_dir(const double *in, double *out, const 
                                            int tid) {
   constexpr int Q = P + 2, QP = odd(Q), HB = Q * QP, NP = 4 * Q * Q;
   constexpr int flo = D == 0 ? 4 : (D == 1 ? 1 : 0), fhi = D == 0 ? 2 : (D == 1 ? 3 : 5);
-  const double *M = CT<P>::NPD(), *KE = CT<P>::KE();
+  const double *KE = CT<P>::KE();
   for (int pc = tid; pc < NP; pc += NT) {
     const int f = pc / (Q * Q), t = pc - f * Q * Q, t1 = t / Q, t2 = t - t1 * Q;
     // (t1, t2): the two other indices in order; base and stride of the pencil
@@ -409,14 +406,12 @@ __device__ __forceinline__ void lifted_dir(const double *in, double *out, const 
     for (int m = 0; m < Q; ++m) x[m] = in[base + m * stride];
     const double hl = clo * Hn[(f * 6 + flo) * HB + t1 * QP + t2];
     const double hh = chi * Hn[(f * 6 + fhi) * HB + t1 * QP + t2];
-#pragma unroll 3   // about 3 coefficient rows live in scalar registers at a time
-    for (int o = 0; o < Q; ++o) {
-      double s = 0.0;
+    double y[Q];
+    eo_apply<EO_NNA, Q, Q>(EO<P>::NPD().h, x, y);
 #pragma unroll
-      for (int m = 0; m < Q; ++m) s = fma(M[o * Q + m], x[m], s);
-      s = fma(KE[o], hl, s);
-      s = fma(KE[Q + o], hh, s);
-      out[base + o * stride] = s;
+    for (int o = 0; o < Q; ++o) {   // KE_hi[o] = KE_lo[rev o]
+      const double s = fma(KE[o], hl, y[o]);
+      out[base + o * stride] = fma(KE[Q - 1 - o], hh, s);
     }
   }
 }
@@ -524,13 +519,13 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
   __syncthreads();
   // face lift of the jumps: (PW (x) PW) Jq -> H[4][6][L][L], then its values at
   // each face's own GLL points Hn[4][6][Q][Q] = (BT (x) BT) H, kept in the Jq region
-  con_mid<24, QF, 1, QF, L, FP, FP, NT>(CT<P>::PW(), Jq, A, tid);     // [24][L][QF]
+  con_mid<24, QF, 1, QF, L, FP, FP, NT>(EO<P>::PW(), Jq, A, tid);     // [24][L][QF]
   __syncthreads();
-  con_last<24 * L, QF, L, FP, LP, NT>(CT<P>::PW(), A, Jq, tid);     // [24][L][L]
+  con_last<24 * L, QF, L, FP, LP, NT>(EO<P>::PW(), A, Jq, tid);     // [24][L][L]
   __syncthreads();
-  con_mid<24, L, 1, L, Q, LP, LP, NT>(CT<P>::BT(), Jq, A, tid);     // [24][Q][L]
+  con_mid<24, L, 1, L, Q, LP, LP, NT>(EO<P>::BT(), Jq, A, tid);     // [24][Q][L]
   __syncthreads();
-  con_last<24 * Q, L, Q, LP, QP, NT>(CT<P>::BT(), A, Jq, tid);      // [24][Q][Q]
+  con_last<24 * Q, L, Q, LP, QP, NT>(EO<P>::BT(), A, Jq, tid);      // [24][Q][Q]
   __syncthreads();
   const double *Hn = Jq;
   constexpr int HB = Q * QP;   // one nodal face block
@@ -560,11 +555,11 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
       }
     }
     __syncthreads();
-    if constexpr (d == 2) con_mid<4 * Q, Q, 1, Q, Q, QP, QP, NT>(CT<P>::NP1(), A, B, tid);   // along b
-    else con_last<4 * Q * Q, Q, Q, QP, QP, NT>(CT<P>::NP1(), A, B, tid);                    // along c
+    if constexpr (d == 2) con_mid<4 * Q, Q, 1, Q, Q, QP, QP, NT>(EO<P>::NP1(), A, B, tid);   // along b
+    else con_last<4 * Q * Q, Q, Q, QP, QP, NT>(EO<P>::NP1(), A, B, tid);                    // along c
     __syncthreads();
-    if constexpr (d == 0) con_mid<4 * Q, Q, 1, Q, Q, QP, QP, NT>(CT<P>::NP1(), B, A, tid);  // along b
-    else con_mid<4, Q, Q, Q, Q, QP, QP, NT>(CT<P>::NP1(), B, A, tid);                       // along a
+    if constexpr (d == 0) con_mid<4 * Q, Q, 1, Q, Q, QP, QP, NT>(EO<P>::NP1(), B, A, tid);  // along b
+    else con_mid<4, Q, Q, Q, Q, QP, QP, NT>(EO<P>::NP1(), B, A, tid);                       // along a
     __syncthreads();
     const double g0 = mt[3 * d], g1 = mt[3 * d + 1], g2 = mt[3 * d + 2];
     const double inv = 1.0 / sqrt(g0 * g0 + g1 * g1 + g2 * g2);
@@ -668,9 +663,9 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
   if constexpr (BR2) {
     // lift of the flux difference on the element's own faces, into the volume term:
     // (PW Ig (x) PW Ig) difference -> modal face blocks [4][6][L][L] in B
-    con_mid<24, Q, 1, Q, L, QP, QP, NT>(CT<P>::PI(), B, Jq, tid);   // [24][L][Q]
+    con_mid<24, Q, 1, Q, L, QP, QP, NT>(EO<P>::PI(), B, Jq, tid);   // [24][L][Q]
     __syncthreads();
-    con_last<24 * L, Q, L, QP, LP, NT>(CT<P>::PI(), Jq, B, tid);    // [24][L][L]
+    con_last<24 * L, Q, L, QP, LP, NT>(EO<P>::PI(), Jq, B, tid);    // [24][L][L]
     __syncthreads();
     double jr6[6];
 #pragma unroll
@@ -689,9 +684,9 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
 #pragma unroll
       for (int l = 0; l < L; ++l) acc[k][l] = 0.0;
   }
-  con_mid<24, Q, 1, Q, QF, QP, QP, NT>(CT<P>::Ig(), Lay, Gs, tid);   // [24][QF][Q]
+  con_mid<24, Q, 1, Q, QF, QP, QP, NT>(EO<P>::Ig(), Lay, Gs, tid);   // [24][QF][Q]
   __syncthreads();
-  con_last<24 * QF, Q, QF, QP, FP, NT>(CT<P>::Ig(), Gs, A, tid);     // [24][QF][QF]
+  con_last<24 * QF, Q, QF, QP, FP, NT>(EO<P>::Ig(), Gs, A, tid);     // [24][QF][QF]
   __syncthreads();
   for (int i = tid; i < 24 * QF2; i += NT) {
     const int sq = i / QF2, q = i - sq * QF2;

@@ -40,8 +40,8 @@ __global__ void __launch_bounds__(64) k_vtraces2(VarpArgs a) {
     A[i] = a.U[((size_t)v * a.ne + e) * a.NM + (i - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 2, 2, NT>(CT<P>::Bend(), A, Kb, tid);   // [NF][L][2]: edges 0 / 2
-  contract<NF, L, L, 1, 2, NT>(CT<P>::Bend(), A, Ka, tid);   // [NF][2][L]: edges 3 / 1
+  contract<NF, L, L, 2, 2, NT>(EO<P>::Bend(), A, Kb, tid);   // [NF][L][2]: edges 0 / 2
+  contract<NF, L, L, 1, 2, NT>(EO<P>::Bend(), A, Ka, tid);   // [NF][2][L]: edges 3 / 1
   __syncthreads();
   double *Te = a.T + (size_t)e * 4 * NF * QFM;
   for (int s = 0; s < 4; ++s) {
@@ -80,9 +80,9 @@ __global__ void __launch_bounds__(64) k_vrhs2(VarpArgs a) {
     M[i] = a.U[((size_t)v * ne + e) * a.NM + (i - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 1, Q, NT>(CT<P>::BT(), M, X1, tid);   // [NF][Q][L]
+  contract<NF, L, L, 1, Q, NT>(EO<P>::BT(), M, X1, tid);   // [NF][Q][L]
   __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(CT<P>::BT(), X1, N1, tid);  // [NF][Q][Q]
+  contract<NF, Q, L, 2, Q, NT>(EO<P>::BT(), X1, N1, tid);  // [NF][Q][Q]
   __syncthreads();
   double un[NPT][NF];
 #pragma unroll
@@ -157,12 +157,12 @@ __global__ void __launch_bounds__(64) k_vrhs2(VarpArgs a) {
     for (int k = 0; k < n; ++k) acc = fma(PW[l * n + k], g[k], acc);
     H[i] = acc;
   }
-  contract<NF, Q, Q, 2, L, NT>(CT<P>::BW(), N1, X1, tid);
-  contract<NF, Q, Q, 2, L, NT>(CT<P>::QD(), N2, X2, tid);
+  contract<NF, Q, Q, 2, L, NT>(EO<P>::BW(), N1, X1, tid);
+  contract<NF, Q, Q, 2, L, NT>(EO<P>::QD(), N2, X2, tid);
   __syncthreads();
-  contract<NF, Q, L, 1, L, NT>(CT<P>::QD(), X1, M, tid);
+  contract<NF, Q, L, 1, L, NT>(EO<P>::QD(), X1, M, tid);
   __syncthreads();
-  contract<NF, Q, L, 1, L, NT, true>(CT<P>::BW(), X2, M, tid);
+  contract<NF, Q, L, 1, L, NT, true>(EO<P>::BW(), X2, M, tid);
   __syncthreads();
   const double cw[4] = {1.0, 1.0, 1.0, 1.0};
   for (int i = tid; i < NF * a.NM; i += NT) {
@@ -185,9 +185,9 @@ __global__ void __launch_bounds__(64) k_vforward2(VarpArgs a) {
   const double *src = a.X + ((size_t)v * a.ne + e) * a.QM;
   for (int i = tid; i < Q2; i += NT) A[i] = src[i];
   __syncthreads();
-  contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), A, X, tid);
+  contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), A, X, tid);
   __syncthreads();
-  contract<1, Q, L, 1, L, NT>(CT<P>::BW(), X, O, tid);
+  contract<1, Q, L, 1, L, NT>(EO<P>::BW(), X, O, tid);
   __syncthreads();
   double *dst = a.Y + ((size_t)v * a.ne + e) * a.NM;
   for (int i = tid; i < a.NM; i += NT) dst[i] = i < L2 ? O[i] : 0.0;
@@ -201,9 +201,9 @@ __global__ void __launch_bounds__(64) k_vbackward2(VarpArgs a) {
   const double *src = a.X + ((size_t)v * a.ne + e) * a.NM;
   for (int i = tid; i < L2; i += NT) A[i] = src[i];
   __syncthreads();
-  contract<1, L, L, 1, Q, NT>(CT<P>::BT(), A, X, tid);
+  contract<1, L, L, 1, Q, NT>(EO<P>::BT(), A, X, tid);
   __syncthreads();
-  contract<1, Q, L, 2, Q, NT>(CT<P>::BT(), X, O, tid);
+  contract<1, Q, L, 2, Q, NT>(EO<P>::BT(), X, O, tid);
   __syncthreads();
   double *dst = a.Y + ((size_t)v * a.ne + e) * a.QM;
   for (int i = tid; i < a.QM; i += NT) dst[i] = i < Q2 ? O[i] : 0.0;
