@@ -50,6 +50,7 @@ struct dgx_acoustic {
   std::vector<double *> snaps;
   long long fwd_steps = 0, adj_steps = 0;
   int snaps_used = 0;
+  bool t_valid = false;   // the domain's T holds the traces of its U
 
   size_t n() const { return (size_t)4 * ne * nm; }
 };
@@ -93,15 +94,20 @@ int traces(dgx_acoustic *a, const double *X) {
 int step_forward(dgx_acoustic *a, int k) {
   dgx_domain *d = a->dom;
   dgx::LinArgs la = lin_args(a, false);
-  la.X = d->U; la.T = d->T; la.Y = d->U; la.Yt = d->Ut; la.theta = a->d_theta;
+  la.X = d->U; la.Y = d->U; la.Yt = d->Ut; la.theta = a->d_theta;
   const double tk = k * a->dt;
-  for (int s = 0; s < 14; ++s) {
+  if (!a->t_valid) {
     int rc = traces(a, d->U);
     if (rc) return rc;
+  }
+  for (int s = 0; s < 14; ++s) {   // each stage writes the next one's traces
+    la.T = d->T; la.Tn = d->T2;
     la.ca = dgx::kLsrkA[s]; la.cb = dgx::kLsrkB[s];
     la.g = ricker(tk + dgx::kLsrkC[s] * a->dt, a->f0, a->t0);
     HIPCHK(dgx::launch_lin2(la));
+    std::swap(d->T, d->T2);
   }
+  a->t_valid = true;
   ++a->fwd_steps;
   return DGX_OK;
 }
@@ -115,15 +121,20 @@ int step_adjoint(dgx_acoustic *a, int k) {
     HIPCHK(dgx::launch_observe_adjoint(d->U, a->Ub, a->d_rec_e, a->d_rec_w, a->d_cobs, a->nrec, a->ne, L2,
                                        a->d_data + (size_t)k * a->nrec, a->dt, a->d_J, d->stream));
   dgx::LinArgs la = lin_args(a, true);
-  la.X = a->Ubt; la.T = d->T; la.Y = a->Ub; la.Yt = a->Ubt; la.gtheta = a->d_gtheta;
+  la.X = a->Ubt; la.Y = a->Ub; la.Yt = a->Ubt; la.gtheta = a->d_gtheta;
   const double tk = k * a->dt;
+  // Ubar_t += B_s Ubar and its traces: here for the first reversed stage, in
+  // the stage before for the others
+  a->t_valid = false;
+  HIPCHK(dgx::blas_axpy(dgx::kLsrkB[13], a->Ub, a->Ubt, a->Ubt, n, d->stream));
+  int rc = traces(a, a->Ubt);
+  if (rc) return rc;
   for (int s = 13; s >= 0; --s) {
-    HIPCHK(dgx::blas_axpy(dgx::kLsrkB[s], a->Ub, a->Ubt, a->Ubt, n, d->stream));   // Ubar_t += B_s Ubar
-    int rc = traces(a, a->Ubt);
-    if (rc) return rc;
-    la.ca = dgx::kLsrkA[s];
+    la.T = d->T; la.Tn = s > 0 ? d->T2 : nullptr;
+    la.ca = dgx::kLsrkA[s]; la.bn = s > 0 ? dgx::kLsrkB[s - 1] : 0.0;
     la.g = ricker(tk + dgx::kLsrkC[s] * a->dt, a->f0, a->t0);
     HIPCHK(dgx::launch_lin2(la));
+    if (s > 0) std::swap(d->T, d->T2);
   }
   ++a->adj_steps;
   return DGX_OK;
@@ -131,6 +142,7 @@ int step_adjoint(dgx_acoustic *a, int k) {
 
 int zero_state(dgx_acoustic *a) {
   dgx_domain *d = a->dom;
+  a->t_valid = false;
   HIPCHK(hipMemsetAsync(d->U, 0, a->n() * 8, d->stream));
   HIPCHK(hipMemsetAsync(d->Ut, 0, a->n() * 8, d->stream));
   return DGX_OK;
@@ -280,6 +292,7 @@ int dgx_acoustic_gradient(dgx_acoustic_handle a, const double *theta, const doub
   HIPCHK(hipMemcpyAsync(a->snaps[0], d->U, n * 8, hipMemcpyDeviceToDevice, st));
   Revolve rv;
   rv.restore = [&](int s) {
+    a->t_valid = false;
     if (hipMemcpyAsync(d->U, a->snaps[s], n * 8, hipMemcpyDeviceToDevice, st) != hipSuccess)
       return fail(DGX_ERR_DEVICE, "checkpoint restore");
     return (int)DGX_OK;

@@ -330,7 +330,7 @@ dgx::LaunchArgs launch_args(dgx_domain *d, int op, const double *U, double *out)
   a.op = op; a.p = d->p; a.ne = d->ne; a.nfield = d->nf; a.ns = d->visc;
   a.U = U; a.T = d->T; a.R = out; a.G = d->G; a.V = d->V; a.TV = d->TV;
   a.flag = d->d_flag; a.tab = d->tab; a.geo = d->geo; a.phys = d->phys; a.stream = d->stream;
-  a.eqn = d->eqn; a.Bal = d->Bal; a.bal = (op == dgx::OP_RHS || op == dgx::OP_STEP) ? d->bal : 0;
+  a.eqn = d->eqn; a.Bal = d->Bal; a.bal = (op == dgx::OP_RHS || op == dgx::OP_STAGE) ? d->bal : 0;
   a.mixed = d->mixed && d->nsd == 2;
   return a;
 }
@@ -343,6 +343,7 @@ int launch(dgx_domain *d, int op, const double *U, double *out) {
   });
   if (e != hipSuccess) return fail(DGX_ERR_DEVICE, std::string("kernel launch: ") + hipGetErrorString(e));
   if (op == dgx::OP_RHS && d->bal == 1) d->bal = 2;   // the first residual is stored
+  if (op == dgx::OP_TRACES) d->t_of = U;
   return DGX_OK;
 }
 
@@ -451,23 +452,24 @@ int residual_core(dgx_domain *d, const double *U, double *R) {
   return DGX_OK;
 }
 
-// One LSRK stage of an affine 2D domain (not curved, one order): the traces
-// (unless the previous stage of this call wrote them) and the viscous terms,
-// then the residual fused with the register update Ut = A Ut - dt R,
-// U += B Ut and with the traces of the new state (k_step2), bitwise the same
-// as the residual followed by the axpby and axpy.
-int step2(dgx_domain *d, double A, double B, double dt, bool traces_ready) {
+// One stage of an affine 2D domain (not curved, one order) at the state X: the
+// traces (unless an earlier stage of this call wrote them) and the viscous
+// terms, then the residual fused with the register update `st` and with the
+// traces of the new state (k_quad2).
+int stage2(dgx_domain *d, const double *X, const dgx::QuadStep &st, bool traces_ready) {
   int rc;
-  if (!traces_ready && (rc = launch(d, dgx::OP_TRACES, d->U, nullptr))) return rc;
+  if (!(traces_ready && d->t_of == X) && (rc = launch(d, dgx::OP_TRACES, X, nullptr))) return rc;
   if (d->visc) {
-    if ((rc = launch(d, dgx::OP_GRAD, d->U, nullptr))) return rc;
-    if ((rc = launch(d, dgx::OP_VISC, d->U, nullptr))) return rc;
+    if ((rc = launch(d, dgx::OP_GRAD, X, nullptr))) return rc;
+    if ((rc = launch(d, dgx::OP_VISC, X, nullptr))) return rc;
   }
-  dgx::LaunchArgs a = launch_args(d, dgx::OP_STEP, d->U, nullptr);
-  a.Us = d->U; a.Ut = d->Ut; a.ca = A; a.cb = B; a.dt = dt; a.Tn = d->T2;
+  dgx::LaunchArgs a = launch_args(d, dgx::OP_STAGE, X, nullptr);
+  a.step = st;
+  a.Tn = d->T2;
   hipError_t e = timed(d, dgx::OP_RHS, [&] { return dgx::launch_2d(a); });
   if (e != hipSuccess) return fail(DGX_ERR_DEVICE, std::string("stage launch: ") + hipGetErrorString(e));
   std::swap(d->T, d->T2);        // the next stage's traces
+  d->t_of = st.Xn;
   if (d->bal == 1) d->bal = 2;   // the first residual is stored
   ++d->stages;
   return DGX_OK;
@@ -1293,6 +1295,14 @@ int build(dgx_domain *d, const dgx_domain_desc *desc) {
   d->geo.metric = d->d_metric; d->geo.fnorm = d->d_fnorm; d->geo.fjr = d->d_fjr;
   d->geo.nbr = d->d_nbr; d->geo.nside = d->d_nside; d->geo.permid = d->d_permid; d->geo.perm = d->d_perm;
   d->geo.master = d->d_master;
+  if (nsd == 2) {   // a side's neighbour, its side and whether their points run reversed, in one word
+    std::vector<int> link((size_t)ne * 4);
+    for (size_t i = 0; i < link.size(); ++i)
+      link[i] = nbr[i] < 0 ? nbr[i] : (nbr[i] * 4 + nside[i]) * 2 + (permtab[(size_t)permid[i] * qs] != 0);
+    HIPCHK(hipMalloc((void **)&d->d_link2, link.size() * sizeof(int)));
+    HIPCHK(hipMemcpy(d->d_link2, link.data(), link.size() * sizeof(int), hipMemcpyHostToDevice));
+  }
+  d->geo.link2 = d->d_link2;
   d->phys.gamma = d->gamma; d->phys.vis = d->vis; d->phys.Pr = d->Pr; d->phys.flux = d->flux;
   d->phys.visc = desc->viscous;
   for (int v = 0; v < 5; ++v) d->phys.bcU[v] = desc->bc_state[v];
@@ -1376,7 +1386,7 @@ int build(dgx_domain *d, const dgx_domain_desc *desc) {
 }
 
 void release(dgx_domain *d) {
-  void *ptrs[] = {d->d_tab, d->d_metric, d->d_fnorm, d->d_fjr, d->d_nbr, d->d_nside, d->d_flag,
+  void *ptrs[] = {d->d_tab, d->d_metric, d->d_fnorm, d->d_fjr, d->d_nbr, d->d_nside, d->d_link2, d->d_flag,
                   d->d_permid, d->d_perm, d->U, d->Ut, d->R0, d->R1, d->T, d->G, d->V, d->TV, d->nodal,
                   d->T2, d->Vf, d->TVf, d->d_gm, d->d_fgeo, d->d_jav, d->d_pre, d->d_iters, d->Bal, d->d_master,
                   d->d_fcode, d->d_fconst, d->d_fxy, d->d_xn, d->d_J, d->d_cgeo, d->d_part, d->d_chol,
@@ -1412,7 +1422,7 @@ int dgx_domain_bytes(const dgx_domain_desc *desc, size_t *bytes) {
     b += ne * (nf - 1) * (desc->xnodes ? nq : nm) * w + ne * ns * (nf - 1) * qs * w;
   }
   b += nf * ne * nq * 8;                                    // nodal transfer buffer
-  b += ne * (9 + 4 * ns) * 8 + ne * ns * (4 + 4 + 1);       // geometry and links
+  b += ne * (9 + 4 * ns) * 8 + ne * ns * (4 + 4 + 4 + 1);   // geometry and links
   b += 8 * qs * 2 + (size_t)(1 << 20);                      // orientation tables, tables, rounding
   const bool fns = desc->bc_function || desc->source;
   if (desc->xnodes || fns || !all_quads_affine(desc))   // curved: nodal metrics, face geometry
@@ -1597,6 +1607,7 @@ int dgx_state_device_ptr(dgx_handle h, double **U) {
 int dgx_state_upload(dgx_handle h, const double *U, int layout, int on_device) {
   if (!h || !U) return fail(DGX_ERR_ARGUMENT, "null argument");
   const hipMemcpyKind kind = on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
+  h->t_of = nullptr;
   if (layout == DGX_MODAL) {
     HIPCHK(hipMemcpyAsync(h->U, U, h->state_len() * 8, kind, h->stream));
     return DGX_OK;
@@ -1657,10 +1668,27 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
 #define BL(x) do { hipError_t _e = timed(h, 6, [&] { return (x); }); if (_e != hipSuccess) return fail(DGX_ERR_DEVICE, hipGetErrorString(_e)); } while (0)
   if (st == 0) h->t_step = h->time;
   const double tn = h->t_step;
-  if (inttype == DGX_RK4) {
-    static const double a[3] = {0.5, 0.5, 1.0};
-    static const double b[4] = {0.16666666666666667, 0.33333333333333333, 0.33333333333333333,
-                                0.16666666666666667};
+  static const double a[3] = {0.5, 0.5, 1.0};
+  static const double b[4] = {0.16666666666666667, 0.33333333333333333, 0.33333333333333333, 0.16666666666666667};
+  if (inttype != DGX_LSRK14 && h->nsd == 2 && !h->curved && !h->varp) {
+    // affine quads: one launch per stage; the intermediate states in Ut
+    const int last = nstages(inttype) - 1;
+    dgx::QuadStep q;
+    q.Xn = st == last ? h->U : h->Ut;
+    q.acc = h->R0;
+    q.base = h->U;
+    q.dt = dt;
+    if (inttype == DGX_RK4) {
+      q.mode = st == 0 ? dgx::QS_RK4_FIRST : (st < 3 ? dgx::QS_RK4_MID : dgx::QS_RK4_LAST);
+      q.a = st < 3 ? a[st] : 0.0;
+      q.b = b[st];
+      h->time = tn + (st == 0 || st == 1 ? 0.5 : 1.0) * dt;
+    } else {
+      q.mode = st == 0 ? dgx::QS_TVD_1 : (st == 1 ? dgx::QS_TVD_2 : dgx::QS_TVD_3);
+      h->time = tn + (st == 1 ? 0.5 : 1.0) * dt;
+    }
+    RUN(stage2(h, st == 0 ? h->U : h->Ut, q, traces_ready));
+  } else if (inttype == DGX_RK4) {
     if (st == 0) {
       RUN(residual(h, h->U, h->R0));
       BL(dgx::blas_axpy(-a[0] * dt, h->R0, h->U, h->Ut, n, s));
@@ -1699,7 +1727,7 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
     if (h->fused && !h->bulk) {
       // one fused kernel per stage: residual, register update, next traces
       // (the bulk forcing needs the whole residual before any update)
-      if (!traces_ready) RUN(launch(h, dgx::OP_TRACES, h->U, nullptr));
+      if (!(traces_ready && h->t_of == h->U)) RUN(launch(h, dgx::OP_TRACES, h->U, nullptr));
       if (h->visc) RUN(vterm(h, h->U, h->T));
       dgx::StageLaunch sa = stage_args(h);
       sa.op = 1; sa.update = true; sa.U = h->U; sa.Ut = h->Ut; sa.T = h->T; sa.Tn = h->T2;
@@ -1709,7 +1737,9 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
       std::swap(h->T, h->T2);
       ++h->stages;
     } else if (h->nsd == 2 && !h->curved && !h->varp && !h->bulk) {
-      RUN(step2(h, A, B, dt, traces_ready));
+      dgx::QuadStep q;
+      q.mode = dgx::QS_LSRK; q.Xn = h->U; q.acc = h->Ut; q.a = A; q.b = B; q.dt = dt;
+      RUN(stage2(h, h->U, q, traces_ready));
     } else if (h->nsd == 3 && h->curved && !h->bulk) {
       RUN(step_curved3(h, A, B, dt));
     } else {

@@ -196,6 +196,7 @@ struct Geo {
   const uint8_t *permid;         // [ne][nsides] row of `perm`
   const uint16_t *perm;          // [nperm][QF^(d-1)] own point -> neighbour point
   const uint8_t *master;         // [ne][nsides] 1: master or boundary side, 0: slave
+  const int *link2;              // 2D [ne][4]: (nbr 4 + nside) 2 + (points reversed), or nbr when negative
 };
 
 struct Phys {

@@ -44,12 +44,13 @@ struct dgx_domain {
   std::vector<double> gm_host;   // curved: host copy of the nodal metrics d_gm
   // device
   double *d_tab = nullptr, *d_metric = nullptr, *d_fnorm = nullptr, *d_fjr = nullptr;
-  int *d_nbr = nullptr, *d_nside = nullptr, *d_flag = nullptr;
+  int *d_nbr = nullptr, *d_nside = nullptr, *d_link2 = nullptr, *d_flag = nullptr;
   uint8_t *d_permid = nullptr, *d_master = nullptr;
   uint16_t *d_perm = nullptr;
   double *U = nullptr, *Ut = nullptr, *R0 = nullptr, *R1 = nullptr, *T = nullptr;
   double *G = nullptr, *V = nullptr, *TV = nullptr, *nodal = nullptr, *T2 = nullptr;
   float *Vf = nullptr, *TVf = nullptr;   // viscous terms of the mixed path
+  const double *t_of = nullptr;          // the state whose face traces T holds, where a stage or launch put them
   bool fused = false;   // hex fused stage kernels available for this order
   bool curved = false;  // curved hexes (dgx_curved3d.hip): nodal metrics, mass-matrix projection
   double *d_gm = nullptr, *d_fgeo = nullptr, *d_jav = nullptr;

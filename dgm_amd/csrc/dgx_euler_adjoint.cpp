@@ -48,21 +48,24 @@ struct dgx_euler_adjoint {
   int *d_rec_e = nullptr, *d_grp = nullptr;   // d_grp: receivers grouped by element (ObsArgs)
   int ngrp = 0;
   double *d_rec_w = nullptr, *d_y = nullptr, *d_data = nullptr, *d_J = nullptr, *d_coef = nullptr;
-  double *lamU = nullptr, *lamT = nullptr, *Lt = nullptr, *SB = nullptr;
+  double *lamU = nullptr, *lamT = nullptr, *Lt = nullptr, *SB = nullptr, *TB = nullptr;
   std::vector<double *> snaps;
   int rec_step = -1;       // the step whose stage states the next advance records
-  int have_step = -1;      // the step whose stage states SB holds
+  int have_step = -1;      // the step whose stage states SB and their traces TB hold
   long long fwd_steps = 0, adj_steps = 0;
   int snaps_used = 0;
 
+  bool t_valid = false;    // the domain's T holds the traces of its U
+
   size_t n() const { return (size_t)4 * ne * nm; }
+  size_t nt() const { return (size_t)ne * 16 * (p + 1); }   // face traces of a state
 };
 
 namespace {
 
 void release(dgx_euler_adjoint *a) {
   void *ptrs[] = {a->d_rec_e, a->d_grp, a->d_rec_w, a->d_y, a->d_data, a->d_J, a->d_coef,
-                  a->lamU, a->lamT, a->Lt, a->SB};
+                  a->lamU, a->lamT, a->Lt, a->SB, a->TB};
   for (void *p : ptrs)
     if (p) (void)hipFree(p);
   for (double *s : a->snaps)
@@ -79,41 +82,36 @@ dgx::ObsArgs obs_args(dgx_euler_adjoint *a) {
   return o;
 }
 
-int traces(dgx_euler_adjoint *a, const double *U) {
+int traces(dgx_euler_adjoint *a, const double *U, double *T) {
   dgx_domain *d = a->dom;
   dgx::LaunchArgs la;
-  la.op = dgx::OP_TRACES; la.p = a->p; la.ne = a->ne; la.nfield = 4; la.U = U; la.T = d->T;
+  la.op = dgx::OP_TRACES; la.p = a->p; la.ne = a->ne; la.nfield = 4; la.U = U; la.T = T;
   la.tab = d->tab; la.geo = d->geo; la.phys = d->phys; la.stream = d->stream;
   HIPCHK(dgx::launch_2d(la));
   return DGX_OK;
 }
 
-// one LSRK14 stage of the domain's state: the residual fused with the
-// register update Ut = A Ut - dt R, U += B Ut and with the traces of the new
-// state for the next stage (k_step2); stage 0 evaluates its own traces
-int stage(dgx_euler_adjoint *a, int s) {
+// LSRK14 stage s from the state X with traces T to the state Xn with traces Tn
+// (k_quad2: residual, register update and traces in one launch)
+int stage(dgx_euler_adjoint *a, int s, const double *X, double *T, double *Xn, double *Tn) {
   dgx_domain *d = a->dom;
-  int rc;
-  if (s == 0 && (rc = traces(a, d->U))) return rc;
   dgx::LaunchArgs la;
-  la.op = dgx::OP_STEP; la.p = a->p; la.ne = a->ne; la.nfield = 4; la.eqn = DGX_EULER;
-  la.U = d->U; la.Us = d->U; la.Ut = d->Ut; la.T = d->T; la.Tn = d->T2; la.flag = d->d_flag;
-  la.ca = dgx::kLsrkA[s]; la.cb = dgx::kLsrkB[s]; la.dt = a->dt;
+  la.op = dgx::OP_STAGE; la.p = a->p; la.ne = a->ne; la.nfield = 4; la.eqn = DGX_EULER;
+  la.U = X; la.T = T; la.Tn = Tn; la.flag = d->d_flag;
+  la.step.mode = dgx::QS_LSRK; la.step.Xn = Xn; la.step.acc = d->Ut;
+  la.step.a = dgx::kLsrkA[s]; la.step.b = dgx::kLsrkB[s]; la.step.dt = a->dt;
   la.tab = d->tab; la.geo = d->geo; la.phys = d->phys; la.stream = d->stream;
   HIPCHK(dgx::launch_2d(la));
-  std::swap(d->T, d->T2);
   return DGX_OK;
 }
 
 // out = (dR/dU(U))^T lam; or, with `s` >= 0, reversed LSRK stage s at the
 // stage state U: g = lam + B_s lamU, lamU -= dt (dR/dU(U))^T g, lam = A_s g
-// (lam = lamT, out = lamU).  Overwrites the domain's traces with those of U.
-int vjp(dgx_euler_adjoint *a, const double *U, double *lam, double *out, int s) {
+// (lam = lamT, out = lamU).  T: the face traces of U.
+int vjp(dgx_euler_adjoint *a, const double *U, const double *T, double *lam, double *out, int s) {
   dgx_domain *d = a->dom;
-  int rc = traces(a, U);
-  if (rc) return rc;
   dgx::AdjArgs aa;
-  aa.p = a->p; aa.ne = a->ne; aa.U = U; aa.T = d->T; aa.lam = lam; aa.Lt = a->Lt; aa.out = out;
+  aa.p = a->p; aa.ne = a->ne; aa.U = U; aa.T = T; aa.lam = lam; aa.Lt = a->Lt; aa.out = out;
   aa.gamma = d->gamma; aa.flux = d->phys.flux; aa.geo = d->geo; aa.stream = d->stream;
   if (s >= 0) {
     aa.lamU = out; aa.B = dgx::kLsrkB[s]; aa.A = dgx::kLsrkA[s]; aa.stage = true;
@@ -126,16 +124,28 @@ int vjp(dgx_euler_adjoint *a, const double *U, double *lam, double *out, int s) 
   return DGX_OK;
 }
 
-// forward step k: state_k (in the domain's U) -> state_{k+1}
+// forward step k: state_k (in the domain's U) -> state_{k+1}.  The step to be
+// reversed next runs through the stage buffers, which then hold its stage
+// states and their traces.
 int step_forward(dgx_euler_adjoint *a, int k) {
   dgx_domain *d = a->dom;
-  const size_t n = a->n();
+  const size_t n = a->n(), nt = a->nt();
   const bool record = k == a->rec_step;
+  int rc;
+  if (record) HIPCHK(hipMemcpyAsync(a->SB, d->U, n * 8, hipMemcpyDeviceToDevice, d->stream));
+  if (record && a->t_valid) HIPCHK(hipMemcpyAsync(a->TB, d->T, nt * 8, hipMemcpyDeviceToDevice, d->stream));
+  else if (!a->t_valid && (rc = traces(a, d->U, record ? a->TB : d->T))) return rc;
   for (int s = 0; s < kStages; ++s) {
-    if (record) HIPCHK(hipMemcpyAsync(a->SB + s * n, d->U, n * 8, hipMemcpyDeviceToDevice, d->stream));
-    int rc = stage(a, s);
+    const bool last = s == kStages - 1;
+    if (record)
+      rc = stage(a, s, a->SB + s * n, a->TB + s * nt, last ? d->U : a->SB + (s + 1) * n,
+                 last ? d->T : a->TB + (s + 1) * nt);
+    else
+      rc = stage(a, s, d->U, d->T, d->U, d->T2);
     if (rc) return rc;
+    if (!record) std::swap(d->T, d->T2);
   }
+  a->t_valid = true;
   if (record) a->have_step = k;
   ++a->fwd_steps;
   return DGX_OK;
@@ -153,7 +163,7 @@ int step_adjoint(dgx_euler_adjoint *a, int k) {
     HIPCHK(dgx::launch_pobs2_adj(o));
   }
   for (int s = kStages - 1; s >= 0; --s) {
-    int rc = vjp(a, a->SB + s * n, a->lamT, a->lamU, s);
+    int rc = vjp(a, a->SB + s * n, a->TB + s * a->nt(), a->lamT, a->lamU, s);
     if (rc) return rc;
   }
   a->have_step = -1;
@@ -168,6 +178,7 @@ int upload_state(dgx_euler_adjoint *a, const double *U0) {
   const size_t n = a->n();
   for (size_t i = 0; i < n; ++i)
     if (!std::isfinite(U0[i])) return fail(DGX_ERR_ARGUMENT, "initial state is not finite");
+  a->t_valid = false;
   HIPCHK(hipMemcpyAsync(d->U, U0, n * 8, hipMemcpyHostToDevice, d->stream));
   HIPCHK(hipMemsetAsync(d->Ut, 0, n * 8, d->stream));
   HIPCHK(hipMemsetAsync(d->d_flag, 0, sizeof(int), d->stream));
@@ -258,7 +269,8 @@ int dgx_euler_adjoint_create(const dgx_domain_desc *mesh, const dgx_euler_adjoin
       hipMalloc((void **)&a->d_y, nobs * 8) != hipSuccess || hipMalloc((void **)&a->d_data, nobs * 8) != hipSuccess ||
       hipMalloc((void **)&a->d_J, 8) != hipSuccess || hipMalloc((void **)&a->lamU, n * 8) != hipSuccess ||
       hipMalloc((void **)&a->lamT, n * 8) != hipSuccess || hipMalloc((void **)&a->Lt, nlt * 8) != hipSuccess ||
-      hipMalloc((void **)&a->SB, kStages * n * 8) != hipSuccess)
+      hipMalloc((void **)&a->SB, kStages * n * 8) != hipSuccess ||
+      hipMalloc((void **)&a->TB, kStages * nlt * 8) != hipSuccess)
     return fail_mem("Euler adjoint buffers");
   a->snaps.assign(a->nsnap, nullptr);
   for (int s = 0; s < a->nsnap; ++s)
@@ -321,6 +333,7 @@ int dgx_euler_adjoint_gradient(dgx_euler_adjoint_handle a, const double *U0, con
   a->have_step = -1;
   dgx::Revolve rv;
   rv.restore = [&](int s) {
+    a->t_valid = false;
     if (hipMemcpyAsync(d->U, a->snaps[s], n * 8, hipMemcpyDeviceToDevice, st) != hipSuccess ||
         hipMemsetAsync(d->Ut, 0, n * 8, st) != hipSuccess)
       return fail(DGX_ERR_DEVICE, "checkpoint restore");
@@ -348,7 +361,9 @@ int dgx_euler_adjoint_vjp(dgx_euler_adjoint_handle a, const double *U, const dou
   const size_t n = a->n();
   HIPCHK(hipMemcpyAsync(d->U, U, n * 8, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(a->lamT, lam, n * 8, hipMemcpyHostToDevice, st));
-  int rc = vjp(a, d->U, a->lamT, a->lamU, -1);
+  a->t_valid = false;
+  int rc = traces(a, d->U, d->T);
+  if (!rc) rc = vjp(a, d->U, d->T, a->lamT, a->lamU, -1);
   if (rc) return rc;
   HIPCHK(hipMemcpyAsync(out, a->lamU, n * 8, hipMemcpyDeviceToHost, st));
   HIPCHK(hipStreamSynchronize(st));

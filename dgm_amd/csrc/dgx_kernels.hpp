@@ -14,7 +14,19 @@ enum Op {
   OP_VISC = 3,      // U, G -> viscous volume V, traces TV  (Navier-Stokes)
   OP_FORWARD = 4,   // nodal X -> modal Y
   OP_BACKWARD = 5,  // modal X -> nodal Y
-  OP_STEP = 6       // 2D: U, T [, V, TV] -> one LSRK stage in place: Ut = ca Ut - dt R, U += cb Ut
+  OP_STAGE = 6      // 2D: U, T [, V, TV] -> one stage (QuadStep), and the traces of the new state
+};
+
+// What a 2D stage does with the residual R of its state X: the register
+// updates of the explicit integrators, one stage each (QuadUpdate).  From
+// QS_RK4_MID on they read `base`, the state the step began with.
+enum QuadMode { QS_RESIDUAL, QS_LSRK, QS_RK4_FIRST, QS_TVD_1, QS_RK4_MID, QS_RK4_LAST, QS_TVD_2, QS_TVD_3 };
+struct QuadStep {
+  int mode = QS_RESIDUAL;
+  double *Xn = nullptr;            // the new state (may be X), or the residual
+  double *acc = nullptr;           // LSRK register, RK4 increment
+  const double *base = nullptr;
+  double a = 0.0, b = 0.0, dt = 0.0;
 };
 
 struct LaunchArgs {
@@ -28,15 +40,29 @@ struct LaunchArgs {
   int eqn = 0;                   // eqntype (shallow water: 30)
   double *Bal = nullptr;         // shallow water: the stored first residual
   int bal = 0;                   // 0 no balance term, 1 store the residual in Bal, 2 subtract Bal
-  double *Us = nullptr, *Ut = nullptr;   // OP_STEP: the state (updated in place) and the LSRK register
-  double ca = 0.0, cb = 0.0, dt = 0.0;   // OP_STEP: LSRK coefficients and time step
-  double *Tn = nullptr;                  // OP_STEP: if set, the face traces of the new state go here
+  QuadStep step;                 // OP_STAGE
+  double *Tn = nullptr;          // OP_STAGE: if set, the face traces of the new state go here
   bool mixed = false;            // quads, inviscid: FP32 LDS tensors and contractions (traces, residual, step)
   Tab tab;
   Geo geo;
   Phys phys;
   hipStream_t stream = nullptr;
 };
+
+// Elements per wavefront of a packed 2D stage (dgx_quad2.hpp): the most whose
+// pencils of all fields, and whose face points, fit its 64 lanes.  Packed,
+// fewer and fuller wavefronts run more instructions each, so it pays where an
+// element alone leaves most lanes idle and the mesh still gives every SIMD a
+// wavefront.  Measured per LSRK14 stage, one element per wavefront against
+// packed (Euler, FP64): p = 2 7.8 / 6.9 us at 64^2 and 63 / 38 us at 256^2, but
+// 5.2 / 5.9 us at 32^2; p = 4 10.8 / 11.0 us at 64^2 and 31.2 / 28.7 us at 128^2;
+// p = 5 37.4 / 39.2 us at 128^2, where the larger LDS block costs wavefronts:
+// not packed.
+constexpr int quad_epw(int p, int nf) {
+  const int a = 64 / (nf * (p + 2)), b = 64 / (4 * (p + 1)), m = a < b ? a : b;
+  return p <= 4 && m > 1 ? m : 1;
+}
+constexpr bool quad_packed(int p, int ne) { return ne >= (p <= 3 ? 4096 : 8192); }
 
 // One member request of a batched 2D group (serving): its modal state U,
 // LSRK register Ut, face traces T, balance term, error flag, geometry and
@@ -46,7 +72,7 @@ struct Batch2 {
   int *flag = nullptr;
   Geo geo{};
   Phys phys{};
-  int ne = 0, off = 0, bal = 0;
+  int ne = 0, off = 0, bal = 0;  // off: its first work item (BatchLaunch::packed)
   double dt = 0.0;
 };
 
@@ -66,6 +92,7 @@ struct BatchLaunch {
   double lsrkA[14] = {}, lsrkB[14] = {};   // op 2: the LSRK14 coefficients of every stage
   int grid = 0;                  // op 2, out: workgroups launched
   bool mixed = false;            // FP32 LDS tensors and contractions
+  bool packed = false;           // a work item is quad_epw elements of a member, else one
   hipStream_t stream = nullptr;
 };
 
@@ -180,6 +207,8 @@ struct LinArgs {
   double ca = 0, cb = 0, dt = 0, g = 0;   // LSRK coefficients, source amplitude g(t_stage)
   int ne = 0, p = 0;
   bool adjoint = false;
+  double *Tn = nullptr;          // if set, the face traces of the new state (adjoint: of the next stage's
+  double bn = 0.0;               // register, ca X + bn Y, which Yt then holds) go here
   bool mixed = false;            // FP32 LDS tensors and contractions, FP64 state and registers
   Tab tab;
   Geo geo;

@@ -14,7 +14,7 @@
 #include <type_traits>
 #include <vector>
 
-#include "dgx_kernels.hpp"
+#include "dgx_quad2.hpp"
 
 namespace dgx {
 
@@ -57,327 +57,52 @@ __device__ __forceinline__ void backward2(const Tab &tb, const double *m, double
   __syncthreads();
 }
 
-// Gauss-point traces of the NF fields of element e on its four edges, all
-// fields per contraction (one load phase, four contraction phases).
-// LDS of the traces: A [NF][L2], Kb, Ka [NF][2][L], O [NF][2][QF], carved from `sm`.
-template <int P, int NF>
-constexpr int traces2_lds() { return NF * (P + 1) * (P + 1) + 4 * NF * (P + 1) + 2 * NF * (P + 1); }
-
-template <int P, int NF, typename R>
-__device__ __forceinline__ void traces2_core(const double *__restrict__ U, double *__restrict__ T, int ne, int e,
+// Gauss-point traces of a state's NF fields on the elements' edges.
+template <int P, int NF, int EPW, typename R>
+__device__ __forceinline__ void load_traces2(const double *__restrict__ U, double *__restrict__ T, int ne, int e0,
                                              R *sm) {
-  using S = H2<P>;
-  constexpr int L = S::L, QF = S::QF, L2 = S::L2, NT = S::NT;
-  R *A = sm, *Kb = A + NF * L2, *Ka = Kb + NF * 2 * L, *O = Ka + NF * 2 * L;
+  using S = Q2S<P, NF, EPW>;
+  constexpr int L2 = S::L2, NT = S::NT;
+  R *M = sm, *K = M + S::NM;
   const int tid = threadIdx.x;
-  double *Te = T + (size_t)e * 4 * NF * QF;
-  for (int i = tid; i < NF * L2; i += NT) {
-    const int v = i / L2;
-    A[i] = (R)U[((size_t)v * ne + e) * L2 + (i - v * L2)];
+#pragma unroll
+  for (int k = 0; k < S::NU; ++k) {
+    const int i = tid + k * NT, el = i / (NF * L2), r = i - el * NF * L2, v = r / L2;
+    if (i < S::NM) M[i] = (R)U[((size_t)v * ne + min(e0 + el, ne - 1)) * L2 + (r - v * L2)];
   }
   __syncthreads();
-  contract<NF, L, L, 2, 2, NT>(TE<R, P>::Bend(), A, Kb, tid);   // [NF][L][2]
-  contract<NF, L, L, 1, 2, NT>(TE<R, P>::Bend(), A, Ka, tid);   // [NF][2][L]
-  __syncthreads();
-  contract<NF, L, 2, 1, QF, NT>(TB<R, P>::Bg(), Kb, O, tid);    // [NF][QF][2]: edges 0 / 2
-  __syncthreads();
-  for (int i = tid; i < NF * 2 * QF; i += NT) {
-    const int v = i / (2 * QF), r = i - v * 2 * QF, a = r >> 1, end = r & 1;
-    Te[((end ? 2 : 0) * NF + v) * QF + a] = O[i];
-  }
-  __syncthreads();
-  contract<NF, 2, L, 2, QF, NT>(TB<R, P>::Bg(), Ka, O, tid);    // [NF][2][QF]: edges 3 / 1
-  __syncthreads();
-  for (int i = tid; i < NF * 2 * QF; i += NT) {
-    const int v = i / (2 * QF), r = i - v * 2 * QF, end = r / QF, b = r - end * QF;
-    Te[((end ? 1 : 3) * NF + v) * QF + b] = O[i];
-  }
-  __syncthreads();
-}
-
-template <int P, int NF, typename R = double>
-__device__ __forceinline__ void traces2_elem(const double *__restrict__ U, double *__restrict__ T, int ne, int e) {
-  __shared__ R sm[traces2_lds<P, NF>()];
-  traces2_core<P, NF, R>(U, T, ne, e, sm);
+  quad_traces<P, NF, EPW, R, TE<R, P>>(M, K, T, e0, ne, tid);
 }
 
 template <int P, typename R = double>
 __global__ void __launch_bounds__(64)
-k_traces2(const double *__restrict__ U, double *__restrict__ T, Tab tb, int ne, int nf) {
-  if (nf == 3) traces2_elem<P, 3, R>(U, T, ne, blockIdx.x);
-  else traces2_elem<P, 4, R>(U, T, ne, blockIdx.x);
-}
-
-// Residual of element e (Euler, or with NS the BR1 viscous terms from V, TV);
-// out(o, r) receives the modal residual r at offset o = (v*ne + e)*L2 + k.
-// Every contraction runs on all fields of the element at once, so a pass
-// keeps NF x Q pencils busy instead of Q.
-template <int P, int NF>
-struct H2F {
-  static constexpr int L = P + 1, Q = P + 2, QF = P + 1, L2 = L * L, Q2 = Q * Q;
-  // LDS (doubles): M [NF][L2] (modal, then the modal residual), X1, X2 [NF][Q][L],
-  // N1, N2 [NF][Q2] (nodal state, then the contravariant fluxes), gF [NF][4][QF], H [NF][4][L]
-  static constexpr int NM = NF * L2, NX = NF * Q * L, NN = NF * Q2;
-};
-
-template <int P, int NF, typename R = double>
-__device__ __forceinline__ R *rhs2_smem() {
-  using F = H2F<P, NF>;
-  __shared__ R sm[F::NM + 2 * F::NX + 2 * F::NN + NF * 4 * F::QF + NF * 4 * F::L];
-  return sm;
-}
-
-// Element state modal -> nodal for all NF fields; each thread keeps its nodes
-// k = tid + r*NT in registers (un[r][v]).
-template <int P, int NF, int NPT, typename R = double>
-__device__ __forceinline__ void load_nodal2(const double *__restrict__ U, int ne, int e, R *M, R *X,
-                                            R *N, double (&un)[NPT][NF], int tid) {
-  using F = H2F<P, NF>;
-  constexpr int L = F::L, Q = F::Q, L2 = F::L2, Q2 = F::Q2, NT = 64;
-  for (int i = tid; i < NF * L2; i += NT) {
-    const int v = i / L2;
-    M[i] = (R)U[((size_t)v * ne + e) * L2 + (i - v * L2)];
-  }
-  __syncthreads();
-  contract<NF, L, L, 1, Q, NT>(TE<R, P>::BT(), M, X, tid);   // [NF][Q][L]
-  __syncthreads();
-  contract<NF, Q, L, 2, Q, NT>(TE<R, P>::BT(), X, N, tid);   // [NF][Q][Q]
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < NPT; ++r) {
-    const int k = tid + r * NT;
-#pragma unroll
-    for (int v = 0; v < NF; ++v) un[r][v] = k < Q2 ? N[v * Q2 + k] : 1.0;
+k_traces2(const double *__restrict__ U, double *__restrict__ T, int ne, int nf) {
+  if (nf == 3) {
+    constexpr int E = quad_epw(P, 3);
+    __shared__ R sm[Q2S<P, 3, E>::size];
+    load_traces2<P, 3, E, R>(U, T, ne, blockIdx.x * E, sm);
+  } else {
+    constexpr int E = quad_epw(P, 4);
+    __shared__ R sm[Q2S<P, 4, E>::size];
+    load_traces2<P, 4, E, R>(U, T, ne, blockIdx.x * E, sm);
   }
 }
 
-// Projected strong-form residual of all NF fields from the contravariant
-// fluxes in N1 (r) and N2 (s) and the face terms gF; result in M [NF][L2].
-template <int P, int NF, typename R = double>
-__device__ __forceinline__ void divergence2(R *M, R *X1, R *X2, R *N1, R *N2, const R *gF, R *H, int tid) {
-  using F = H2F<P, NF>;
-  constexpr int L = F::L, Q = F::Q, QF = F::QF, NT = 64;
-  contract<NF, Q, Q, 2, L, NT>(TE<R, P>::BW(), N1, X1, tid);
-  contract<NF, Q, Q, 2, L, NT>(TE<R, P>::QD(), N2, X2, tid);
-  contract<NF, 4, QF, 2, L, NT>(TB<R, P>::PW(), gF, H, tid);
-  __syncthreads();
-  contract<NF, Q, L, 1, L, NT>(TE<R, P>::QD(), X1, M, tid);
-  __syncthreads();
-  contract<NF, Q, L, 1, L, NT, true>(TE<R, P>::BW(), X2, M, tid);
-  __syncthreads();
-}
-
-template <int P, bool NS, typename R = double, class Out>
-__device__ __forceinline__ void rhs2_elem(const double *__restrict__ U, const double *__restrict__ T,
-                                          const double *__restrict__ V, const double *__restrict__ TV,
-                                          const Geo &geo, const Phys &ph, int ne, int e, int *__restrict__ flag,
-                                          Out out) {
-  using F = H2F<P, 4>;
-  constexpr int L = F::L, QF = F::QF, L2 = F::L2, Q2 = F::Q2, NT = 64;
-  constexpr int NPT = (Q2 + NT - 1) / NT;
-  R *M = rhs2_smem<P, 4, R>(), *X1 = M + F::NM, *X2 = X1 + F::NX, *N1 = X2 + F::NX, *N2 = N1 + F::NN;
-  R *gF = N2 + F::NN, *H = gF + 16 * QF;
-  const int tid = threadIdx.x;
-  const double gm1 = ph.gamma - 1.0;
-  double un[NPT][4];
-  load_nodal2<P, 4, NPT, R>(U, ne, e, M, X1, N1, un, tid);
-  bool bad = false;
-  for (int i = tid; i < 4 * QF; i += NT) {
-    const int s = i / QF, a = i - s * QF;
-    const int es = e * 4 + s;
-    const int nb = geo.nbr[es], ns = geo.nside[es];
-    const int an = nb >= 0 ? geo.perm[geo.permid[es] * QF + a] : a;
-    const double nx = geo.fnorm[3 * es], ny = geo.fnorm[3 * es + 1];
-    const double jr = geo.fjr[es];
-    double UL[4], UR[4], FL[4], FR[4], Fh[4], lL, lR;
-    const double *tl = T + ((size_t)e * 4 + s) * 4 * QF;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) UL[v] = tl[v * QF + a];
-    if (nb >= 0) {
-      const double *tr = T + ((size_t)nb * 4 + ns) * 4 * QF;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) UR[v] = tr[v * QF + an];
-    } else {   // boundary side of type -1 - nb (Navier-Stokes meshes have none: rejected at creation)
-      ghost2(-1 - nb, UL, nx, ny, ph.bcU, UR);
-    }
-    bool bl, br;
-    euler_normal_flux2(UL, nx, ny, gm1, FL, lL, bl);
-    euler_normal_flux2(UR, nx, ny, gm1, FR, lR, br);
-    bad |= bl | br;
-    if (ph.flux == 1) {
-      roe_flux2(UL, UR, nx, ny, ph.gamma, FL, Fh);
-    } else {
-      const double lmax = fmax(lL, lR);
-#pragma unroll
-      for (int v = 0; v < 4; ++v) Fh[v] = 0.5 * (FL[v] + FR[v] + lmax * (UL[v] - UR[v]));
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      double g = jr * (Fh[v] - FL[v]);
-      if (NS && v > 0 && nb >= 0) {
-        const double *vl = TV + ((size_t)e * 4 + s) * 3 * QF;
-        const double *vr = TV + ((size_t)nb * 4 + ns) * 3 * QF;
-        g += 0.5 * jr * (vl[(v - 1) * QF + a] + vr[(v - 1) * QF + an]);
-      }
-      gF[(v * 4 + s) * QF + a] = (R)g;
-    }
-  }
-  if (bad) atomicOr(flag, 1);
-  const double *mt = geo.metric + 9 * (size_t)e;
-  const double rx = mt[0], ry = mt[1], sx = mt[3], sy = mt[4];
-#pragma unroll
-  for (int rr = 0; rr < NPT; ++rr) {
-    const int k = tid + rr * NT;
-    if (k >= Q2) continue;
-    const double r = un[rr][0], ru = un[rr][1], rv = un[rr][2], rE = un[rr][3];
-    const double ir = 1.0 / r, u = ru * ir, vv = rv * ir;
-    const double p = gm1 * (rE - 0.5 * (ru * u + rv * vv));
-    const double h = rE + p;
-    const double fx[4] = {ru, ru * u + p, rv * u, u * h}, fy[4] = {rv, ru * vv, rv * vv + p, vv * h};
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      N1[v * Q2 + k] = (R)(rx * fx[v] + ry * fy[v]);
-      N2[v * Q2 + k] = (R)(sx * fx[v] + sy * fy[v]);
-    }
-  }
-  __syncthreads();
-  divergence2<P, 4, R>(M, X1, X2, N1, N2, gF, H, tid);
-  const double cw[4] = {1.0, 1.0, 1.0, 1.0};
-  for (int i = tid; i < 4 * L2; i += NT) {
-    const int v = i / L2, k = i - v * L2, l = k / L, m = k - l * L;
-    double r = M[i] + face_add2<P>(TB<R, P>::Bend(), H + v * 4 * L, l, m, cw);
-    if (NS && v > 0) r -= V[((size_t)e * 3 + (v - 1)) * L2 + k];
-    out(((size_t)v * ne + e) * L2 + k, r);
-  }
-  __syncthreads();
-}
-
-template <int P, bool NS, typename RT = double>
+// One stage of an affine domain (quad_stage): EQ 0 Euler, 1 Navier-Stokes with
+// the BR1 viscous terms V, TV, 2 shallow water.
+template <int P, int EPW, typename R, int EQ>
 __global__ void __launch_bounds__(64)
-k_rhs2(const double *__restrict__ U, const double *__restrict__ T, const double *__restrict__ V,
-       const double *__restrict__ TV, double *__restrict__ R, Tab tb, Geo geo, Phys ph, int ne,
-       int *__restrict__ flag) {
-  rhs2_elem<P, NS, RT>(U, T, V, TV, geo, ph, ne, blockIdx.x, flag, [=](size_t o, double r) { R[o] = r; });
-}
-
-// One LSRK14 stage of an affine 2D domain in one kernel after the traces (and
-// the viscous terms): the residual of element e fused with the register
-// update Ut = A Ut - dt R, U += B Ut in its store, bitwise the same as the
-// residual followed by the axpby and axpy.  An element reads its own modes
-// only (its neighbours' through the traces), before its own store.
-// With Tn, the element then writes the face traces of its new state into Tn
-// (the next stage's traces, in the residual's LDS): it reads back its own
-// modes, which its workgroup has just stored.
-template <int P, bool NS, typename R = double>
-__global__ void __launch_bounds__(64)
-k_step2(double *U, const double *__restrict__ T, const double *__restrict__ V, const double *__restrict__ TV,
-        double *__restrict__ Ut, Geo geo, Phys ph, int ne, int *__restrict__ flag, double A, double B, double mdt,
-        double *__restrict__ Tn) {
-  rhs2_elem<P, NS, R>(U, T, V, TV, geo, ph, ne, blockIdx.x, flag, [=](size_t o, double r) {
-    const double ut = fma(mdt, r, A * Ut[o]);
-    Ut[o] = ut;
-    U[o] = fma(B, ut, U[o]);
-  });
-  if (Tn) traces2_core<P, 4, R>(U, Tn, ne, blockIdx.x, rhs2_smem<P, 4, R>());
-}
-
-// Shallow water (Shallow::time_derivative, src/Shallow.cpp:255-336): flux
-// divergence at the GLL points, Lax-Friedrichs face flux, lift, projection.
-// The balance term (src/Shallow.cpp:251-266): bal 1 stores this residual in
-// Bal and returns R - Bal = 0, bal 2 returns R - Bal.
-template <int P, typename R = double, class Out>
-__device__ __forceinline__ void shallow2_elem(const double *__restrict__ U, const double *__restrict__ T,
-                                              double *__restrict__ Bal, int bal, const Geo &geo, const Phys &ph,
-                                              int ne, int e, int *__restrict__ flag, Out out) {
-  using F = H2F<P, 3>;
-  constexpr int L = F::L, QF = F::QF, L2 = F::L2, Q2 = F::Q2, NT = 64;
-  constexpr int NPT = (Q2 + NT - 1) / NT;
-  R *M = rhs2_smem<P, 3, R>(), *X1 = M + F::NM, *X2 = X1 + F::NX, *N1 = X2 + F::NX, *N2 = N1 + F::NN;
-  R *gF = N2 + F::NN, *H = gF + 12 * QF;
-  const int tid = threadIdx.x;
-  double un[NPT][3];
-  load_nodal2<P, 3, NPT, R>(U, ne, e, M, X1, N1, un, tid);
-  bool bad = false;
-  for (int i = tid; i < 4 * QF; i += NT) {
-    const int s = i / QF, a = i - s * QF;
-    const int es = e * 4 + s;
-    const int nb = geo.nbr[es];
-    const double nx = geo.fnorm[3 * es], ny = geo.fnorm[3 * es + 1];
-    const double jr = geo.fjr[es];
-    double UL[3], UR[3], FL[3], FR[3], lL, lR;
-    const double *tl = T + ((size_t)e * 4 + s) * 3 * QF;
-#pragma unroll
-    for (int v = 0; v < 3; ++v) UL[v] = tl[v * QF + a];
-    if (nb < 0) {
-      ghost_shallow2(-1 - nb, UL, nx, ny, ph.bcU, UR);
-    } else {
-      const int an = geo.perm[geo.permid[es] * QF + a];
-      const double *tr = T + ((size_t)nb * 4 + geo.nside[es]) * 3 * QF;
-#pragma unroll
-      for (int v = 0; v < 3; ++v) UR[v] = tr[v * QF + an];
-    }
-    bad |= shallow_normal_flux2(UL, nx, ny, FL, lL);
-    bad |= shallow_normal_flux2(UR, nx, ny, FR, lR);
-    const double lmax = fmax(lL, lR);
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-      const double Fh = 0.5 * (FL[v] + FR[v] + lmax * (UL[v] - UR[v]));
-      gF[(v * 4 + s) * QF + a] = (R)(jr * (Fh - FL[v]));
-    }
-  }
-  if (bad) atomicOr(flag, 1);
-  const double *mt = geo.metric + 9 * (size_t)e;
-  const double rx = mt[0], ry = mt[1], sx = mt[3], sy = mt[4];
-#pragma unroll
-  for (int rr = 0; rr < NPT; ++rr) {
-    const int k = tid + rr * NT;
-    if (k >= Q2) continue;
-    const double phi = un[rr][0], mx = un[rr][1], my = un[rr][2];
-    const double u = mx / phi, vv = my / phi, p = 0.5 * (phi * phi);
-    const double fx[3] = {mx, mx * u + p, my * u}, fy[3] = {my, mx * vv, my * vv + p};
-#pragma unroll
-    for (int v = 0; v < 3; ++v) {
-      N1[v * Q2 + k] = (R)(rx * fx[v] + ry * fy[v]);
-      N2[v * Q2 + k] = (R)(sx * fx[v] + sy * fy[v]);
-    }
-  }
-  __syncthreads();
-  divergence2<P, 3, R>(M, X1, X2, N1, N2, gF, H, tid);
-  const double cw[4] = {1.0, 1.0, 1.0, 1.0};
-  for (int i = tid; i < 3 * L2; i += NT) {
-    const int v = i / L2, k = i - v * L2, l = k / L, m = k - l * L;
-    const double r = M[i] + face_add2<P>(TB<R, P>::Bend(), H + v * 4 * L, l, m, cw);
-    const size_t o = ((size_t)v * ne + e) * L2 + k;
-    if (bal == 0) {
-      out(o, r);
-    } else {
-      double b;
-      if (bal == 1) { b = r; Bal[o] = r; }
-      else b = Bal[o];
-      out(o, -1.0 * b + r);
-    }
-  }
-  __syncthreads();
-}
-
-template <int P, typename RT = double>
-__global__ void __launch_bounds__(64)
-k_shallow2(const double *__restrict__ U, const double *__restrict__ T, double *__restrict__ R,
-           double *__restrict__ Bal, int bal, Tab tb, Geo geo, Phys ph, int ne, int *__restrict__ flag) {
-  shallow2_elem<P, RT>(U, T, Bal, bal, geo, ph, ne, blockIdx.x, flag, [=](size_t o, double r) { R[o] = r; });
-}
-
-template <int P, typename R = double>
-__global__ void __launch_bounds__(64)
-k_shallow_step2(double *U, const double *__restrict__ T, double *__restrict__ Ut, double *__restrict__ Bal, int bal,
-                Geo geo, Phys ph, int ne, int *__restrict__ flag, double A, double B, double mdt,
-                double *__restrict__ Tn) {
-  shallow2_elem<P, R>(U, T, Bal, bal, geo, ph, ne, blockIdx.x, flag, [=](size_t o, double r) {
-    const double ut = fma(mdt, r, A * Ut[o]);
-    Ut[o] = ut;
-    U[o] = fma(B, ut, U[o]);
-  });
-  if (Tn) traces2_core<P, 3, R>(U, Tn, ne, blockIdx.x, rhs2_smem<P, 3, R>());
+k_quad2(const double *X, const double *__restrict__ T, const double *__restrict__ V, const double *__restrict__ TV,
+        Geo geo, Phys ph, int ne, int *__restrict__ flag, QuadStep s, double *Bal, int bal, double *__restrict__ Tn) {
+  constexpr int NF = EQ == 2 ? 3 : 4;
+  __shared__ R sm[Q2S<P, NF, EPW>::size];
+  const int e0 = xcd_element(blockIdx.x, gridDim.x) * EPW;
+  const QuadUpdate up{s};
+  if constexpr (EQ == 2)
+    quad_stage<P, EPW, R, TE<R, P>, false>(X, T, V, TV, geo, ne, e0, flag, QuadShallow{ph}, QuadBalanced{up, Bal, bal},
+                                           Tn, sm);
+  else
+    quad_stage<P, EPW, R, TE<R, P>, EQ == 1>(X, T, V, TV, geo, ne, e0, flag, QuadEuler{ph}, up, Tn, sm);
 }
 
 // lifted, projected gradients of (u, v, e): G[e][2*prim + dir][L2]
@@ -565,89 +290,17 @@ k_backward2(const double *__restrict__ Fm, double *__restrict__ Fn, Tab tb, int 
 // modal coordinates (exact quadrature throughout), and the kernel performs one
 // reversed stage: Ubar += -dt L^T X, dJ/dtheta_e += 2 g dt X[E][e][0],
 // Ubar_t = ca X.
-template <int P, bool ADJ, typename R = double>
+template <int P, int EPW, bool ADJ, typename R = double>
 __global__ void __launch_bounds__(64)
 k_lin2(LinArgs a) {
-  using F = H2F<P, 4>;
-  constexpr int L = F::L, QF = F::QF, L2 = F::L2, Q2 = F::Q2, NT = 64;
-  constexpr int NPT = (Q2 + NT - 1) / NT;
-  R *M = rhs2_smem<P, 4, R>(), *X1 = M + F::NM, *X2 = X1 + F::NX, *N1 = X2 + F::NX, *N2 = N1 + F::NN;
-  R *gF = N2 + F::NN, *H = gF + 16 * QF;
-  const int e = blockIdx.x, tid = threadIdx.x, ne = a.ne;
-  const Geo &geo = a.geo;
-  const double *mt = geo.metric + 9 * (size_t)e;
-  const double rx = mt[0], ry = mt[1], sx = mt[3], sy = mt[4];
-  const double dm = rx * sy - ry * sx;   // 1 / J_e
-  const double sc = ADJ ? dm : 1.0;
-  double un[NPT][4];
-  load_nodal2<P, 4, NPT, R>(a.X, ne, e, M, X1, N1, un, tid);
-  for (int i = tid; i < 4 * QF; i += NT) {
-    const int s = i / QF, q = i - s * QF;
-    const int es = e * 4 + s;
-    const int nb = geo.nbr[es], ns = geo.nside[es];
-    const int qn = geo.perm[geo.permid[es] * QF + q];
-    const double nx = geo.fnorm[3 * es], ny = geo.fnorm[3 * es + 1];
-    const double jr = geo.fjr[es];
-    double scn = 1.0;
-    if (ADJ) {
-      const double *mn = geo.metric + 9 * (size_t)nb;
-      scn = mn[0] * mn[4] - mn[1] * mn[3];
-    }
-    const double *tl = a.T + ((size_t)e * 4 + s) * 4 * QF;
-    const double *tr = a.T + ((size_t)nb * 4 + ns) * 4 * QF;
-    double UL[4], UR[4];
-#pragma unroll
-    for (int v = 0; v < 4; ++v) { UL[v] = sc * tl[v * QF + q]; UR[v] = scn * tr[v * QF + qn]; }
-    const double lam = fabs(a.u0 * nx + a.v0 * ny) + a.c0;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      double fl = 0.0, fr = 0.0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double An = nx * a.Ax[4 * v + j] + ny * a.Ay[4 * v + j];
-        fl = fma(An, UL[j], fl);
-        fr = fma(An, UR[j], fr);
-      }
-      const double fh = 0.5 * (fl + fr + lam * (UL[v] - UR[v]));
-      gF[(v * 4 + s) * QF + q] = (R)(jr * (fh - fl));
-    }
-  }
-#pragma unroll
-  for (int rr = 0; rr < NPT; ++rr) {
-    const int k = tid + rr * NT;
-    if (k >= Q2) continue;
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      double fx = 0.0, fy = 0.0;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const double u = sc * un[rr][j];
-        fx = fma(a.Ax[4 * v + j], u, fx);
-        fy = fma(a.Ay[4 * v + j], u, fy);
-      }
-      N1[v * Q2 + k] = (R)(rx * fx + ry * fy);
-      N2[v * Q2 + k] = (R)(sx * fx + sy * fy);
-    }
-  }
-  __syncthreads();
-  divergence2<P, 4, R>(M, X1, X2, N1, N2, gF, H, tid);
-  const double cw[4] = {1.0, 1.0, 1.0, 1.0};
-  for (int i = tid; i < 4 * L2; i += NT) {
-    const int v = i / L2, k = i - v * L2, l = k / L, m = k - l * L;
-    double r = M[i] + face_add2<P>(TB<R, P>::Bend(), H + v * 4 * L, l, m, cw);
-    const size_t gi = ((size_t)v * ne + e) * L2 + k;
-    if (!ADJ) {
-      if (v == 3 && k == 0) r -= 2.0 * a.theta[e] * a.g;   // source: mode 0 of the constant theta_e
-      const double ut = a.ca * a.Yt[gi] - a.dt * r;
-      a.Yt[gi] = ut;
-      a.Y[gi] = fma(a.cb, ut, a.Y[gi]);
-    } else {
-      const double x = a.X[gi];
-      a.Y[gi] = fma(-a.dt, r / dm, a.Y[gi]);
-      if (v == 3 && k == 0) a.gtheta[e] += 2.0 * a.g * a.dt * x;
-      a.Yt[gi] = a.ca * x;
-    }
-  }
+  __shared__ R sm[Q2S<P, 4, EPW>::size];
+  const int e0 = xcd_element(blockIdx.x, gridDim.x) * EPW;
+  if constexpr (ADJ)
+    quad_stage<P, EPW, R, TE<R, P>, false>(a.X, a.T, nullptr, nullptr, a.geo, a.ne, e0, nullptr, QuadLinear<true>{a},
+                                           LinearAdjoint{a}, a.Tn, sm);
+  else
+    quad_stage<P, EPW, R, TE<R, P>, false>(a.X, a.T, nullptr, nullptr, a.geo, a.ne, e0, nullptr, QuadLinear<false>{a},
+                                           LinearForward{a}, a.Tn, sm);
 }
 
 // Observations (one workgroup per receiver) and the objective's adjoint (one
@@ -711,41 +364,48 @@ k_observe_adjoint(const double *__restrict__ U, double *__restrict__ Ubar, const
 // are in work-item order, b[r].off their first item.  The step kernel fuses
 // the LSRK14 register update of the direct path (vField axpby, axpy:
 // Ut = A Ut - dt R, U += B Ut) into the residual's store.
-template <int P, int NF, typename R = double>
+template <int P, int E, int NF, typename R = double>
 __global__ void __launch_bounds__(64)
 k_batch_traces2(const Batch2 *__restrict__ b, int nreq, int nwork) {
+  __shared__ R sm[Q2S<P, NF, E>::size];
   int r = 0;
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
     while (r + 1 < nreq && b[r + 1].off <= w) ++r;
-    traces2_elem<P, NF, R>(b[r].U, b[r].T, b[r].ne, w - b[r].off);
+    load_traces2<P, NF, E, R>(b[r].U, b[r].T, b[r].ne, (w - b[r].off) * E, sm);
+    __syncthreads();
   }
+}
+
+// Work item w - off of member m: a stage of its elements.
+template <int P, int E, bool SHALLOW, typename R>
+__device__ __forceinline__ void batch_stage2(const Batch2 &m, int w, const double *Tc, double *Tn, double A, double B,
+                                             R *sm) {
+  const Geo geo = m.geo;
+  const Phys ph = m.phys;
+  QuadStep s;
+  s.mode = QS_LSRK; s.Xn = m.U; s.acc = m.Ut; s.a = A; s.b = B; s.dt = m.dt;
+  const int e0 = (w - m.off) * E;
+  if constexpr (SHALLOW)
+    quad_stage<P, E, R, TE<R, P>, false>(m.U, Tc, nullptr, nullptr, geo, m.ne, e0, m.flag, QuadShallow{ph},
+                                         QuadBalanced{QuadUpdate{s}, m.Bal, m.bal}, Tn, sm);
+  else
+    quad_stage<P, E, R, TE<R, P>, false>(m.U, Tc, nullptr, nullptr, geo, m.ne, e0, m.flag, QuadEuler{ph},
+                                         QuadUpdate{s}, Tn, sm);
+  __syncthreads();
 }
 
 // odd: the stage reads the traces of T2 and writes the next ones into T
 // (else T and T2); next: write the next stage's traces at all.
-template <int P, bool SHALLOW, typename R = double>
+template <int P, int E, bool SHALLOW, typename R = double>
 __global__ void __launch_bounds__(64)
 k_batch_step2(const Batch2 *__restrict__ b, int nreq, int nwork, double A, double B, int odd, int next) {
   constexpr int NF = SHALLOW ? 3 : 4;
+  __shared__ R sm[Q2S<P, NF, E>::size];
   int r = 0;
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
     while (r + 1 < nreq && b[r + 1].off <= w) ++r;
-    const double *Tc = odd ? b[r].T2 : b[r].T;
-    double *Tn = odd ? b[r].T : b[r].T2;
-    double *U = b[r].U, *Ut = b[r].Ut;
-    const double mdt = -b[r].dt;
-    auto update = [=](size_t o, double rr) {
-      const double ut = fma(mdt, rr, A * Ut[o]);   // as the direct path's axpby
-      Ut[o] = ut;
-      U[o] = fma(B, ut, U[o]);
-    };
-    const Geo geo = b[r].geo;
-    const Phys ph = b[r].phys;
-    if constexpr (SHALLOW)
-      shallow2_elem<P, R>(U, Tc, b[r].Bal, b[r].bal, geo, ph, b[r].ne, w - b[r].off, b[r].flag, update);
-    else
-      rhs2_elem<P, false, R>(U, Tc, nullptr, nullptr, geo, ph, b[r].ne, w - b[r].off, b[r].flag, update);
-    if (next) traces2_core<P, NF, R>(U, Tn, b[r].ne, w - b[r].off, rhs2_smem<P, NF, R>());
+    batch_stage2<P, E, SHALLOW, R>(b[r], w, odd ? b[r].T2 : b[r].T, next ? (odd ? b[r].T : b[r].T2) : nullptr, A, B,
+                                   sm);
   }
 }
 
@@ -764,51 +424,37 @@ struct LsrkTab {
 // the even number of stages of a step the current traces are in T again.
 // Each element's arithmetic is that of k_batch_traces2 and k_batch_step2, so
 // the results are bitwise those of the per-stage launches.
-template <int P, bool SHALLOW, typename R = double>
+template <int P, int E, bool SHALLOW, typename R = double>
 __global__ void __launch_bounds__(64)
 k_batch_persist2(const Batch2 *__restrict__ b, int nreq, int nwork, int nsteps, LsrkTab c) {
   constexpr int NF = SHALLOW ? 3 : 4;
+  __shared__ R sm[Q2S<P, NF, E>::size];
   cooperative_groups::grid_group grid = cooperative_groups::this_grid();
   {
     int r = 0;
     for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
       while (r + 1 < nreq && b[r + 1].off <= w) ++r;
-      traces2_core<P, NF, R>(b[r].U, b[r].T, b[r].ne, w - b[r].off, rhs2_smem<P, NF, R>());
+      load_traces2<P, NF, E, R>(b[r].U, b[r].T, b[r].ne, (w - b[r].off) * E, sm);
+      __syncthreads();
     }
   }
   grid.sync();
   for (int step = 0; step < nsteps; ++step)
     for (int st = 0; st < 14; ++st) {
-      const double A = c.A[st], B = c.B[st];
       const bool odd = st & 1, last = step == nsteps - 1 && st == 13;
       int r = 0;
       for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
         while (r + 1 < nreq && b[r + 1].off <= w) ++r;
-        const int e = w - b[r].off, ne = b[r].ne;
-        double *U = b[r].U, *Ut = b[r].Ut;
-        const double *Tc = odd ? b[r].T2 : b[r].T;
-        double *Tn = odd ? b[r].T : b[r].T2;
-        const double mdt = -b[r].dt;
-        auto update = [=](size_t o, double rr) {
-          const double ut = fma(mdt, rr, A * Ut[o]);   // as the direct path's axpby
-          Ut[o] = ut;
-          U[o] = fma(B, ut, U[o]);
-        };
-        const Geo geo = b[r].geo;
-        const Phys ph = b[r].phys;
-        if constexpr (SHALLOW)
-          shallow2_elem<P, R>(U, Tc, b[r].Bal, b[r].bal, geo, ph, ne, e, b[r].flag, update);
-        else
-          rhs2_elem<P, false, R>(U, Tc, nullptr, nullptr, geo, ph, ne, e, b[r].flag, update);
-        if (!last) traces2_core<P, NF, R>(U, Tn, ne, e, rhs2_smem<P, NF, R>());   // its new state, read back
+        batch_stage2<P, E, SHALLOW, R>(b[r], w, odd ? b[r].T2 : b[r].T, last ? nullptr : (odd ? b[r].T : b[r].T2),
+                                       c.A[st], c.B[st], sm);
       }
       grid.sync();
     }
 }
 
-template <int P, bool SHALLOW, typename R>
+template <int P, int E, bool SHALLOW, typename R>
 static hipError_t launch_persist2(BatchLaunch &a) {
-  const void *kern = reinterpret_cast<const void *>(&k_batch_persist2<P, SHALLOW, R>);
+  const void *kern = reinterpret_cast<const void *>(&k_batch_persist2<P, E, SHALLOW, R>);
   int dev = 0, ncu = 0, per = 0;
   hipError_t e;
   if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
@@ -831,29 +477,29 @@ static hipError_t launch_persist2(BatchLaunch &a) {
   return hipLaunchCooperativeKernel(kern, dim3(grid), dim3(64), args, 0, a.stream);
 }
 
-template <int P, typename R>
-static hipError_t launch_batch2_pr(BatchLaunch &a) {
-  if (a.op == 2) return a.shallow ? launch_persist2<P, true, R>(a) : launch_persist2<P, false, R>(a);
+template <int P, int E, bool SHALLOW, typename R>
+static hipError_t launch_batch2_k(BatchLaunch &a) {
+  if (a.op == 2) return launch_persist2<P, E, SHALLOW, R>(a);
   const int grid = std::max(1, std::min(a.nwork, kBatchGrid));
-  if (a.op == 0) {
-    if (a.shallow)
-      hipLaunchKernelGGL((k_batch_traces2<P, 3, R>), dim3(grid), dim3(64), 0, a.stream, a.b, a.nreq, a.nwork);
-    else
-      hipLaunchKernelGGL((k_batch_traces2<P, 4, R>), dim3(grid), dim3(64), 0, a.stream, a.b, a.nreq, a.nwork);
-  } else {
-    if (a.shallow)
-      hipLaunchKernelGGL((k_batch_step2<P, true, R>), dim3(grid), dim3(64), 0, a.stream, a.b, a.nreq, a.nwork,
-                         a.A, a.B, a.odd, a.next);
-    else
-      hipLaunchKernelGGL((k_batch_step2<P, false, R>), dim3(grid), dim3(64), 0, a.stream, a.b, a.nreq, a.nwork,
-                         a.A, a.B, a.odd, a.next);
-  }
+  if (a.op == 0)
+    hipLaunchKernelGGL((k_batch_traces2<P, E, SHALLOW ? 3 : 4, R>), dim3(grid), dim3(64), 0, a.stream, a.b, a.nreq,
+                       a.nwork);
+  else
+    hipLaunchKernelGGL((k_batch_step2<P, E, SHALLOW, R>), dim3(grid), dim3(64), 0, a.stream, a.b, a.nreq, a.nwork,
+                       a.A, a.B, a.odd, a.next);
   return hipGetLastError();
+}
+
+template <int P, bool SHALLOW, typename R>
+static hipError_t launch_batch2_e(BatchLaunch &a) {
+  constexpr int E = quad_epw(P, SHALLOW ? 3 : 4);
+  return a.packed ? launch_batch2_k<P, E, SHALLOW, R>(a) : launch_batch2_k<P, 1, SHALLOW, R>(a);
 }
 
 template <int P>
 static hipError_t launch_batch2_p(BatchLaunch &a) {
-  return a.mixed ? launch_batch2_pr<P, float>(a) : launch_batch2_pr<P, double>(a);
+  if (a.mixed) return a.shallow ? launch_batch2_e<P, true, float>(a) : launch_batch2_e<P, false, float>(a);
+  return a.shallow ? launch_batch2_e<P, true, double>(a) : launch_batch2_e<P, false, double>(a);
 }
 
 hipError_t launch_batch2(BatchLaunch &a) {
@@ -867,17 +513,20 @@ hipError_t launch_batch2(BatchLaunch &a) {
   }
 }
 
+template <int P, int EPW>
+static hipError_t launch_lin2_pe(const LinArgs &a) {
+  const dim3 grid((a.ne + EPW - 1) / EPW);
+  if (a.adjoint && a.mixed) hipLaunchKernelGGL((k_lin2<P, EPW, true, float>), grid, dim3(64), 0, a.stream, a);
+  else if (a.adjoint) hipLaunchKernelGGL((k_lin2<P, EPW, true>), grid, dim3(64), 0, a.stream, a);
+  else if (a.mixed) hipLaunchKernelGGL((k_lin2<P, EPW, false, float>), grid, dim3(64), 0, a.stream, a);
+  else hipLaunchKernelGGL((k_lin2<P, EPW, false>), grid, dim3(64), 0, a.stream, a);
+  return hipGetLastError();
+}
+
 template <int P>
 static hipError_t launch_lin2_p(const LinArgs &a) {
-  if (a.adjoint && a.mixed)
-    hipLaunchKernelGGL((k_lin2<P, true, float>), dim3(a.ne), dim3(64), 0, a.stream, a);
-  else if (a.adjoint)
-    hipLaunchKernelGGL((k_lin2<P, true>), dim3(a.ne), dim3(64), 0, a.stream, a);
-  else if (a.mixed)
-    hipLaunchKernelGGL((k_lin2<P, false, float>), dim3(a.ne), dim3(64), 0, a.stream, a);
-  else
-    hipLaunchKernelGGL((k_lin2<P, false>), dim3(a.ne), dim3(64), 0, a.stream, a);
-  return hipGetLastError();
+  constexpr int E = quad_epw(P, 4);
+  return quad_packed(P, a.ne) ? launch_lin2_pe<P, E>(a) : launch_lin2_pe<P, 1>(a);
 }
 
 hipError_t launch_lin2(const LinArgs &a) {
@@ -904,50 +553,44 @@ hipError_t launch_observe_adjoint(const double *U, double *Ubar, const int *rec_
   return hipGetLastError();
 }
 
+template <int P, int EPW, typename R, int EQ>
+static hipError_t launch_quad2_k(const LaunchArgs &a, const QuadStep &s, double *Tn) {
+  hipLaunchKernelGGL((k_quad2<P, EPW, R, EQ>), dim3((a.ne + EPW - 1) / EPW), dim3(64), 0, a.stream, a.U, a.T, a.V,
+                     a.TV, a.geo, a.phys, a.ne, a.flag, s, a.Bal, a.bal, Tn);
+  return hipGetLastError();
+}
+
+template <int P, typename R, int EQ>
+static hipError_t launch_quad2_e(const LaunchArgs &a, const QuadStep &s, double *Tn) {
+  constexpr int E = quad_epw(P, EQ == 2 ? 3 : 4);
+  return quad_packed(P, a.ne) ? launch_quad2_k<P, E, R, EQ>(a, s, Tn) : launch_quad2_k<P, 1, R, EQ>(a, s, Tn);
+}
+
+template <int P>
+static hipError_t launch_quad2(const LaunchArgs &a, const QuadStep &s, double *Tn) {
+  if (a.eqn == 30) return a.mixed ? launch_quad2_e<P, float, 2>(a, s, Tn) : launch_quad2_e<P, double, 2>(a, s, Tn);
+  if (a.mixed) return launch_quad2_e<P, float, 0>(a, s, Tn);
+  return a.ns ? launch_quad2_e<P, double, 1>(a, s, Tn) : launch_quad2_e<P, double, 0>(a, s, Tn);
+}
+
 template <int P>
 static hipError_t launch2(const LaunchArgs &a) {
   const int ne = a.ne;
   switch (a.op) {
-    case OP_TRACES:
+    case OP_TRACES: {
+      const int E = quad_epw(P, a.nfield), grid = (ne + E - 1) / E;
       if (a.mixed)
-        hipLaunchKernelGGL((k_traces2<P, float>), dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.tab, ne, a.nfield);
+        hipLaunchKernelGGL((k_traces2<P, float>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
       else
-        hipLaunchKernelGGL(k_traces2<P>, dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.tab, ne, a.nfield);
+        hipLaunchKernelGGL(k_traces2<P>, dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
       break;
-    case OP_RHS:
-      if (a.mixed && a.eqn == 30)
-        hipLaunchKernelGGL((k_shallow2<P, float>), dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.R, a.Bal, a.bal,
-                           a.tab, a.geo, a.phys, ne, a.flag);
-      else if (a.mixed)
-        hipLaunchKernelGGL((k_rhs2<P, false, float>), dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.V, a.TV,
-                           a.R, a.tab, a.geo, a.phys, ne, a.flag);
-      else if (a.eqn == 30)
-        hipLaunchKernelGGL(k_shallow2<P>, dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.R, a.Bal, a.bal,
-                           a.tab, a.geo, a.phys, ne, a.flag);
-      else if (a.ns)
-        hipLaunchKernelGGL((k_rhs2<P, true>), dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.V, a.TV,
-                           a.R, a.tab, a.geo, a.phys, ne, a.flag);
-      else
-        hipLaunchKernelGGL((k_rhs2<P, false>), dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.V, a.TV,
-                           a.R, a.tab, a.geo, a.phys, ne, a.flag);
-      break;
-    case OP_STEP:
-      if (a.mixed && a.eqn == 30)
-        hipLaunchKernelGGL((k_shallow_step2<P, float>), dim3(ne), dim3(64), 0, a.stream, a.Us, a.T, a.Ut, a.Bal,
-                           a.bal, a.geo, a.phys, ne, a.flag, a.ca, a.cb, -a.dt, a.Tn);
-      else if (a.mixed)
-        hipLaunchKernelGGL((k_step2<P, false, float>), dim3(ne), dim3(64), 0, a.stream, a.Us, a.T, a.V, a.TV,
-                           a.Ut, a.geo, a.phys, ne, a.flag, a.ca, a.cb, -a.dt, a.Tn);
-      else if (a.eqn == 30)
-        hipLaunchKernelGGL(k_shallow_step2<P>, dim3(ne), dim3(64), 0, a.stream, a.Us, a.T, a.Ut, a.Bal, a.bal,
-                           a.geo, a.phys, ne, a.flag, a.ca, a.cb, -a.dt, a.Tn);
-      else if (a.ns)
-        hipLaunchKernelGGL((k_step2<P, true>), dim3(ne), dim3(64), 0, a.stream, a.Us, a.T, a.V, a.TV, a.Ut,
-                           a.geo, a.phys, ne, a.flag, a.ca, a.cb, -a.dt, a.Tn);
-      else
-        hipLaunchKernelGGL((k_step2<P, false>), dim3(ne), dim3(64), 0, a.stream, a.Us, a.T, a.V, a.TV, a.Ut,
-                           a.geo, a.phys, ne, a.flag, a.ca, a.cb, -a.dt, a.Tn);
-      break;
+    }
+    case OP_RHS: {
+      QuadStep s;
+      s.Xn = a.R;
+      return launch_quad2<P>(a, s, nullptr);
+    }
+    case OP_STAGE: return launch_quad2<P>(a, a.step, a.Tn);
     case OP_GRAD:
       hipLaunchKernelGGL(k_grad2<P>, dim3(ne), dim3(64), 0, a.stream, a.U, a.T, a.G, a.tab, a.geo, ne);
       break;

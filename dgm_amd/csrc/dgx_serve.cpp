@@ -75,6 +75,7 @@ struct Group {
   dgx::Batch2 *dd = nullptr;
   size_t cap = 0;
   int nwork = 0, k = 0;
+  bool packed = false;               // work items of several elements (BatchLaunch::packed)
   bool dirty = true, inflight = false;
   bool shared_stream = false;        // persistent slices: the server's stream
   hipStream_t stream = nullptr;
@@ -221,7 +222,10 @@ int enqueue_group(dgx_server *s, Group *g) {
   if (k <= 0) return DGX_OK;
   if (g->dirty) {
     g->hd.resize(g->members.size());
-    int off = 0;
+    int total = 0, off = 0;
+    for (const Request *r : g->members) total += r->h->ne;
+    g->packed = dgx::quad_packed(g->p, total);
+    const int epw = g->packed ? dgx::quad_epw(g->p, g->eqn == DGX_SHALLOW ? 3 : 4) : 1;   // elements of a work item
     for (size_t i = 0; i < g->members.size(); ++i) {
       const dgx_domain *d = g->members[i]->h;
       dgx::Batch2 &b = g->hd[i];
@@ -229,7 +233,7 @@ int enqueue_group(dgx_server *s, Group *g) {
       b.U = d->U; b.Ut = d->Ut; b.T = d->T; b.T2 = d->T2; b.Bal = d->Bal; b.flag = d->d_flag;
       b.geo = d->geo; b.phys = d->phys; b.ne = d->ne; b.off = off; b.bal = d->bal;
       b.dt = g->members[i]->dt;
-      off += d->ne;
+      off += (d->ne + epw - 1) / epw;
     }
     g->nwork = off;
     if (g->hd.size() > g->cap) {
@@ -247,7 +251,7 @@ int enqueue_group(dgx_server *s, Group *g) {
   }
   dgx::BatchLaunch a;
   a.p = g->p; a.nreq = (int)g->hd.size(); a.nwork = g->nwork; a.shallow = g->eqn == DGX_SHALLOW;
-  a.mixed = g->mixed; a.b = g->dd; a.stream = g->stream;
+  a.mixed = g->mixed; a.packed = g->packed; a.b = g->dd; a.stream = g->stream;
   if (s->cfg.persistent) {   // the whole slice in one cooperative launch
     a.op = 2; a.nsteps = k;
     std::copy(dgx::kLsrkA, dgx::kLsrkA + 14, a.lsrkA);
