@@ -475,13 +475,14 @@ int stage2(dgx_domain *d, const double *X, const dgx::QuadStep &st, bool traces_
   return DGX_OK;
 }
 
-// One LSRK stage of a curved hex domain: the traces, on Navier-Stokes the
-// lifted gradients and viscous terms, then k_rhs3c with the register update
-// fused into its store (bitwise the same as the residual followed by the
-// axpby and axpy).
-int step_curved3(dgx_domain *d, double A, double B, double dt) {
+// One LSRK stage of a curved hex domain: the traces (unless the previous stage
+// of this call wrote them), on Navier-Stokes the lifted gradients and viscous
+// terms, then k_rhs3c with the register update fused into its store (bitwise
+// the same as the residual followed by the axpby and axpy) and the traces of
+// the new state after it.
+int step_curved3(dgx_domain *d, double A, double B, double dt, bool traces_ready) {
   int rc;
-  if ((rc = launch(d, dgx::OP_TRACES, d->U, nullptr))) return rc;
+  if (!(traces_ready && d->t_of == d->U) && (rc = launch(d, dgx::OP_TRACES, d->U, nullptr))) return rc;
   dgx::CurvedArgs ca = curved_args(d);
   ca.U = d->U; ca.T = d->T; ca.R = nullptr;
   for (int op : {1, 2}) {   // Navier-Stokes: lifted gradients, then the viscous terms
@@ -491,9 +492,11 @@ int step_curved3(dgx_domain *d, double A, double B, double dt) {
     if (e != hipSuccess) return fail(DGX_ERR_DEVICE, std::string("curved viscous terms: ") + hipGetErrorString(e));
   }
   ca.op = 0;
-  ca.update = true; ca.Us = d->U; ca.Ut = d->Ut; ca.ca = A; ca.cb = B; ca.dt = dt;
+  ca.update = true; ca.Us = d->U; ca.Ut = d->Ut; ca.Tn = d->T2; ca.ca = A; ca.cb = B; ca.dt = dt;
   hipError_t e = timed(d, dgx::OP_RHS, [&] { return launch_curved(d, ca); });
   if (e != hipSuccess) return fail(DGX_ERR_DEVICE, std::string("curved stage: ") + hipGetErrorString(e));
+  std::swap(d->T, d->T2);        // the next stage's traces
+  d->t_of = d->U;
   ++d->stages;
   return DGX_OK;
 }
@@ -1361,9 +1364,9 @@ int build(dgx_domain *d, const dgx_domain_desc *desc) {
     if ((rc = alloc(&d->d_J, ne))) return rc;
     HIPCHK(hipMemcpy(d->d_J, d->J.data(), ne * sizeof(double), hipMemcpyHostToDevice));
   }
-  // a second trace buffer: the fused hex stages write the next stage's traces
-  // into it; affine quads keep it for the serving loop's persistent slices
-  if ((d->fused || (d->nsd == 2 && !d->curved && !d->varp)) &&
+  // a second trace buffer: the hex stages and those of affine quads write the
+  // next stage's traces into it
+  if ((d->fused || (d->nsd == 3 && d->curved) || (d->nsd == 2 && !d->curved && !desc->porder)) &&
       (rc = alloc(&d->T2, (size_t)ne * d->ns * d->nf * qs)))
     return rc;
   d->mixed = d->prec == DGX_MIXED;
@@ -1415,7 +1418,7 @@ int dgx_domain_bytes(const dgx_domain_desc *desc, size_t *bytes) {
   const bool fused = nsd == 3 && dgx::stage3_supported(desc->p) && !desc->xnodes;
   const bool mixed = desc->precision == DGX_MIXED;
   size_t b = 4 * nf * ne * nm * 8;                          // U, Ut, R0, R1
-  b += (fused || (nsd == 2 && !desc->porder) ? 2 : 1) * ne * ns * nf * qs * 8;   // face traces
+  b += (fused || (nsd == 3 && desc->xnodes) || (nsd == 2 && !desc->porder) ? 2 : 1) * ne * ns * nf * qs * 8;   // face traces
   if (visc) {
     const size_t w = mixed ? 4 : 8;
     if (!fused && !mixed) b += ne * (nsd == 2 ? 6 : 12) * nm * 8;
@@ -1741,7 +1744,7 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
       q.mode = dgx::QS_LSRK; q.Xn = h->U; q.acc = h->Ut; q.a = A; q.b = B; q.dt = dt;
       RUN(stage2(h, h->U, q, traces_ready));
     } else if (h->nsd == 3 && h->curved && !h->bulk) {
-      RUN(step_curved3(h, A, B, dt));
+      RUN(step_curved3(h, A, B, dt, traces_ready));
     } else {
       RUN(residual(h, h->U, h->R0));
       BL(dgx::blas_axpby(-dt, h->R0, A, h->Ut, h->Ut, n, s));

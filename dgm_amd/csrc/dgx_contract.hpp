@@ -1,5 +1,5 @@
-// FP64 sum-factorization contractions over LDS tensors, shared by the fused
-// hex kernels.  One thread owns one pencil at a time and computes all of its
+// Sum-factorization contractions over LDS tensors, shared by the hex kernels
+// (FP64; FP32 in the mixed curved residual).  One thread owns one pencil at a time and computes all of its
 // outputs with the even-odd form of the matrix (dgx_device.hpp), whose
 // coefficients come from constant memory as scalar operands.
 #pragma once
@@ -21,18 +21,18 @@ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 
 // [A][N][B][C] (last-dim pitch PI) -> [A][NO][B][C] (pitch PO), contracting N
 // with an even-odd matrix; one thread computes all outputs of a pencil.
-template <int A, int N, int B, int C, int NO, int PI, int PO, int NT, bool ACC = false, int K>
-__device__ __forceinline__ void con_mid(EoMat<K, double> M, const double *in, double *out, int tid) {
+template <int A, int N, int B, int C, int NO, int PI, int PO, int NT, bool ACC = false, int K, typename T>
+__device__ __forceinline__ void con_mid(EoMat<K, T> M, const T *in, T *out, int tid) {
   constexpr int NP = A * B * C;
   auto pencil = [&](int pc) {
     const int c = pc % C, t = pc / C, b = t % B, a = t / B;
-    double x[N], y[NO];
+    T x[N], y[NO];
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = in[((a * N + i) * B + b) * PI + c];
     eo_apply<K, N, NO>(M.h, x, y);
 #pragma unroll
     for (int o = 0; o < NO; ++o) {
-      double *dst = out + ((a * NO + o) * B + b) * PO + c;
+      T *dst = out + ((a * NO + o) * B + b) * PO + c;
       if (ACC) *dst += y[o]; else *dst = y[o];
     }
   };
@@ -44,10 +44,10 @@ __device__ __forceinline__ void con_mid(EoMat<K, double> M, const double *in, do
 }
 
 // [R][NI] (pitch PI) -> [R][NO] (pitch PO), contracting the last dimension.
-template <int R, int NI, int NO, int PI, int PO, int NT, int K>
-__device__ __forceinline__ void con_last(EoMat<K, double> M, const double *in, double *out, int tid) {
+template <int R, int NI, int NO, int PI, int PO, int NT, int K, typename T>
+__device__ __forceinline__ void con_last(EoMat<K, T> M, const T *in, T *out, int tid) {
   auto pencil = [&](int r) {
-    double x[NI], y[NO];
+    T x[NI], y[NO];
 #pragma unroll
     for (int i = 0; i < NI; ++i) x[i] = in[r * PI + i];
     eo_apply<K, NI, NO>(M.h, x, y);
@@ -58,6 +58,50 @@ __device__ __forceinline__ void con_last(EoMat<K, double> M, const double *in, d
     if (tid < R) pencil(tid);
   } else {
     for (int r = tid; r < R; r += NT) pencil(r);
+  }
+}
+
+// Values at the Gauss points of an element's six faces, Te [6][5][QF^2], of the
+// modal state in A ([5][L][L][L], last pitch odd(L)): the end values across
+// each direction in B (20 L odd(L) + 15 L^2 values), then Bg (x) Bg per pair of
+// faces in A (10 QF max(odd(L), 3 L) + 15 QF^2 values).
+template <int P, int NT>
+__device__ __forceinline__ void face_traces3(double *A, double *B, double *__restrict__ Te, int tid) {
+  constexpr int L = P + 1, QF = P + 1, L2 = L * L, QF2 = QF * QF, LP = odd(L), FP = odd(QF);
+  constexpr int KP = 3;   // pitch of the [..][2] collapse
+  double *K0 = B, *K1 = B + 10 * L * LP, *K2 = B + 20 * L * LP;
+  con_mid<5, L, L, L, 2, LP, LP, NT>(EO<P>::Bend(), A, K0, tid);       // [5][2][L][L]
+  con_mid<5 * L, L, 1, L, 2, LP, LP, NT>(EO<P>::Bend(), A, K1, tid);   // [5][L][2][L]
+  con_last<5 * L2, L, 2, LP, KP, NT>(EO<P>::Bend(), A, K2, tid);       // [5][L][L][2]
+  __syncthreads();
+  double *W = A, *O = A + 10 * QF * cmax(LP, KP * L);
+  // faces 4 / 2: [5][2][QF][QF]
+  con_mid<10, L, 1, L, QF, LP, LP, NT>(EO<P>::Bg(), K0, W, tid);      // [10][QF][L]
+  __syncthreads();
+  con_last<10 * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);       // [10][QF][QF]
+  __syncthreads();
+  for (int i = tid; i < 10 * QF2; i += NT) {
+    const int ve = i / QF2, q = i - ve * QF2, v = ve >> 1, end = ve & 1;
+    Te[((end ? 2 : 4) * 5 + v) * QF2 + q] = O[(ve * QF + q / QF) * FP + q % QF];
+  }
+  // faces 1 / 3: [5][QF][2][QF]
+  con_mid<5, L, 2, L, QF, LP, LP, NT>(EO<P>::Bg(), K1, W, tid);       // [5][QF][2][L]
+  __syncthreads();
+  con_last<10 * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);       // [5][QF][2][QF]
+  __syncthreads();
+  for (int i = tid; i < 10 * QF2; i += NT) {
+    const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
+    const int ia = q / QF, ic = q - ia * QF;
+    Te[((end ? 3 : 1) * 5 + v) * QF2 + q] = O[((v * QF + ia) * 2 + end) * FP + ic];
+  }
+  // faces 0 / 5: [5][QF][QF][2]
+  con_mid<5, L, L, 2, QF, KP, KP, NT>(EO<P>::Bg(), K2, W, tid);       // [5][QF][L][2]
+  __syncthreads();
+  con_mid<5 * QF, L, 1, 2, QF, KP, KP, NT>(EO<P>::Bg(), W, O, tid);   // [5][QF][QF][2]
+  __syncthreads();
+  for (int i = tid; i < 10 * QF2; i += NT) {
+    const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
+    Te[((end ? 5 : 0) * 5 + v) * QF2 + q] = O[(v * QF2 + q) * KP + end];
   }
 }
 

@@ -186,6 +186,20 @@ struct EoBaseD {
 };
 template <int P> using EO = EOx<EoBaseD, P>;
 
+// p as a pointer to memory that no thread writes while the kernel runs, the
+// same for the whole wavefront: its loads are scalar loads.  The compiler sees
+// a new pointer at each call, so that it loads a loop's coefficients where
+// they are used; hoisted out of the loop, several matrices at once overflow
+// the scalar registers and come back lane by lane from vector registers.
+template <typename T> __device__ __forceinline__ const T *uniform_const(const T *p) {
+  auto q = (const __attribute__((address_space(4))) T *)p;
+  asm volatile("" : "+s"(q));
+  return (const T *)q;
+}
+template <int K, typename T> __device__ __forceinline__ EoMat<K, T> fresh(EoMat<K, T> M) {
+  return {uniform_const(M.h)};
+}
+
 // Per-element affine geometry and face links (device memory).
 struct Geo {
   const double *metric;          // [ne][9]: rx ry rz sx sy sz tx ty tz

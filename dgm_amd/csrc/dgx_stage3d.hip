@@ -344,44 +344,7 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
     }
   }
   __syncthreads();
-  constexpr int KP = 3;   // pitch of the [..][2] collapse
-  double *K0 = B, *K1 = B + 10 * L * LP, *K2 = B + 20 * L * LP;
-  con_mid<5, L, L, L, 2, LP, LP, NT>(EO<P>::Bend(), A, K0, tid);       // [5][2][L][L]
-  con_mid<5 * L, L, 1, L, 2, LP, LP, NT>(EO<P>::Bend(), A, K1, tid);   // [5][L][2][L]
-  con_last<5 * L2, L, 2, LP, KP, NT>(EO<P>::Bend(), A, K2, tid);       // [5][L][L][2]
-  __syncthreads();
-  double *W = A, *O = A + 10 * QF * cmax(LP, KP * L);
-  double *Te = a.Tn + (size_t)e * 6 * 5 * QF2;
-  // faces 4 / 2: [5][2][QF][QF]
-  con_mid<10, L, 1, L, QF, LP, LP, NT>(EO<P>::Bg(), K0, W, tid);      // [10][QF][L]
-  __syncthreads();
-  con_last<10 * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);       // [10][QF][QF]
-  __syncthreads();
-  for (int i = tid; i < 10 * QF2; i += NT) {
-    const int ve = i / QF2, q = i - ve * QF2, v = ve >> 1, end = ve & 1;
-    Te[((end ? 2 : 4) * 5 + v) * QF2 + q] = O[(ve * QF + q / QF) * FP + q % QF];
-  }
-  __syncthreads();
-  // faces 1 / 3: [5][QF][2][QF]
-  con_mid<5, L, 2, L, QF, LP, LP, NT>(EO<P>::Bg(), K1, W, tid);       // [5][QF][2][L]
-  __syncthreads();
-  con_last<10 * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);       // [5][QF][2][QF]
-  __syncthreads();
-  for (int i = tid; i < 10 * QF2; i += NT) {
-    const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
-    const int ia = q / QF, ic = q - ia * QF;
-    Te[((end ? 3 : 1) * 5 + v) * QF2 + q] = O[((v * QF + ia) * 2 + end) * FP + ic];
-  }
-  __syncthreads();
-  // faces 0 / 5: [5][QF][QF][2]
-  con_mid<5, L, L, 2, QF, KP, KP, NT>(EO<P>::Bg(), K2, W, tid);       // [5][QF][L][2]
-  __syncthreads();
-  con_mid<5 * QF, L, 1, 2, QF, KP, KP, NT>(EO<P>::Bg(), W, O, tid);   // [5][QF][QF][2]
-  __syncthreads();
-  for (int i = tid; i < 10 * QF2; i += NT) {
-    const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
-    Te[((end ? 5 : 0) * 5 + v) * QF2 + q] = O[(v * QF2 + q) * KP + end];
-  }
+  face_traces3<P, NT>(A, B, a.Tn + (size_t)e * 6 * 5 * QF2, tid);
 }
 
 // Last contraction of the lifted gradient along reference direction D for the

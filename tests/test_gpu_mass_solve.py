@@ -1,0 +1,61 @@
+"""The curved hexes' mass solve where its corrections converge slowly: hexes
+twisted so far that the Jacobian varies up to fivefold inside an element and
+is not separable (a correction leaves 14-39 % of the residual, and the solve
+goes on by conjugate gradients), and slightly (3-6 %, either way), for every
+order, one to two fields short of a wavefront and beyond one.  Residuals
+against the CPU oracle, which factors the mass matrices.
+"""
+import numpy as np
+import pytest
+
+from dgm_amd import dgx, mesh as meshgen
+from oracle_lib import Oracle
+
+pytestmark = pytest.mark.gpu
+
+
+def _twist(a):
+    def fn(x, y, z):
+        s = a * np.sin(2 * np.pi * x) * np.sin(2 * np.pi * y) * np.sin(2 * np.pi * z)
+        return x + s, y + s, z + s
+    return fn
+
+
+def _state(x):
+    s = [np.sin(2 * np.pi * (x[0] + 0.1 * k)) * np.cos(2 * np.pi * (x[1] - x[2] + 0.2 * k)) for k in range(5)]
+    return np.stack([1.0 + 0.1 * s[0], 0.3 + 0.1 * s[1], 0.1 * s[2] - 0.1, 0.1 * s[3], 2.5 + 0.1 * s[4]])
+
+
+def _rel(a, b):
+    return np.sqrt(((a - b) ** 2).sum((1, 2)) / (b ** 2).sum((1, 2)))
+
+
+@pytest.mark.parametrize("eqn,p,a", [(8, 1, 0.1), (8, 2, 0.1), (8, 3, 0.02), (8, 4, 0.1), (8, 5, 0.02), (8, 5, 0.1),
+                                     (8, 6, 0.08), (8, 7, 0.1), (8, 8, 0.05), (9, 1, 0.08), (9, 2, 0.1),
+                                     (9, 4, 0.02), (9, 4, 0.1), (9, 5, 0.1), (9, 7, 0.05)])
+def test_rhs_on_strongly_curved_hexes(eqn, p, a):
+    print(f"[mass solve] eqn={eqn} p={p} twist={a}", flush=True)
+    vis = 0.01 if eqn == 9 else 0.0
+    m = meshgen.periodic_hexes(2, 2, 2)
+    xn = meshgen.mapped_nodes(m, p, _twist(a))
+    orc = Oracle(m, p, eqn, vis=vis)
+    orc.set_nodes(xn)
+    orc.set_state(_state(xn))
+    orc.project_state()
+    Up = orc.state()
+    gpu = dgx.GPUDomain(m, p, eqn, vis=vis, xnodes=xn)
+    gpu.upload(Up)
+    F, ref = gpu.rhs(), orc.rhs(Up)
+    its = gpu.solver_iterations()
+    gpu.close()
+    # the residual's own sensitivity: a random last-bit change of the state
+    # moves the oracle's by this much, and two orders of summation cannot agree
+    # better; three times it covers the two evaluations and the solve
+    rng = np.random.default_rng(1)
+    moved = orc.rhs(Up * (1.0 + 2.2e-16 * rng.choice([-1.0, 1.0], Up.shape)))
+    bar = np.maximum(1e-12, 3.0 * _rel(moved, ref))
+    err = _rel(F, ref)
+    print(f"[mass solve] rel L2 per field: {err}, bar {bar}, {its} iterations", flush=True)
+    assert np.all(err <= bar), err
+    if a >= 0.05 and p >= 2:
+        assert its > 8, its      # the slow path was taken
