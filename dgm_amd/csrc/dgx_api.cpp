@@ -456,7 +456,7 @@ int residual_core(dgx_domain *d, const double *U, double *R) {
 // traces (unless an earlier stage of this call wrote them) and the viscous
 // terms, then the residual fused with the register update `st` and with the
 // traces of the new state (k_quad2).
-int stage2(dgx_domain *d, const double *X, const dgx::QuadStep &st, bool traces_ready) {
+int stage2(dgx_domain *d, const double *X, const dgx::StageStep &st, bool traces_ready) {
   int rc;
   if (!(traces_ready && d->t_of == X) && (rc = launch(d, dgx::OP_TRACES, X, nullptr))) return rc;
   if (d->visc) {
@@ -471,6 +471,32 @@ int stage2(dgx_domain *d, const double *X, const dgx::QuadStep &st, bool traces_
   std::swap(d->T, d->T2);        // the next stage's traces
   d->t_of = st.Xn;
   if (d->bal == 1) d->bal = 2;   // the first residual is stored
+  ++d->stages;
+  return DGX_OK;
+}
+
+// One stage of an affine hex domain (fused, FP64) at the state X, as stage2;
+// the channel's bulk forcing needs the whole residual (into R1) and its means
+// before the update.
+int stage3(dgx_domain *d, const double *X, const dgx::StageStep &st, bool traces_ready) {
+  int rc;
+  if (!(traces_ready && d->t_of == X) && (rc = launch(d, dgx::OP_TRACES, X, nullptr))) return rc;
+  if (d->visc && (rc = vterm(d, X, d->T))) return rc;
+  dgx::StageLaunch s = stage_args(d);
+  s.op = 1; s.U = const_cast<double *>(X); s.T = d->T; s.V = d->V; s.TV = d->TV;
+  s.update = !d->bulk; s.step = st; s.Tn = d->T2; s.R = d->R1;
+  if ((rc = launch_stage(d, s))) return rc;
+  if (d->bulk) {
+    dgx::LaunchArgs a = launch_args(d, dgx::OP_UPDATE, X, d->R1);
+    a.step = st; a.Tn = d->T2; a.mean = d->d_J + d->ne;
+    hipError_t e = timed(d, 6, [&] {
+      hipError_t f = dgx::bulk_mean(d->R1, d->d_J, d->ne, d->nm, d->nf, d->d_J + d->ne, d->stream);
+      return f == hipSuccess ? dgx::launch_3d(a) : f;
+    });
+    if (e != hipSuccess) return fail(DGX_ERR_DEVICE, std::string("bulk forcing: ") + hipGetErrorString(e));
+  }
+  std::swap(d->T, d->T2);        // the next stage's traces
+  d->t_of = st.Xn;
   ++d->stages;
   return DGX_OK;
 }
@@ -1361,7 +1387,7 @@ int build(dgx_domain *d, const dgx_domain_desc *desc) {
   }
   if (desc->bulk_forcing) {
     d->bulk = true;
-    if ((rc = alloc(&d->d_J, ne))) return rc;
+    if ((rc = alloc(&d->d_J, (size_t)ne + 3))) return rc;   // Jacobians, then the three means
     HIPCHK(hipMemcpy(d->d_J, d->J.data(), ne * sizeof(double), hipMemcpyHostToDevice));
   }
   // a second trace buffer: the hex stages and those of affine quads write the
@@ -1440,7 +1466,7 @@ int dgx_domain_bytes(const dgx_domain_desc *desc, size_t *bytes) {
   if (nsd == 2) b += ne * 5 * ((desc->xnodes || fns || !all_quads_affine(desc)) ? nq : 1) * 8;   // CFL geometry
   if (nsd == 2 && (desc->xnodes || fns || !all_quads_affine(desc)) && ne * nm * (nm + 1) / 2 * 8 <= (size_t(1) << 30))
     b += ne * nm * (nm + 1) / 2 * 8;                        // curved quads: mass-matrix factors
-  if (desc->bulk_forcing) b += ne * 8;
+  if (desc->bulk_forcing) b += (ne + 3) * 8;
   *bytes = b;
   return DGX_OK;
 }
@@ -1673,24 +1699,33 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
   const double tn = h->t_step;
   static const double a[3] = {0.5, 0.5, 1.0};
   static const double b[4] = {0.16666666666666667, 0.33333333333333333, 0.33333333333333333, 0.16666666666666667};
-  if (inttype != DGX_LSRK14 && h->nsd == 2 && !h->curved && !h->varp) {
-    // affine quads: one launch per stage; the intermediate states in Ut
+  const bool hex = h->fused && !h->mixed, quad = h->nsd == 2 && !h->curved && !h->varp;
+  if (hex || quad) {
+    // affine elements: the whole stage in one kernel after the viscous terms;
+    // RK4 and TVD-RK3 keep the intermediate states in Ut
     const int last = nstages(inttype) - 1;
-    dgx::QuadStep q;
-    q.Xn = st == last ? h->U : h->Ut;
-    q.acc = h->R0;
+    const bool lsrk = inttype == DGX_LSRK14;
+    const double *X = st == 0 || lsrk ? h->U : h->Ut;
+    dgx::StageStep q;
+    q.Xn = st == last || lsrk ? h->U : h->Ut;
+    q.acc = lsrk ? h->Ut : h->R0;
     q.base = h->U;
     q.dt = dt;
-    if (inttype == DGX_RK4) {
-      q.mode = st == 0 ? dgx::QS_RK4_FIRST : (st < 3 ? dgx::QS_RK4_MID : dgx::QS_RK4_LAST);
+    if (lsrk) {
+      q.mode = dgx::ST_LSRK;
+      q.a = dgx::kLsrkA[st];
+      q.b = dgx::kLsrkB[st];
+      h->time = st == last ? tn + dt : tn + dgx::kLsrkC[st] * dt;
+    } else if (inttype == DGX_RK4) {
+      q.mode = st == 0 ? dgx::ST_RK4_FIRST : (st < 3 ? dgx::ST_RK4_MID : dgx::ST_RK4_LAST);
       q.a = st < 3 ? a[st] : 0.0;
       q.b = b[st];
       h->time = tn + (st == 0 || st == 1 ? 0.5 : 1.0) * dt;
     } else {
-      q.mode = st == 0 ? dgx::QS_TVD_1 : (st == 1 ? dgx::QS_TVD_2 : dgx::QS_TVD_3);
+      q.mode = st == 0 ? dgx::ST_TVD_1 : (st == 1 ? dgx::ST_TVD_2 : dgx::ST_TVD_3);
       h->time = tn + (st == 1 ? 0.5 : 1.0) * dt;
     }
-    RUN(stage2(h, st == 0 ? h->U : h->Ut, q, traces_ready));
+    RUN(hex ? stage3(h, X, q, traces_ready) : stage2(h, X, q, traces_ready));
   } else if (inttype == DGX_RK4) {
     if (st == 0) {
       RUN(residual(h, h->U, h->R0));
@@ -1727,9 +1762,8 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
   } else {
     const double A = dgx::kLsrkA[st], B = dgx::kLsrkB[st];
     h->time = tn + dgx::kLsrkC[st] * dt;
-    if (h->fused && !h->bulk) {
-      // one fused kernel per stage: residual, register update, next traces
-      // (the bulk forcing needs the whole residual before any update)
+    if (h->fused) {
+      // mixed: one fused kernel per stage: residual, register update, next traces
       if (!(traces_ready && h->t_of == h->U)) RUN(launch(h, dgx::OP_TRACES, h->U, nullptr));
       if (h->visc) RUN(vterm(h, h->U, h->T));
       dgx::StageLaunch sa = stage_args(h);
@@ -1738,11 +1772,8 @@ int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) 
       sa.ca = A; sa.cb = B; sa.dt = dt;
       RUN(launch_stage(h, sa));
       std::swap(h->T, h->T2);
+      h->t_of = h->U;
       ++h->stages;
-    } else if (h->nsd == 2 && !h->curved && !h->varp && !h->bulk) {
-      dgx::QuadStep q;
-      q.mode = dgx::QS_LSRK; q.Xn = h->U; q.acc = h->Ut; q.a = A; q.b = B; q.dt = dt;
-      RUN(stage2(h, h->U, q, traces_ready));
     } else if (h->nsd == 3 && h->curved && !h->bulk) {
       RUN(step_curved3(h, A, B, dt, traces_ready));
     } else {

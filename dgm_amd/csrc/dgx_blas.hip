@@ -35,8 +35,8 @@ __global__ void __launch_bounds__(256) k_scale(double a, double *__restrict__ x,
 // of the mode-0 coefficients from every element's mode 0.  One workgroup; the
 // reduction order is fixed, so the result does not depend on the launch.
 constexpr int kBulkThreads = 1024;
-__global__ void __launch_bounds__(kBulkThreads) k_bulk_hold(double *__restrict__ R, const double *__restrict__ J,
-                                                            int ne, int nm, int nf) {
+__global__ void __launch_bounds__(kBulkThreads) k_bulk_hold(double *R, const double *__restrict__ J, int ne, int nm,
+                                                            int nf, double *__restrict__ mean) {
   __shared__ double red[4][kBulkThreads];
   const int tid = threadIdx.x;
   const int fld[3] = {0, 1, nf - 1};
@@ -58,13 +58,22 @@ __global__ void __launch_bounds__(kBulkThreads) k_bulk_hold(double *__restrict__
   }
   const double inv = 1.0 / red[3][0];
   const double m[3] = {red[0][0] * inv, red[1][0] * inv, red[2][0] * inv};
+  if (mean) {   // the means only
+    if (tid < 3) mean[tid] = m[tid];
+    return;
+  }
   for (int e = tid; e < ne; e += kBulkThreads)
 #pragma unroll
     for (int k = 0; k < 3; ++k) R[((size_t)fld[k] * ne + e) * nm] -= m[k];
 }
 
 hipError_t bulk_hold(double *R, const double *J, int ne, int nm, int nf, hipStream_t s) {
-  hipLaunchKernelGGL(k_bulk_hold, dim3(1), dim3(kBulkThreads), 0, s, R, J, ne, nm, nf);
+  hipLaunchKernelGGL(k_bulk_hold, dim3(1), dim3(kBulkThreads), 0, s, R, J, ne, nm, nf, (double *)nullptr);
+  return hipGetLastError();
+}
+
+hipError_t bulk_mean(const double *R, const double *J, int ne, int nm, int nf, double *mean, hipStream_t s) {
+  hipLaunchKernelGGL(k_bulk_hold, dim3(1), dim3(kBulkThreads), 0, s, const_cast<double *>(R), J, ne, nm, nf, mean);
   return hipGetLastError();
 }
 

@@ -14,6 +14,13 @@ namespace dgx {
 // Threads per workgroup (one element per workgroup) of the fused hex kernels.
 constexpr int kStageThreads = DGX_STAGE_THREADS;
 
+constexpr int round64(int n) { return (n + 63) / 64 * 64; }
+// Wavefronts per SIMD that the LDS of workgroups of nt threads allows, at
+// most 4: the register budget to ask the compiler for.
+constexpr int lds_waves(int lds, int nt) {
+  const int w = (160 * 1024 / lds) * (nt / 64) / 4;
+  return w < 1 ? 1 : (w > 4 ? 4 : w);
+}
 constexpr int odd(int n) { return n | 1; }
 template <int V> struct IC { static constexpr int value = V; };
 constexpr int cmax(int a, int b) { return a > b ? a : b; }

@@ -41,14 +41,6 @@ template <int P> struct TB3<float, P> {
   __device__ static __forceinline__ const float *DN() { return c_tabf3 + (CT<P>::DN() - c_tab); }
 };
 
-constexpr int round64(int n) { return (n + 63) / 64 * 64; }
-// Wavefronts per SIMD that the LDS of workgroups of nt threads allows, at
-// most 4: the register budget to ask the compiler for.
-constexpr int lds_waves(int lds, int nt) {
-  const int w = (160 * 1024 / lds) * (nt / 64) / 4;
-  return w < 1 ? 1 : (w > 4 ? 4 : w);
-}
-
 template <int P> struct C3 {
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1;
   static constexpr int L2 = L * L, L3 = L2 * L, Q2 = Q * Q, Q3 = Q2 * Q, QF2 = QF * QF;

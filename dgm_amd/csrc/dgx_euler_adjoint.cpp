@@ -98,7 +98,7 @@ int stage(dgx_euler_adjoint *a, int s, const double *X, double *T, double *Xn, d
   dgx::LaunchArgs la;
   la.op = dgx::OP_STAGE; la.p = a->p; la.ne = a->ne; la.nfield = 4; la.eqn = DGX_EULER;
   la.U = X; la.T = T; la.Tn = Tn; la.flag = d->d_flag;
-  la.step.mode = dgx::QS_LSRK; la.step.Xn = Xn; la.step.acc = d->Ut;
+  la.step.mode = dgx::ST_LSRK; la.step.Xn = Xn; la.step.acc = d->Ut;
   la.step.a = dgx::kLsrkA[s]; la.step.b = dgx::kLsrkB[s]; la.step.dt = a->dt;
   la.tab = d->tab; la.geo = d->geo; la.phys = d->phys; la.stream = d->stream;
   HIPCHK(dgx::launch_2d(la));

@@ -14,20 +14,64 @@ enum Op {
   OP_VISC = 3,      // U, G -> viscous volume V, traces TV  (Navier-Stokes)
   OP_FORWARD = 4,   // nodal X -> modal Y
   OP_BACKWARD = 5,  // modal X -> nodal Y
-  OP_STAGE = 6      // 2D: U, T [, V, TV] -> one stage (QuadStep), and the traces of the new state
+  OP_STAGE = 6,     // 2D: U, T [, V, TV] -> one stage (StageStep), and the traces of the new state
+  OP_UPDATE = 7     // 3D: U, its residual R -> the update of one stage, and the traces of the new state
 };
 
-// What a 2D stage does with the residual R of its state X: the register
-// updates of the explicit integrators, one stage each (QuadUpdate).  From
-// QS_RK4_MID on they read `base`, the state the step began with.
-enum QuadMode { QS_RESIDUAL, QS_LSRK, QS_RK4_FIRST, QS_TVD_1, QS_RK4_MID, QS_RK4_LAST, QS_TVD_2, QS_TVD_3 };
-struct QuadStep {
-  int mode = QS_RESIDUAL;
+// What a stage does with the residual R of its state X: the register updates
+// of the explicit integrators, one stage each (stage_update).  From ST_RK4_MID
+// on they read `base`, the state the step began with.
+enum StageMode { ST_RESIDUAL, ST_LSRK, ST_RK4_FIRST, ST_TVD_1, ST_RK4_MID, ST_RK4_LAST, ST_TVD_2, ST_TVD_3 };
+struct StageStep {
+  int mode = ST_RESIDUAL;
   double *Xn = nullptr;            // the new state (may be X), or the residual
   double *acc = nullptr;           // LSRK register, RK4 increment
   const double *base = nullptr;
   double a = 0.0, b = 0.0, dt = 0.0;
 };
+
+__host__ __device__ constexpr bool stage_reads_acc(int mode) {
+  return mode == ST_LSRK || mode == ST_RK4_MID || mode == ST_RK4_LAST;
+}
+
+// Entry o of the update from the residual r, the stage's own state x, the
+// register and the step's initial state; returns the new state.  Rounds as the
+// vField BLAS-1 operations of the reference's integrators
+// (src/vField.hpp:1002-1031) applied one by one.
+__device__ __forceinline__ double stage_update(const StageStep &s, size_t o, double r, double x, double acc,
+                                               double base) {
+  double xn, t;
+  switch (s.mode) {
+    case ST_RESIDUAL: s.Xn[o] = r; return 0.0;
+    case ST_LSRK:            // Ut = A Ut - dt R; U += B Ut
+      t = fma(-s.dt, r, s.a * acc);
+      s.acc[o] = t;
+      xn = fma(s.b, t, x);
+      break;
+    case ST_RK4_FIRST:       // w = U - a dt R; k = -b R
+      s.acc[o] = -s.b * r;
+      xn = fma(-s.a * s.dt, r, x);
+      break;
+    case ST_RK4_MID:         // w = U - a dt R; k -= b R
+      s.acc[o] = fma(-s.b, r, acc);
+      xn = fma(-s.a * s.dt, r, base);
+      break;
+    case ST_RK4_LAST:        // k -= b R; U += dt k
+      xn = fma(s.dt, fma(-s.b, r, acc), base);
+      break;
+    case ST_TVD_1:           // w = U - dt R
+      xn = fma(-s.dt, r, x);
+      break;
+    case ST_TVD_2:           // w = 3/4 U + 1/4 (w - dt R)
+      xn = fma(3.0 / 4.0, base, 1.0 / 4.0 * fma(-s.dt, r, x));
+      break;
+    default:                 // U = 2/3 (w - dt R) + 1/3 U
+      xn = fma(2.0 / 3.0, fma(-s.dt, r, x), 1.0 / 3.0 * base);
+      break;
+  }
+  s.Xn[o] = xn;
+  return xn;
+}
 
 struct LaunchArgs {
   int op = 0, p = 0, ne = 0, nfield = 0;
@@ -40,8 +84,9 @@ struct LaunchArgs {
   int eqn = 0;                   // eqntype (shallow water: 30)
   double *Bal = nullptr;         // shallow water: the stored first residual
   int bal = 0;                   // 0 no balance term, 1 store the residual in Bal, 2 subtract Bal
-  QuadStep step;                 // OP_STAGE
-  double *Tn = nullptr;          // OP_STAGE: if set, the face traces of the new state go here
+  StageStep step;                // OP_STAGE, OP_UPDATE
+  double *Tn = nullptr;          // OP_STAGE, OP_UPDATE: if set, the face traces of the new state go here
+  const double *mean = nullptr;  // OP_UPDATE: subtracted from mode 0 of the density, x-momentum and energy residuals
   bool mixed = false;            // quads, inviscid: FP32 LDS tensors and contractions (traces, residual, step)
   Tab tab;
   Geo geo;
@@ -114,6 +159,7 @@ struct StageLaunch {
   int op = 1;                    // 0: BR1 viscous terms (k_vterm3), 1: stage (k_stage3)
   int p = 0, ne = 0;
   bool ns = false, update = false;
+  StageStep step;                // dgx_stage3d.hip, update: the stage from U (mixed: ca, cb, dt on U and Ut)
   const double *T = nullptr, *V = nullptr, *TV = nullptr;
   double *U = nullptr, *Ut = nullptr, *R = nullptr, *Tn = nullptr, *Vw = nullptr, *TVw = nullptr;
   const float *Vf = nullptr, *TVf = nullptr;   // mixed precision: FP32 viscous terms
@@ -327,7 +373,9 @@ hipError_t blas_axpy(double a, const double *x, const double *y, double *z, size
 hipError_t blas_axpby(double a, const double *x, double b, const double *y, double *z, size_t n,
                       hipStream_t s);
 hipError_t blas_scale(double a, double *x, size_t n, hipStream_t s);
-// Channel bulk forcing on a modal residual [nf][ne][nm] of affine elements with Jacobians J[ne].
+// Channel bulk forcing on a modal residual [nf][ne][nm] of affine elements with Jacobians J[ne]; or only its
+// three means, into `mean`.
 hipError_t bulk_hold(double *R, const double *J, int ne, int nm, int nf, hipStream_t s);
+hipError_t bulk_mean(const double *R, const double *J, int ne, int nm, int nf, double *mean, hipStream_t s);
 
 }  // namespace dgx

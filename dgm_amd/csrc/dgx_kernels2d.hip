@@ -93,7 +93,7 @@ k_traces2(const double *__restrict__ U, double *__restrict__ T, int ne, int nf) 
 template <int P, int EPW, typename R, int EQ>
 __global__ void __launch_bounds__(64)
 k_quad2(const double *X, const double *__restrict__ T, const double *__restrict__ V, const double *__restrict__ TV,
-        Geo geo, Phys ph, int ne, int *__restrict__ flag, QuadStep s, double *Bal, int bal, double *__restrict__ Tn) {
+        Geo geo, Phys ph, int ne, int *__restrict__ flag, StageStep s, double *Bal, int bal, double *__restrict__ Tn) {
   constexpr int NF = EQ == 2 ? 3 : 4;
   __shared__ R sm[Q2S<P, NF, EPW>::size];
   const int e0 = xcd_element(blockIdx.x, gridDim.x) * EPW;
@@ -382,8 +382,8 @@ __device__ __forceinline__ void batch_stage2(const Batch2 &m, int w, const doubl
                                              R *sm) {
   const Geo geo = m.geo;
   const Phys ph = m.phys;
-  QuadStep s;
-  s.mode = QS_LSRK; s.Xn = m.U; s.acc = m.Ut; s.a = A; s.b = B; s.dt = m.dt;
+  StageStep s;
+  s.mode = ST_LSRK; s.Xn = m.U; s.acc = m.Ut; s.a = A; s.b = B; s.dt = m.dt;
   const int e0 = (w - m.off) * E;
   if constexpr (SHALLOW)
     quad_stage<P, E, R, TE<R, P>, false>(m.U, Tc, nullptr, nullptr, geo, m.ne, e0, m.flag, QuadShallow{ph},
@@ -554,20 +554,20 @@ hipError_t launch_observe_adjoint(const double *U, double *Ubar, const int *rec_
 }
 
 template <int P, int EPW, typename R, int EQ>
-static hipError_t launch_quad2_k(const LaunchArgs &a, const QuadStep &s, double *Tn) {
+static hipError_t launch_quad2_k(const LaunchArgs &a, const StageStep &s, double *Tn) {
   hipLaunchKernelGGL((k_quad2<P, EPW, R, EQ>), dim3((a.ne + EPW - 1) / EPW), dim3(64), 0, a.stream, a.U, a.T, a.V,
                      a.TV, a.geo, a.phys, a.ne, a.flag, s, a.Bal, a.bal, Tn);
   return hipGetLastError();
 }
 
 template <int P, typename R, int EQ>
-static hipError_t launch_quad2_e(const LaunchArgs &a, const QuadStep &s, double *Tn) {
+static hipError_t launch_quad2_e(const LaunchArgs &a, const StageStep &s, double *Tn) {
   constexpr int E = quad_epw(P, EQ == 2 ? 3 : 4);
   return quad_packed(P, a.ne) ? launch_quad2_k<P, E, R, EQ>(a, s, Tn) : launch_quad2_k<P, 1, R, EQ>(a, s, Tn);
 }
 
 template <int P>
-static hipError_t launch_quad2(const LaunchArgs &a, const QuadStep &s, double *Tn) {
+static hipError_t launch_quad2(const LaunchArgs &a, const StageStep &s, double *Tn) {
   if (a.eqn == 30) return a.mixed ? launch_quad2_e<P, float, 2>(a, s, Tn) : launch_quad2_e<P, double, 2>(a, s, Tn);
   if (a.mixed) return launch_quad2_e<P, float, 0>(a, s, Tn);
   return a.ns ? launch_quad2_e<P, double, 1>(a, s, Tn) : launch_quad2_e<P, double, 0>(a, s, Tn);
@@ -586,7 +586,7 @@ static hipError_t launch2(const LaunchArgs &a) {
       break;
     }
     case OP_RHS: {
-      QuadStep s;
+      StageStep s;
       s.Xn = a.R;
       return launch_quad2<P>(a, s, nullptr);
     }

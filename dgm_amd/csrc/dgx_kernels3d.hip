@@ -9,6 +9,7 @@
 //   numerical flux   Euler3d::convective_flux (LF)          src/Euler3d.cpp:584-817
 //   lift + project   Hex::lift, Element::project            src/Hex.cpp:1786-1952, src/Element.hpp:427-437
 //   BR1 viscous      Navier_Stokes3d::diffusion             src/Navier_Stokes3d.cpp:182-391
+#include "dgx_contract.hpp"
 #include "dgx_kernels.hpp"
 
 namespace dgx {
@@ -83,54 +84,50 @@ __device__ __forceinline__ void face_project3(const Tab &tb, const double *g, do
 // ---------------------------------------------------------------------------
 // Face traces: modal U -> conservative values at the Gauss points of all six
 // faces, T[e][s][field][a] (face-local order of src/Hex.cpp:817-866).
+// All five fields per contraction, one thread per pencil.
+template <int P> struct T3 {
+  static constexpr int L = P + 1, QF = P + 1, L2 = L * L, L3 = L2 * L, QF2 = QF * QF, LP = odd(L);
+  static constexpr int NT = round64(5 * L2) < 512 ? round64(5 * L2) : 512;
+  static constexpr int NA = cmax(5 * L2 * LP, 10 * QF * cmax(LP, 3 * L) + 15 * QF2);   // modal state, then faces
+  static constexpr int lds = (NA + 20 * L * LP + 15 * L2) * 8;
+};
+
 template <int P>
-__global__ void __launch_bounds__(H3<P>::NT)
-k_traces3(const double *__restrict__ U, double *__restrict__ T, Tab tb, int ne, int nf) {
-  using S = H3<P>;
-  constexpr int L = S::L, QF = S::QF, L2 = S::L2, L3 = S::L3, QF2 = S::QF2, NT = S::NT;
+__global__ void __launch_bounds__(T3<P>::NT)
+k_traces3(const double *__restrict__ U, double *__restrict__ T, int ne) {
+  using S = T3<P>;
+  constexpr int L = S::L, L2 = S::L2, L3 = S::L3, LP = S::LP, NT = S::NT;
   extern __shared__ double sm[];
-  double *A = sm, *K0 = A + L3, *K1 = K0 + 2 * L2, *K2 = K1 + 2 * L2;
-  double *W = K2 + 2 * L2, *O = W + 2 * QF * L;
   const int e = xcd_element(blockIdx.x, ne), tid = threadIdx.x;
-  for (int v = 0; v < nf; ++v) {
-    copy_block<NT>(U + ((size_t)v * ne + e) * L3, A, L3, tid);
-    __syncthreads();
-    contract<L, L, L, 0, 2, NT>(EO<P>::Bend(), A, K0, tid);
-    contract<L, L, L, 1, 2, NT>(EO<P>::Bend(), A, K1, tid);
-    contract<L, L, L, 2, 2, NT>(EO<P>::Bend(), A, K2, tid);
-    __syncthreads();
-    double *Te = T + (size_t)e * 6 * nf * QF2;
-    // faces 4 (xi=-1) and 2 (xi=+1): [2][QF(b)][QF(c)]
-    contract<2, L, L, 1, QF, NT>(EO<P>::Bg(), K0, W, tid);
-    __syncthreads();
-    contract<2, QF, L, 2, QF, NT>(EO<P>::Bg(), W, O, tid);
-    __syncthreads();
-    for (int i = tid; i < 2 * QF2; i += NT) {
-      const int end = i / QF2, a = i - end * QF2;
-      Te[((end ? 2 : 4) * nf + v) * QF2 + a] = O[i];
-    }
-    __syncthreads();
-    // faces 1 (eta=-1) and 3 (eta=+1): [QF(a)][2][QF(c)]
-    contract<L, 2, L, 0, QF, NT>(EO<P>::Bg(), K1, W, tid);
-    __syncthreads();
-    contract<QF, 2, L, 2, QF, NT>(EO<P>::Bg(), W, O, tid);
-    __syncthreads();
-    for (int i = tid; i < 2 * QF2; i += NT) {
-      const int ia = i / (2 * QF), r = i - ia * 2 * QF, end = r / QF, ic = r - end * QF;
-      Te[((end ? 3 : 1) * nf + v) * QF2 + ia * QF + ic] = O[i];
-    }
-    __syncthreads();
-    // faces 0 (zeta=-1) and 5 (zeta=+1): [QF(a)][QF(b)][2]
-    contract<L, L, 2, 0, QF, NT>(EO<P>::Bg(), K2, W, tid);
-    __syncthreads();
-    contract<QF, L, 2, 1, QF, NT>(EO<P>::Bg(), W, O, tid);
-    __syncthreads();
-    for (int i = tid; i < 2 * QF2; i += NT) {
-      const int ab = i >> 1, end = i & 1;
-      Te[((end ? 5 : 0) * nf + v) * QF2 + ab] = O[i];
-    }
-    __syncthreads();
+  for (int i = tid; i < 5 * L3; i += NT) {
+    const int v = i / L3, m = i - v * L3;
+    sm[(v * L2 + m / L) * LP + m % L] = U[((size_t)v * ne + e) * L3 + m];
   }
+  __syncthreads();
+  face_traces3<P, NT>(sm, sm + S::NA, T + (size_t)e * 30 * S::QF2, tid);
+}
+
+// The register update of one stage whose residual needed the whole domain
+// first (the channel's bulk forcing: `mean` is subtracted from mode 0 of the
+// density, x-momentum and energy), with the traces of the new state.
+template <int P>
+__global__ void __launch_bounds__(T3<P>::NT)
+k_update3(const double *X, const double *__restrict__ R, const double *__restrict__ mean, StageStep s,
+          double *__restrict__ Tn, int ne) {
+  using S = T3<P>;
+  constexpr int L = S::L, L2 = S::L2, L3 = S::L3, LP = S::LP, NT = S::NT;
+  extern __shared__ double sm[];
+  const int e = xcd_element(blockIdx.x, ne), tid = threadIdx.x;
+  for (int i = tid; i < 5 * L3; i += NT) {
+    const int v = i / L3, m = i - v * L3;
+    const size_t o = ((size_t)v * ne + e) * L3 + m;
+    double r = R[o];
+    if (m == 0 && (v < 2 || v == 4)) r -= mean[v < 2 ? v : 2];
+    sm[(v * L2 + m / L) * LP + m % L] = stage_update(s, o, r, X[o], stage_reads_acc(s.mode) ? s.acc[o] : 0.0,
+                                                     s.mode >= ST_RK4_MID ? s.base[o] : 0.0);
+  }
+  __syncthreads();
+  face_traces3<P, NT>(sm, sm + S::NA, Tn + (size_t)e * 30 * S::QF2, tid);
 }
 
 // ---------------------------------------------------------------------------
@@ -492,7 +489,6 @@ static int lds3(int which) {
   constexpr int L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2, L2 = S::L2, Q = S::Q, L = S::L, QF = S::QF,
                 Q2 = S::Q2;
   switch (which) {
-    case 0: return (L3 + 6 * L2 + 2 * QF * L + 2 * QF2) * 8;                       // traces
     case 1: return (5 * Q3 + 30 * QF2 + Q3 + S::SX + S::SY) * 8;                  // rhs
     case 2: return (5 * Q3 + 24 * QF2 + Q3 + 2 * S::SX + 3 * Q * L2 + 3 * L3) * 8;  // grad
     case 3: {                                                                     // visc
@@ -510,8 +506,15 @@ static hipError_t launch3(const LaunchArgs &a) {
   const int ne = a.ne;
   switch (a.op) {
     case OP_TRACES: {
-      const int sh = lds3<P>(0);
-      hipLaunchKernelGGL(k_traces3<P>, dim3(ne), dim3(S::NT), sh, a.stream, a.U, a.T, a.tab, ne, 5);
+      const int sh = T3<P>::lds;
+      (void)hipFuncSetAttribute((const void *)k_traces3<P>, hipFuncAttributeMaxDynamicSharedMemorySize, sh);
+      hipLaunchKernelGGL(k_traces3<P>, dim3(ne), dim3(T3<P>::NT), sh, a.stream, a.U, a.T, ne);
+      break;
+    }
+    case OP_UPDATE: {
+      const int sh = T3<P>::lds;
+      (void)hipFuncSetAttribute((const void *)k_update3<P>, hipFuncAttributeMaxDynamicSharedMemorySize, sh);
+      hipLaunchKernelGGL(k_update3<P>, dim3(ne), dim3(T3<P>::NT), sh, a.stream, a.U, a.R, a.mean, a.step, a.Tn, ne);
       break;
     }
     case OP_RHS: {

@@ -132,47 +132,15 @@ template <bool SC> struct QuadLinear {
 
 // What a stage does with its residual r: x is the stage's own state, pre the
 // inputs loaded with it; returns the state whose traces the stage writes.
-// The updates round as the vField BLAS-1 operations of the reference's
-// integrators (src/vField.hpp:1002-1031) applied one by one.
 struct QuadUpdate {
   static constexpr int NPRE = 2;
-  QuadStep s;
+  StageStep s;
   __device__ __forceinline__ void pre(size_t o, int, int, double *p) const {
-    p[0] = s.mode == QS_LSRK || s.mode == QS_RK4_MID || s.mode == QS_RK4_LAST ? s.acc[o] : 0.0;
-    p[1] = s.mode >= QS_RK4_MID ? s.base[o] : 0.0;
+    p[0] = stage_reads_acc(s.mode) ? s.acc[o] : 0.0;
+    p[1] = s.mode >= ST_RK4_MID ? s.base[o] : 0.0;
   }
   __device__ __forceinline__ double post(size_t o, int, int, int, double r, double x, const double *p) const {
-    double xn, t;
-    switch (s.mode) {
-      case QS_RESIDUAL: s.Xn[o] = r; return 0.0;
-      case QS_LSRK:            // Ut = A Ut - dt R; U += B Ut
-        t = fma(-s.dt, r, s.a * p[0]);
-        s.acc[o] = t;
-        xn = fma(s.b, t, x);
-        break;
-      case QS_RK4_FIRST:       // w = U - a dt R; k = -b R
-        s.acc[o] = -s.b * r;
-        xn = fma(-s.a * s.dt, r, x);
-        break;
-      case QS_RK4_MID:         // w = U - a dt R; k -= b R
-        s.acc[o] = fma(-s.b, r, p[0]);
-        xn = fma(-s.a * s.dt, r, p[1]);
-        break;
-      case QS_RK4_LAST:        // k -= b R; U += dt k
-        xn = fma(s.dt, fma(-s.b, r, p[0]), p[1]);
-        break;
-      case QS_TVD_1:           // w = U - dt R
-        xn = fma(-s.dt, r, x);
-        break;
-      case QS_TVD_2:           // w = 3/4 U + 1/4 (w - dt R)
-        xn = fma(3.0 / 4.0, p[1], 1.0 / 4.0 * fma(-s.dt, r, x));
-        break;
-      default:                 // U = 2/3 (w - dt R) + 1/3 U
-        xn = fma(2.0 / 3.0, fma(-s.dt, r, x), 1.0 / 3.0 * p[1]);
-        break;
-    }
-    s.Xn[o] = xn;
-    return xn;
+    return stage_update(s, o, r, x, p[0], p[1]);
   }
 };
 

@@ -1,9 +1,10 @@
 // Fused hex stage kernels (p <= 9).
 //
-// One workgroup of 512 threads per element for both kernels, two workgroups
-// per CU (4 waves per SIMD, at most 128 VGPRs).  Every sum-factorized
-// contraction runs on all conserved fields of the element at once (pencils of
-// 5 fields x q^2 fill the workgroup instead of q^2 = 81 pencils at p = 7),
+// One workgroup per element for both kernels, one thread per pencil
+// (hex_threads); at p = 7 two workgroups per CU (4 waves per SIMD, at most 128
+// VGPRs).  Every sum-factorized contraction runs on all conserved fields of
+// the element at once (pencils of 5 fields x q^2 fill the workgroup instead of
+// q^2 = 81 pencils at p = 7),
 // nodal values live in registers (one thread per node), and the last
 // contraction of each chain accumulates modal results in registers, so a
 // workgroup needs only two LDS tensors of about 5 q^3 doubles.  The last
@@ -148,28 +149,28 @@ struct StageArgs {
   const double *T;       // face traces of the input state
   const double *V;       // viscous volume term [ne][4][L3] (Navier-Stokes)
   const double *TV;      // viscous normal flux [ne][6][4][QF2] (Navier-Stokes)
-  double *U;             // modal state (read; written when updating)
-  double *Ut;            // LSRK register (update mode)
-  double *R;             // residual output (residual mode)
+  const double *U;       // modal state
+  StageStep s;           // what to do with the residual
   double *Tn;            // traces of the updated state (update mode)
-  double ca, cb, dt;     // Ut = ca*Ut - dt*R ; U += cb*Ut
   int ne;
   int *flag;
 };
 
-// The stage kernel (125 VGPRs, 76 KB LDS at p = 7) runs 8 waves per element:
-// every contraction phase is then a single pass, and a CU holds 4 waves per
-// SIMD instead of 2 within the same LDS.
-constexpr int kStage3Threads = 2 * kStageThreads;
-#ifndef DGX_VTERM_THREADS
-#define DGX_VTERM_THREADS 512
-#endif
-constexpr int kVterm3Threads = DGX_VTERM_THREADS;
+// Threads per element: up to p = 5 one per pencil of 5 fields, so that every
+// contraction phase is a single pass whose lanes are nearly all busy (p = 4:
+// also one per node); from p = 6 on, where the LDS holds two workgroups per
+// CU, 512, for four wavefronts per SIMD (320 at p = 6 were 10 % slower).  512
+// for all orders left 76 % of the lanes idle at p = 3: an Euler LSRK14 step of
+// 1.2 M modes per field 8.31 -> 2.76 ms at p = 2, 4.27 -> 1.83 at p = 3,
+// 2.67 -> 1.70 at p = 4, 2.18 -> 1.62 at p = 5; with BR2 viscous terms 26.9 ->
+// 7.4, 13.8 -> 5.1, 8.0 -> 4.7, 6.2 -> 4.7.
+constexpr int hex_threads(int p) { return p >= 6 ? 512 : (p == 4 ? 256 : round64(5 * (p + 2) * (p + 2))); }
 
 template <int P, bool NS, bool UPDATE>
-__global__ void __launch_bounds__(kStage3Threads)
-k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
-  using S = S3<P, kStage3Threads>;
+__global__ void __launch_bounds__(hex_threads(P))
+__attribute__((amdgpu_waves_per_eu(lds_waves(S3<P, hex_threads(P)>::lds_stage, hex_threads(P)))))
+k_stage3(StageArgs a, Geo geo, Phys ph) {
+  using S = S3<P, hex_threads(P)>;
   constexpr int L = S::L, Q = S::Q, QF = S::QF, L2 = S::L2, L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2,
                 LP = S::LP, FP = S::FP, NT = S::NT, NPT = S::NPT, NSL = S::NSL;
   extern __shared__ double sm[];
@@ -237,7 +238,7 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
     if (i < 5 * L3) A[(m / L + v * L2) * LP + (m % L)] = um[k];
   }
   __syncthreads();
-  backward_batch<P, 5, kStage3Threads>(A, B, tid);
+  backward_batch<P, 5, S::NT>(A, B, tid);
   constexpr int FS = Q * Q * S::QP;   // padded nodal field size
   double un[NPT][5];
 #pragma unroll
@@ -278,7 +279,7 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
       }
     }
     __syncthreads();
-    nodal_deriv<P, 5, d, d != 2, kStage3Threads>(A, B, tid);
+    nodal_deriv<P, 5, d, d != 2, S::NT>(A, B, tid);
     __syncthreads();
   };
   // nodal divergence of the contravariant fluxes (c first: it writes B), then
@@ -286,11 +287,15 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
   vol_dir(IC<2>());
   vol_dir(IC<1>());
   vol_dir(IC<0>());
-  proj_to_regs<P, 5, NSL, kStage3Threads>(A, B, acc, tid);
+  proj_to_regs<P, 5, NSL, S::NT>(A, B, acc, tid);
 
   // the update's inputs (viscous volume term, RK register, state) are loaded
   // before the face projection, whose barriers then cover their latency
-  double vin[NSL][L], utin[NSL][L], uin[NSL][L];
+  // in0: the register, or a TVD-RK3 stage's own state; in1: the state
+  double vin[NSL][L], in0[NSL][L], in1[NSL][L];
+  const bool tvd = a.s.mode >= ST_TVD_2;
+  const double *src0 = tvd ? a.U : (stage_reads_acc(a.s.mode) ? a.s.acc : nullptr);
+  const double *src1 = a.s.mode >= ST_RK4_MID ? a.s.base : a.U;
 #pragma unroll
   for (int k = 0; k < NSL; ++k) {
     const int G = tid + k * NT;
@@ -300,13 +305,13 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
       const bool in = G < 5 * L2;
       const size_t gi = ((size_t)v * ne + e) * L3 + l * L2 + pp;
       vin[k][l] = (NS && in && v > 0) ? a.V[((size_t)e * 4 + (v - 1)) * L3 + l * L2 + pp] : 0.0;
-      utin[k][l] = (UPDATE && in) ? a.Ut[gi] : 0.0;
-      uin[k][l] = (UPDATE && in) ? a.U[gi] : 0.0;
+      in0[k][l] = (UPDATE && in && src0) ? src0[gi] : 0.0;
+      in1[k][l] = (UPDATE && in) ? src1[gi] : 0.0;
     }
   }
 
   // faces: H = (PW (x) PW) gF for 5 fields x 6 faces, in B
-  face_project<P, 30, kStage3Threads>(gF, A, B, tid);
+  face_project<P, 30, S::NT>(gF, A, B, tid);
   const double one6[6] = {1.0, 1.0, 1.0, 1.0, 1.0, 1.0};
 #pragma unroll
   for (int k = 0; k < NSL; ++k) {
@@ -318,15 +323,8 @@ k_stage3(StageArgs a, Tab tb, Geo geo, Phys ph) {
         double r = acc[k][l] + face_sum<P>(B + v * 6 * L * LP, l, m, nn, one6);
         if (NS && v > 0) r -= vin[k][l];
         const size_t gi = ((size_t)v * ne + e) * L3 + l * L2 + pp;
-        if (!UPDATE) {
-          a.R[gi] = r;
-        } else {
-          const double ut = a.ca * utin[k][l] - a.dt * r;
-          const double u = fma(a.cb, ut, uin[k][l]);
-          a.Ut[gi] = ut;
-          a.U[gi] = u;
-          acc[k][l] = u;
-        }
+        if (!UPDATE) a.s.Xn[gi] = r;
+        else acc[k][l] = stage_update(a.s, gi, r, tvd ? in0[k][l] : in1[k][l], in0[k][l], in1[k][l]);
       }
     }
   }
@@ -405,15 +403,13 @@ __device__ __forceinline__ double visc_flux(const double t[6], const double h[3]
 // sum_d dxi_d/dx (D_d + lift of those two faces / |grad xi_d|), and each
 // direction's nodal contribution goes straight into the stress tensor and heat
 // flux at the thread's nodes.
-// Two 512-thread workgroups per CU (4 waves per SIMD) where their LDS fits,
-// which needs at most 128 VGPRs.
 template <int P, bool BR2>
-__global__ void __launch_bounds__(kVterm3Threads)
-__attribute__((amdgpu_waves_per_eu((BR2 ? S3<P, kVterm3Threads>::lds_vterm_br2 : S3<P, kVterm3Threads>::lds_vterm) <=
-                                           80 * 1024 ? 4 : 1)))
+__global__ void __launch_bounds__(hex_threads(P))
+__attribute__((amdgpu_waves_per_eu(lds_waves(BR2 ? S3<P, hex_threads(P)>::lds_vterm_br2 : S3<P, hex_threads(P)>::lds_vterm,
+                                             hex_threads(P)))))
 k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__restrict__ V,
-         double *__restrict__ TV, Tab tb, Geo geo, Phys ph, int ne) {
-  using S = S3<P, kVterm3Threads>;
+         double *__restrict__ TV, Geo geo, Phys ph, int ne) {
+  using S = S3<P, hex_threads(P)>;
   constexpr int L = S::L, Q = S::Q, QF = S::QF, L2 = S::L2, L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2,
                 LP = S::LP, QP = S::QP, FP = S::FP, NT = S::NT, NPT = S::NPT, NSG = S::NSG;
   extern __shared__ double sm[];
@@ -693,29 +689,30 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
 template <int P>
 static hipError_t launch_stage3_p(const StageLaunch &s) {
   StageArgs a;
-  a.T = s.T; a.V = s.V; a.TV = s.TV; a.U = s.U; a.Ut = s.Ut; a.R = s.R; a.Tn = s.Tn;
-  a.ca = s.ca; a.cb = s.cb; a.dt = s.dt; a.ne = s.ne; a.flag = s.flag;
+  constexpr int NT = hex_threads(P);
+  a.T = s.T; a.V = s.V; a.TV = s.TV; a.U = s.U; a.s = s.step; a.Tn = s.Tn; a.ne = s.ne; a.flag = s.flag;
+  if (!s.update) { a.s = StageStep(); a.s.Xn = s.R; }
   if (s.op == 0) {
     if (s.phys.visc == 1) {
-      const int sh = S3<P, kVterm3Threads>::lds_vterm_br2;
+      const int sh = S3<P, NT>::lds_vterm_br2;
       (void)hipFuncSetAttribute((const void *)k_vterm3<P, true>, hipFuncAttributeMaxDynamicSharedMemorySize, sh);
-      hipLaunchKernelGGL((k_vterm3<P, true>), dim3(s.ne), dim3(kVterm3Threads), sh, s.stream, s.U, s.T, s.Vw,
-                         s.TVw, s.tab, s.geo, s.phys, s.ne);
+      hipLaunchKernelGGL((k_vterm3<P, true>), dim3(s.ne), dim3(NT), sh, s.stream, s.U, s.T, s.Vw,
+                         s.TVw, s.geo, s.phys, s.ne);
     } else {
-      const int sh = S3<P, kVterm3Threads>::lds_vterm;
+      const int sh = S3<P, NT>::lds_vterm;
       (void)hipFuncSetAttribute((const void *)k_vterm3<P, false>, hipFuncAttributeMaxDynamicSharedMemorySize, sh);
-      hipLaunchKernelGGL((k_vterm3<P, false>), dim3(s.ne), dim3(kVterm3Threads), sh, s.stream, s.U, s.T, s.Vw,
-                         s.TVw, s.tab, s.geo, s.phys, s.ne);
+      hipLaunchKernelGGL((k_vterm3<P, false>), dim3(s.ne), dim3(NT), sh, s.stream, s.U, s.T, s.Vw,
+                         s.TVw, s.geo, s.phys, s.ne);
     }
     return hipGetLastError();
   }
-  const int sh = S3<P, kStage3Threads>::lds_stage;
+  const int sh = S3<P, NT>::lds_stage;
 #define DGX_STAGE(NSV, UPD)                                                                          \
   do {                                                                                               \
     (void)hipFuncSetAttribute((const void *)k_stage3<P, NSV, UPD>,                                   \
                               hipFuncAttributeMaxDynamicSharedMemorySize, sh);                       \
-    hipLaunchKernelGGL((k_stage3<P, NSV, UPD>), dim3(s.ne), dim3(kStage3Threads), sh, s.stream, a, s.tab, s.geo, \
-                       s.phys);                                                                      \
+    hipLaunchKernelGGL((k_stage3<P, NSV, UPD>), dim3(s.ne), dim3(NT), sh, s.stream, a, s.geo, s.phys); \
+                                                                                             \
   } while (0)
   if (s.ns) { if (s.update) DGX_STAGE(true, true); else DGX_STAGE(true, false); }
   else { if (s.update) DGX_STAGE(false, true); else DGX_STAGE(false, false); }
