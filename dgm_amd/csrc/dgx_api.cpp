@@ -221,21 +221,14 @@ HostBasis make_basis(int p) {
     b.KE[i] = (double)lo;
     b.KE[Q + i] = (double)hi;
   }
-  // NP1 = BT BW and NPD = BT QD: projection (and projected derivative) from
-  // GLL values back to GLL values, in long double
-  b.NP1.resize(Q * Q); b.NPD.resize(Q * Q);
-  for (int i = 0; i < Q; ++i)
-    for (int m = 0; m < Q; ++m) {
-      ld sp = 0, sd = 0;
-      for (int l = 0; l < L; ++l) {
-        ld qd = 0;
-        for (int j = 0; j < Q; ++j) qd += normleg(l, z[j]) * w[j] * Dl[j * Q + m];
-        sp += normleg(l, z[i]) * normleg(l, z[m]) * w[m];
-        sd += normleg(l, z[i]) * qd;
-      }
-      b.NP1[i * Q + m] = (double)sp;
-      b.NPD[i * Q + m] = (double)sd;
-    }
+  // the order p + 1 mode, of unit length under the GLL weights
+  b.NV.resize(2 * Q);
+  ld nn = 0;
+  for (int i = 0; i < Q; ++i) nn += w[i] * normleg(L, z[i]) * normleg(L, z[i]);
+  for (int i = 0; i < Q; ++i) {
+    b.NV[i] = (double)(normleg(L, z[i]) / sqrtl(nn));
+    b.NV[Q + i] = (double)(w[i] * normleg(L, z[i]) / sqrtl(nn));
+  }
   return b;
 }
 
@@ -249,7 +242,7 @@ int upload_all_tables() {
     HostBasis b = make_basis(p);
     size_t off = dgx::tab_offset(p);
     for (const std::vector<double> *t : {&b.BT, &b.BW, &b.QD, &b.Bg, &b.Bend, &b.PW, &b.Ig, &b.PI, &b.KE, &b.BL, &b.GL,
-                                         &b.D, &b.NP1, &b.NPD}) {
+                                         &b.D, &b.NV}) {
       std::copy(t->begin(), t->end(), packed.begin() + off);
       off += t->size();
     }
@@ -270,7 +263,7 @@ int upload_all_tables() {
     };
     const int L = b.L, Q = b.Q, QF = b.QF;
     rows(b.BW, L, Q, 0); rows(b.QD, L, Q, 1); rows(b.PI, L, Q, 0); rows(b.BL, L, Q, 0); rows(b.PW, L, QF, 0);
-    square(b.Ig, QF, Q); square(b.GL, Q, QF); square(b.D, Q, Q); square(b.NP1, Q, Q); square(b.NPD, Q, Q);
+    square(b.Ig, QF, Q); square(b.GL, Q, QF); square(b.D, Q, Q);
     if (off != (size_t)dgx::tab_offset(p) + dgx::tab_size(p)) return fail(DGX_ERR_ARGUMENT, "table layout");
   }
   hipError_t e;

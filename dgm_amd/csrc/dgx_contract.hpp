@@ -17,9 +17,9 @@ constexpr int kStageThreads = DGX_STAGE_THREADS;
 constexpr int round64(int n) { return (n + 63) / 64 * 64; }
 // Wavefronts per SIMD that the LDS of workgroups of nt threads allows, at
 // most 4: the register budget to ask the compiler for.
-constexpr int lds_waves(int lds, int nt) {
+constexpr int lds_waves(int lds, int nt, int most = 4) {
   const int w = (160 * 1024 / lds) * (nt / 64) / 4;
-  return w < 1 ? 1 : (w > 4 ? 4 : w);
+  return w < 1 ? 1 : (w > most ? most : w);
 }
 constexpr int odd(int n) { return n | 1; }
 template <int V> struct IC { static constexpr int value = V; };
@@ -31,12 +31,13 @@ constexpr int cmax(int a, int b) { return a > b ? a : b; }
 template <int A, int N, int B, int C, int NO, int PI, int PO, int NT, bool ACC = false, int K, typename T>
 __device__ __forceinline__ void con_mid(EoMat<K, T> M, const T *in, T *out, int tid) {
   constexpr int NP = A * B * C;
+  const T *h = uniform_const(M.h);
   auto pencil = [&](int pc) {
     const int c = pc % C, t = pc / C, b = t % B, a = t / B;
     T x[N], y[NO];
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = in[((a * N + i) * B + b) * PI + c];
-    eo_apply<K, N, NO>(M.h, x, y);
+    eo_apply<K, N, NO>(h, x, y);
 #pragma unroll
     for (int o = 0; o < NO; ++o) {
       T *dst = out + ((a * NO + o) * B + b) * PO + c;
@@ -53,11 +54,12 @@ __device__ __forceinline__ void con_mid(EoMat<K, T> M, const T *in, T *out, int 
 // [R][NI] (pitch PI) -> [R][NO] (pitch PO), contracting the last dimension.
 template <int R, int NI, int NO, int PI, int PO, int NT, int K, typename T>
 __device__ __forceinline__ void con_last(EoMat<K, T> M, const T *in, T *out, int tid) {
+  const T *h = uniform_const(M.h);
   auto pencil = [&](int r) {
     T x[NI], y[NO];
 #pragma unroll
     for (int i = 0; i < NI; ++i) x[i] = in[r * PI + i];
-    eo_apply<K, NI, NO>(M.h, x, y);
+    eo_apply<K, NI, NO>(h, x, y);
 #pragma unroll
     for (int o = 0; o < NO; ++o) out[r * PO + o] = y[o];
   };
@@ -135,8 +137,8 @@ __device__ __forceinline__ void br2_flux(R (&fd)[4], const R *Hn, const RT *KE, 
   const bool hi = (f == 2 || f == 3 || f == 5);
   const R c23 = mu * R(2.0 / 3.0);
   R r0 = R(0), r1 = R(0), r2 = R(0), he = R(0);
-#pragma unroll 1
-  for (int d = 0; d < 3; ++d) {   // one direction at a time: fewer live LDS loads
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {   // unrolled: all LDS loads in flight at once
     const int slo = d == 0 ? 4 : (d == 1 ? 1 : 0), shi = d == 0 ? 2 : (d == 1 ? 3 : 5);
     const int x = d == 0 ? i : (d == 1 ? j : k);
     const int t1 = d == 0 ? j : i, t2 = d == 2 ? j : k;

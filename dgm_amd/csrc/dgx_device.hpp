@@ -24,18 +24,18 @@ struct Tab {
 // BT, BW, QD, Bg, Bend, PW, Ig (sizes above), then PI = PW Ig [L][Q] (GLL
 // face layer -> modal face coefficients), KE [2][Q] (KE[s][i] =
 // sum_l Bend[s][l] BT[i][l], the end traces sum_l phi_l(-+1) phi_l(xi_i)),
-// BL [L][Q], GL [Q][QF], DN [Q][Q], NP1 [Q][Q] and NPD [Q][Q] (see CT), then
+// BL [L][Q], GL [Q][QF], DN [Q][Q] and NV [2][Q] (see CT), then
 // the halves of the matrices that act between symmetric point sets (EOx),
 // orders packed in ascending p.
 constexpr int kMaxOrder = 10;
 constexpr int tab_full(int p) {
   return 3 * (p + 2) * (p + 1) + 2 * (p + 1) * (p + 1) + 2 * (p + 1) + (p + 1) * (p + 2) +
-         (p + 1) * (p + 2) + 2 * (p + 2) + (p + 1) * (p + 2) + (p + 2) * (p + 1) + 3 * (p + 2) * (p + 2);
+         (p + 1) * (p + 2) + 2 * (p + 2) + (p + 1) * (p + 2) + (p + 2) * (p + 1) + (p + 2) * (p + 2) + 2 * (p + 2);
 }
 constexpr int half_up(int n) { return (n + 1) / 2; }
 constexpr int tab_half(int p) {
   return 4 * (p + 1) * half_up(p + 2) + (p + 1) * half_up(p + 1) + half_up(p + 1) * (p + 2) +
-         half_up(p + 2) * (p + 1) + 3 * half_up(p + 2) * (p + 2);
+         half_up(p + 2) * (p + 1) + half_up(p + 2) * (p + 2);
 }
 constexpr int tab_size(int p) { return tab_full(p) + tab_half(p); }
 constexpr int tab_offset(int p) {
@@ -64,11 +64,11 @@ template <int P> struct CT {
   __device__ static __forceinline__ const double *BL() { return KE() + 2 * Q; }
   __device__ static __forceinline__ const double *GL() { return BL() + L * Q; }
   __device__ static __forceinline__ const double *DN() { return GL() + Q * QF; }
-  // nodal-to-nodal [Q][Q]: NP1 = BT BW (the L2 projection onto the order-P
-  // modes, evaluated back at the GLL points) and NPD = BT QD (the projected
-  // derivative, at the GLL points)
-  __device__ static __forceinline__ const double *NP1() { return DN() + Q * Q; }
-  __device__ static __forceinline__ const double *NPD() { return NP1() + Q * Q; }
+  // NV [2][Q]: the mode of order P + 1 at the GLL points, of unit length under
+  // the GLL weights, and the same times the weights.  With those, v and w, the
+  // projection of GLL values onto the order-P modes, evaluated back at the
+  // points, is x - v (w . x).
+  __device__ static __forceinline__ const double *NV() { return DN() + Q * Q; }
 };
 
 // Even-odd contractions.  The GLL and Gauss points are symmetric about 0 and
@@ -163,9 +163,8 @@ template <class B, int P> struct EOx {
   using R = typename B::R;
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1, H = half_up(Q), HF = half_up(QF), b = tab_offset(P);
   static constexpr int oBW = b + tab_full(P), oQD = oBW + L * H, oPI = oQD + L * H, oBL = oPI + L * H,
-                       oPW = oBL + L * H, oIg = oPW + L * HF, oGL = oIg + HF * Q, oDN = oGL + H * QF,
-                       oNP1 = oDN + H * Q, oNPD = oNP1 + H * Q;
-  static_assert(oNPD + H * Q == b + tab_size(P), "table layout");
+                       oPW = oBL + L * H, oIg = oPW + L * HF, oGL = oIg + HF * Q, oDN = oGL + H * QF;
+  static_assert(oDN + H * Q == b + tab_size(P), "table layout");
   __device__ static __forceinline__ EoMat<EO_MN, R> BT() { return {B::base() + b}; }
   __device__ static __forceinline__ EoMat<EO_MN, R> Bg() { return {B::base() + b + 3 * Q * L}; }
   __device__ static __forceinline__ EoMat<EO_MN, R> Bend() { return {B::base() + b + 3 * Q * L + QF * L}; }
@@ -177,8 +176,6 @@ template <class B, int P> struct EOx {
   __device__ static __forceinline__ EoMat<EO_NNS, R> Ig() { return {B::base() + oIg}; }
   __device__ static __forceinline__ EoMat<EO_NNS, R> GL() { return {B::base() + oGL}; }
   __device__ static __forceinline__ EoMat<EO_NNA, R> DN() { return {B::base() + oDN}; }
-  __device__ static __forceinline__ EoMat<EO_NNS, R> NP1() { return {B::base() + oNP1}; }
-  __device__ static __forceinline__ EoMat<EO_NNA, R> NPD() { return {B::base() + oNPD}; }
 };
 struct EoBaseD {
   using R = double;
@@ -198,6 +195,14 @@ template <typename T> __device__ __forceinline__ const T *uniform_const(const T 
 }
 template <int K, typename T> __device__ __forceinline__ EoMat<K, T> fresh(EoMat<K, T> M) {
   return {uniform_const(M.h)};
+}
+
+// v, as a new value to the compiler: what a phase derives from it (the indices
+// of a thread's pencils and nodes) is computed there again, instead of being
+// kept in vector registers over the phases between.
+__device__ __forceinline__ int again(int v) {
+  asm volatile("" : "+v"(v));
+  return v;
 }
 
 // Per-element affine geometry and face links (device memory).

@@ -43,10 +43,12 @@ template <int P, int NTH = kStageThreads> struct S3 {
   static constexpr int NSG = (4 * L2 + NT - 1) / NT;    // modal pencil slots (4 fields)
   static constexpr int NG = 30 * QF * FP;               // face corrections
   static constexpr int lds_stage = (2 * NA + NG) * 8;
-  static constexpr int lds_vterm = (2 * NA + 24 * Q * QP) * 8;
+  // gradient kernel: its tensors also hold moment tables [4][Q][Q]
+  static constexpr int NAV = cmax(NA, cmax(24 * Q * QP, 4 * Q2 * QP + 8 * Q * QP));
+  static constexpr int lds_vterm = (2 * NAV + 24 * Q * QP) * 8;
   // BR2: face-lift nodal values, metric rows, end traces (+ layer velocity)
-  static constexpr bool br2_vel_in_b = 42 * Q * QP <= NA;
-  static constexpr int lds_vterm_br2 = (2 * NA + 24 * Q * QP + 16 + 2 * Q + (br2_vel_in_b ? 0 : 18 * Q * QP)) * 8;
+  static constexpr bool br2_vel_in_b = 42 * Q * QP <= NAV;
+  static constexpr int lds_vterm_br2 = (2 * NAV + 24 * Q * QP + 16 + 2 * Q + (br2_vel_in_b ? 0 : 18 * Q * QP)) * 8;
   // padded position of nodal index n = (i*Q + j)*Q + k
   static __device__ __forceinline__ int nidx(int n) { return (n / Q) * QP + (n - (n / Q) * Q); }
 };
@@ -69,7 +71,7 @@ __device__ __forceinline__ void chain_to_regs(EoMat<EO_NM, double> M, const doub
 #pragma unroll
       for (int i = 0; i < Q; ++i) x[i] = in[((f * Q + i) * L + m) * LP + n];
       double y[L];
-      eo_apply<EO_NM, Q, L>(M.h, x, y);
+      eo_apply<EO_NM, Q, L>(fresh(M).h, x, y);
 #pragma unroll
       for (int l = 0; l < L; ++l) acc[k][l] += y[l];
     }
@@ -165,10 +167,18 @@ struct StageArgs {
 // 2.67 -> 1.70 at p = 4, 2.18 -> 1.62 at p = 5; with BR2 viscous terms 26.9 ->
 // 7.4, 13.8 -> 5.1, 8.0 -> 4.7, 6.2 -> 4.7.
 constexpr int hex_threads(int p) { return p >= 6 ? 512 : (p == 4 ? 256 : round64(5 * (p + 2) * (p + 2))); }
+// Wavefronts per SIMD that the register allocation leaves room for, where the
+// LDS does: five at the lowest orders, whose kernels spill eight registers at most
+// for it.  Against four, Euler steps of 4 M modes per field went from 9.48 to 8.10
+// ms at p = 2, 5.86 to 5.52 at p = 3, 5.83 to 5.52 at p = 4, and with BR2 27.8
+// to 25.7 at p = 2; but the Navier-Stokes stage at p = 3 lost 3 % and k_vterm3
+// from p = 3 on gained nothing.
+constexpr int stage_waves(int p, bool ns) { return p > 4 || (ns && p == 3) ? 4 : 5; }
+constexpr int vterm_waves(int p) { return p > 2 ? 4 : 5; }
 
 template <int P, bool NS, bool UPDATE>
 __global__ void __launch_bounds__(hex_threads(P))
-__attribute__((amdgpu_waves_per_eu(lds_waves(S3<P, hex_threads(P)>::lds_stage, hex_threads(P)))))
+__attribute__((amdgpu_waves_per_eu(lds_waves(S3<P, hex_threads(P)>::lds_stage, hex_threads(P), stage_waves(P, NS)))))
 k_stage3(StageArgs a, Geo geo, Phys ph) {
   using S = S3<P, hex_threads(P)>;
   constexpr int L = S::L, Q = S::Q, QF = S::QF, L2 = S::L2, L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2,
@@ -345,16 +355,17 @@ k_stage3(StageArgs a, Geo geo, Phys ph) {
   face_traces3<P, NT>(A, B, a.Tn + (size_t)e * 6 * 5 * QF2, tid);
 }
 
-// Last contraction of the lifted gradient along reference direction D for the
-// 4 primitives: out = NPD x along D plus clo KE_lo Hn[face lo] + chi KE_hi
-// Hn[face hi] (the two face lifts across D at their own GLL points; faces 4/2
-// for a, 1/3 for b, 0/5 for c).  One thread per pencil of 4 Q^2, all Q outputs.
+// Derivative along reference direction D of the 4 primitives' nodal values in
+// [4][Q][Q][Q], plus the face lifts across D: out = DN x along D plus
+// clo KE_lo Hn[face lo] + chi KE_hi Hn[face hi] (at their own GLL points; faces
+// 4/2 for a, 1/3 for b, 0/5 for c).  The pencil's moment w . x (CT::NV) goes to
+// mom[4][Q][Q].  One thread per pencil of 4 Q^2, all Q outputs.
 template <int P, int D, int NT>
-__device__ __forceinline__ void lifted_dir(const double *in, double *out, const double *Hn, double clo, double chi,
-                                           int tid) {
+__device__ __forceinline__ void lifted_dir(const double *in, double *out, double *mom, const double *Hn, double clo,
+                                           double chi, int tid) {
   constexpr int Q = P + 2, QP = odd(Q), HB = Q * QP, NP = 4 * Q * Q;
   constexpr int flo = D == 0 ? 4 : (D == 1 ? 1 : 0), fhi = D == 0 ? 2 : (D == 1 ? 3 : 5);
-  const double *KE = CT<P>::KE();
+  const double *KE = uniform_const(CT<P>::KE()), *w = uniform_const(CT<P>::NV()) + Q;
   for (int pc = tid; pc < NP; pc += NT) {
     const int f = pc / (Q * Q), t = pc - f * Q * Q, t1 = t / Q, t2 = t - t1 * Q;
     // (t1, t2): the two other indices in order; base and stride of the pencil
@@ -367,12 +378,16 @@ __device__ __forceinline__ void lifted_dir(const double *in, double *out, const 
     for (int m = 0; m < Q; ++m) x[m] = in[base + m * stride];
     const double hl = clo * Hn[(f * 6 + flo) * HB + t1 * QP + t2];
     const double hh = chi * Hn[(f * 6 + fhi) * HB + t1 * QP + t2];
+    double s = w[0] * x[0];
+#pragma unroll
+    for (int m = 1; m < Q; ++m) s = fma(w[m], x[m], s);
+    mom[(f * Q + t1) * QP + t2] = s;
     double y[Q];
-    eo_apply<EO_NNA, Q, Q>(EO<P>::NPD().h, x, y);
+    eo_apply<EO_NNA, Q, Q>(fresh(EO<P>::DN()).h, x, y);
 #pragma unroll
     for (int o = 0; o < Q; ++o) {   // KE_hi[o] = KE_lo[rev o]
-      const double s = fma(KE[o], hl, y[o]);
-      out[base + o * stride] = fma(KE[Q - 1 - o], hh, s);
+      const double r = fma(KE[o], hl, y[o]);
+      out[base + o * stride] = fma(KE[Q - 1 - o], hh, r);
     }
   }
 }
@@ -406,14 +421,14 @@ __device__ __forceinline__ double visc_flux(const double t[6], const double h[3]
 template <int P, bool BR2>
 __global__ void __launch_bounds__(hex_threads(P))
 __attribute__((amdgpu_waves_per_eu(lds_waves(BR2 ? S3<P, hex_threads(P)>::lds_vterm_br2 : S3<P, hex_threads(P)>::lds_vterm,
-                                             hex_threads(P)))))
+                                             hex_threads(P), vterm_waves(P)))))
 k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__restrict__ V,
          double *__restrict__ TV, Geo geo, Phys ph, int ne) {
   using S = S3<P, hex_threads(P)>;
   constexpr int L = S::L, Q = S::Q, QF = S::QF, L2 = S::L2, L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2,
                 LP = S::LP, QP = S::QP, FP = S::FP, NT = S::NT, NPT = S::NPT, NSG = S::NSG;
   extern __shared__ double sm[];
-  double *A = sm, *B = A + S::NA, *Jq = B + S::NA;
+  double *A = sm, *B = A + S::NAV, *Jq = B + S::NAV;
   const int e = xcd_element(blockIdx.x, ne), tid = threadIdx.x;
   constexpr int FS = Q * Q * QP;
 
@@ -496,58 +511,126 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
   for (int r = 0; r < NPT; ++r)
 #pragma unroll
     for (int j = 0; j < 9; ++j) tq[r][j] = 0.0;
-  // The lifted gradient along reference direction d, at the GLL nodes: the
-  // projected derivative (BT BW along the two other directions, then BT QD
-  // along d: three contractions on nodal tensors) plus the nodal values of the
-  // two face lifts across d, folded into the last contraction as two more
-  // inputs with the end-trace columns of KE.  Equal to projecting D_d q and the
-  // face terms to modes and evaluating the result back at the nodes.
+  // The lifted gradient along reference direction d is the nodal derivative
+  // D_d, projected onto the order-P modes along the two other directions (along
+  // d the derivative has order P already), plus the nodal values of the face
+  // lifts across d.  A projection takes the part along the order P + 1 mode v
+  // away, x - v (w . x), and commutes with the derivatives, so
+  //   D_a N_b N_c q = D_a q - v_k D_a N_b c_c - v_j D_a c_b,   c_d = w . q along d,
+  // and so on: one contraction of q and of its two moments, which are face
+  // sized, in place of three of q.  Each direction's part goes straight into
+  // the stress tensor and heat flux at the thread's nodes.  What bounds this
+  // kernel is the latency of its phases between barriers, about 50 us each at
+  // p = 7 on 32^3 elements whatever they hold: with the BR2 points' loop below
+  // unrolled it went from 2.05 to 1.93 ms there, a step of 4 M modes per field
+  // from 12.33 to 11.99 ms.
+  constexpr int TB = 4 * Q * QP;   // one [4][Q][Q] table
+  static_assert(4 * FS + 2 * TB <= S::NAV && 6 * TB <= S::NAV, "moment tables");
+  double *cA = A + S::NAV - TB, *cB = B + S::NAV - TB, *cC = B + 4 * FS;
+  const double c43 = mu * (4.0 / 3.0), c23 = mu * (2.0 / 3.0);
+  // physical gradients g[c][x] of (u, v, w, e) -> stress and heat flux
+  auto add_stress = [&](double (&t)[9], const double (&g)[4][3]) {
+    t[0] += c43 * g[0][0] - c23 * (g[1][1] + g[2][2]);
+    t[1] += mu * (g[0][1] + g[1][0]);
+    t[2] += mu * (g[0][2] + g[2][0]);
+    t[3] += c43 * g[1][1] - c23 * (g[0][0] + g[2][2]);
+    t[4] += mu * (g[1][2] + g[2][1]);
+    t[5] += c43 * g[2][2] - c23 * (g[0][0] + g[1][1]);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) t[6 + x] += kap * g[3][x];
+    // the sums are formed here: put off, they keep every direction's terms
+    // in registers, and 94 of those spill at p = 7
+#pragma unroll
+    for (int j = 0; j < 9; ++j) asm volatile("" : "+v"(t[j]));
+  };
+#pragma unroll
+  for (int r = 0; r < NPT; ++r) {
+    const int n = tid + r * NT;
+    if (n < Q3) {
+      const int pn = S::nidx(n);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) A[c * FS + pn] = pv[r][c];
+    }
+  }
+  __syncthreads();
   auto grad_dir = [&](auto Dc) {
     constexpr int d = decltype(Dc)::value;
-#pragma unroll
-    for (int r = 0; r < NPT; ++r) {
-      const int n = tid + r * NT;
-      if (n < Q3) {
-        const int pn = S::nidx(n);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) A[c * FS + pn] = pv[r][c];
-      }
-    }
-    __syncthreads();
-    if constexpr (d == 2) con_mid<4 * Q, Q, 1, Q, Q, QP, QP, NT>(EO<P>::NP1(), A, B, tid);   // along b
-    else con_last<4 * Q * Q, Q, Q, QP, QP, NT>(EO<P>::NP1(), A, B, tid);                    // along c
-    __syncthreads();
-    if constexpr (d == 0) con_mid<4 * Q, Q, 1, Q, Q, QP, QP, NT>(EO<P>::NP1(), B, A, tid);  // along b
-    else con_mid<4, Q, Q, Q, Q, QP, QP, NT>(EO<P>::NP1(), B, A, tid);                       // along a
-    __syncthreads();
-    const double g0 = mt[3 * d], g1 = mt[3 * d + 1], g2 = mt[3 * d + 2];
+    const double *m = uniform_const(mt) + 3 * d, g0 = m[0], g1 = m[1], g2 = m[2];
     const double inv = 1.0 / sqrt(g0 * g0 + g1 * g1 + g2 * g2);
-    lifted_dir<P, d, NT>(A, B, Hn, -inv, inv, tid);                                        // along d
+    lifted_dir<P, d, NT>(A, B, d == 0 ? cA : (d == 1 ? cB : cC), Hn, -inv, inv, again(tid));
     __syncthreads();
-    // nodal d/dxi_d of (u, v, w, e) -> stress and heat flux
-    const double c43 = mu * (4.0 / 3.0), c23 = mu * (2.0 / 3.0);
+    if constexpr (d == 2) return;   // c's part is added with the moments'
 #pragma unroll
     for (int r = 0; r < NPT; ++r) {
-      const int n = tid + r * NT;
+      const int n = again(tid) + r * NT;
       const int pn = S::nidx(n < Q3 ? n : 0);
-      const double au = B[pn], av = B[FS + pn], aw = B[2 * FS + pn], ae = B[3 * FS + pn];
-      const double ux = g0 * au, uy = g1 * au, uz = g2 * au;
-      const double vx = g0 * av, vy = g1 * av, vz = g2 * av;
-      const double wx = g0 * aw, wy = g1 * aw, wz = g2 * aw;
-      tq[r][0] += c43 * ux - c23 * (vy + wz);
-      tq[r][1] += mu * (uy + vx);
-      tq[r][2] += mu * (uz + wx);
-      tq[r][3] += c43 * vy - c23 * (ux + wz);
-      tq[r][4] += mu * (vz + wy);
-      tq[r][5] += c43 * wz - c23 * (ux + vy);
-      tq[r][6] += kap * (g0 * ae);
-      tq[r][7] += kap * (g1 * ae);
-      tq[r][8] += kap * (g2 * ae);
+      double g[4][3];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const double a = B[c * FS + pn];
+        g[c][0] = g0 * a; g[c][1] = g1 * a; g[c][2] = g2 * a;
+      }
+      add_stress(tq[r], g);
     }
+    __syncthreads();
   };
   grad_dir(IC<0>());
   grad_dir(IC<1>());
   grad_dir(IC<2>());
+  // N_b c_c, N_a c_c [i][j] and N_a c_b [i][k], to A
+  for (int t = tid; t < 12 * Q; t += NT) {
+    const int tb = t / (4 * Q), fx = t - tb * 4 * Q, f = fx / Q, x1 = fx - f * Q;
+    const int base = f * Q * QP + (tb == 0 ? x1 * QP : x1), st = tb == 0 ? 1 : QP;
+    const double *src = tb == 2 ? cB : cC, *v = uniform_const(CT<P>::NV()), *w = v + Q;
+    double x[Q], s = 0.0;
+#pragma unroll
+    for (int m = 0; m < Q; ++m) { x[m] = src[base + m * st]; s = fma(w[m], x[m], s); }
+#pragma unroll
+    for (int m = 0; m < Q; ++m) A[tb * TB + base + m * st] = fma(-v[m], s, x[m]);
+  }
+  double vn[NPT][3];   // -v at the thread's nodes
+#pragma unroll
+  for (int r = 0; r < NPT; ++r) {
+    const int n = again(tid) + r * NT, nn = n < Q3 ? n : 0;
+    const double *v = CT<P>::NV();
+    vn[r][0] = -v[nn / (Q * Q)]; vn[r][1] = -v[(nn / Q) % Q]; vn[r][2] = -v[nn % Q];
+  }
+  __syncthreads();
+  // the derivatives, in place but for c_a's two: D_a N_b c_c, D_b N_a c_c [i][j],
+  // D_c N_a c_b [i][k], D_b c_a, D_c c_a [j][k] in A, D_a c_b [i][k] in B
+  for (int t = tid; t < 24 * Q; t += NT) {
+    const int tb = t / (4 * Q), fx = t - tb * 4 * Q, f = fx / Q, x1 = fx - f * Q;
+    const bool row = tb == 1 || tb == 2 || tb == 4;   // along the table's last index
+    const int base = f * Q * QP + (row ? x1 * QP : x1), st = row ? 1 : QP;
+    const double *src = tb < 3 ? A + tb * TB : (tb == 5 ? cB : cA);
+    double *dst = tb == 5 ? cB : A + tb * TB;
+    double x[Q], y[Q];
+#pragma unroll
+    for (int m = 0; m < Q; ++m) x[m] = src[base + m * st];
+    eo_apply<EO_NNA, Q, Q>(uniform_const(EO<P>::DN().h), x, y);
+#pragma unroll
+    for (int m = 0; m < Q; ++m) dst[base + m * st] = y[m];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < NPT; ++r) {
+    const int n = again(tid) + r * NT, nn = n < Q3 ? n : 0, pn = S::nidx(nn);
+    const int i = nn / (Q * Q), j = (nn / Q) % Q, k = nn % Q;
+    const double *m = uniform_const(mt);
+    double g[4][3];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const double *ij = A + (c * Q + i) * QP + j, *ik = A + 2 * TB + (c * Q + i) * QP + k,
+                   *jk = A + 3 * TB + (c * Q + j) * QP + k;
+      const double a = fma(vn[r][2], ij[0], vn[r][1] * cB[(c * Q + i) * QP + k]);
+      const double b = fma(vn[r][2], ij[TB], vn[r][0] * jk[0]);
+      const double d = B[c * FS + pn] + fma(vn[r][1], ik[0], vn[r][0] * jk[TB]);
+#pragma unroll
+      for (int x = 0; x < 3; ++x) g[c][x] = fma(m[x], a, fma(m[3 + x], b, m[6 + x] * d));
+    }
+    add_stress(tq[r], g);
+  }
+  __syncthreads();
 
   double acc[NSG][L];   // modal viscous volume term of the 4 equations
   // BR2 scratch: Hn [24][Q][Q] and gs[9], KE[2][Q] in the Jq region; the
@@ -656,7 +739,7 @@ k_vterm3(const double *__restrict__ U, const double *__restrict__ T, double *__r
   // viscous volume divergence of the 4 equations
   auto visc_dir = [&](auto Dc) {
     constexpr int d = decltype(Dc)::value;
-    const double m0 = mt[3 * d], m1 = mt[3 * d + 1], m2 = mt[3 * d + 2];
+    const double *m = uniform_const(mt) + 3 * d, m0 = m[0], m1 = m[1], m2 = m[2];
 #pragma unroll
     for (int r = 0; r < NPT; ++r) {
       const int n = tid + r * NT;
