@@ -186,14 +186,29 @@ __global__ void __launch_bounds__(kHbThreads) k_hb_backward(HbArgs a) {
 // from one pass over its inputs, which cuts the LDS reads of the contractions
 // about NM-fold against one output per thread, and a wavefront needs no
 // workgroup barrier (its LDS operations complete in order).  The basis is read
-// with uniform addresses (scalar loads).  Per wavefront LDS: X and H of
-// max(Q^3, NM Q^2) doubles each.  Same sums, in the same order, as the
-// generic kernels.
+// with uniform addresses (scalar loads).  A pencil's outputs take the place of
+// its inputs in the element's one [Q][Q][Q] box of LDS.  Same sums, in the same
+// order, as the generic kernels.
+//
+// Bound by the latency of that chain (load, three contractions, store), hidden
+// by other wavefronts on the SIMD: the single box leaves room for twice as many
+// as an input and an output buffer did.  Both transforms and a copy of the slots
+// (24 M points in all): NM = 8 324 -> 253 us, NM = 10 353 -> 286, where the
+// copies' rate would take 205; NM = 3, four elements a wavefront, 303 -> 217.
 constexpr int kHbWaveThreads = 128;
 
 template <int NM, int Q> struct HbW {
   static constexpr int QT = Q * Q * Q, BC = Q * Q, N2 = NM * NM, N3 = N2 * NM;
-  static constexpr int XS = QT > NM * BC ? QT : NM * BC;   // doubles per buffer
+  // elements per wavefront: the smallest are packed, so that most lanes have a pencil
+  static constexpr int EPW = BC > 32 ? 1 : 64 / BC;
+  // wavefronts per SIMD: as the LDS allows, up to the eight that 64 registers
+  // leave room for, six of 80 from NM = 8 on
+  static constexpr int waves_lds = 160 * 1024 / (EPW * QT * 8) / 4, most = NM < 8 ? 8 : 6;
+  static constexpr int waves = waves_lds < 1 ? 1 : (waves_lds > most ? most : waves_lds);
+  // which of the wavefront's elements entry i is of, at n entries each
+  static __device__ __forceinline__ int el(int i, int n) { return EPW == 1 ? 0 : i / n; }
+  // place of modal index o = (i NM + j) NM + k in the box
+  static __device__ __forceinline__ int box(int o) { return o / N2 * BC + o % N2 / NM * Q + o % NM; }
 };
 
 // read-only global data through the scalar (constant) path: uniform loads of
@@ -206,165 +221,116 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// In-place contraction of NP pencils in each of EPW boxes of X: pencil r of a box
+// starts at place(r), its entries ST apart; NI inputs, NO outputs, M [NO][NI], sums in ascending order.
+// The basis is loaded (scalar cache) where it is used rather than held across
+// the elements, which would need far more SGPRs than there are.
+template <int NI, int NO, int NP, int ST, int EPW, int QT, class F>
+__device__ __forceinline__ void hb_pencils(double *X, const double *M, int lane, F place) {
+#pragma clang fp contract(off)
+  asm volatile("" : "+s"(M));
+  cdouble *m = (cdouble *)M;
+  for (int t = lane; t < EPW * NP; t += 64) {
+    const int b = EPW > 1 ? t / NP : 0;
+    double *p = X + b * QT + place(t - b * NP), x[NI];
+#pragma unroll
+    for (int k = 0; k < NI; ++k) x[k] = p[k * ST];
+#pragma unroll 4
+    for (int o = 0; o < NO; ++o) {
+      double s = 0.0;
+#pragma unroll
+      for (int k = 0; k < NI; ++k) s = s + m[o * NI + k] * x[k];
+      p[o * ST] = s;
+    }
+  }
+  wave_lds_sync();
+}
+
 template <int NM, int Q>
-__global__ void __launch_bounds__(kHbWaveThreads) k_hb_inner_w(HbArgs a) {
+__global__ void __launch_bounds__(kHbWaveThreads) __attribute__((amdgpu_waves_per_eu(HbW<NM, Q>::waves)))
+k_hb_inner_w(HbArgs a) {
 #pragma clang fp contract(off)
   using W = HbW<NM, Q>;
-  constexpr int QT = W::QT, BC = W::BC;
+  constexpr int QT = W::QT, BC = W::BC, EPW = W::EPW, ET = EPW * QT;
   extern __shared__ double sm[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = kHbWaveThreads / 64;
-  double *X = sm + wv * 2 * W::XS, *H = X + W::XS;
+  double *X = sm + wv * EPW * QT;
   // the next element's slot is loaded into registers while this one is
   // contracted, so a wavefront waits for HBM only on its first element
-  constexpr int NPL = (QT + 63) / 64;
-  const long long step = (long long)gridDim.x * nw;
+  constexpr int NPL = (ET + 63) / 64;
+  const long long step = (long long)gridDim.x * nw * EPW, first = ((long long)blockIdx.x * nw + wv) * EPW;
   double pre[NPL];
   auto fetch = [&](long long e) {
     const double *ue = a.u + e * QT;
 #pragma unroll
     for (int r = 0; r < NPL; ++r) {
       const int i = lane + 64 * r;
-      pre[r] = (e < a.ne && i < QT) ? ue[i] : 0.0;
+      pre[r] = i < ET && e + W::el(i, QT) < a.ne ? ue[i] : 0.0;
     }
   };
-  fetch((long long)blockIdx.x * nw + wv);
-  for (long long e = (long long)blockIdx.x * nw + wv; e < a.ne; e += step) {
-    // the basis is reloaded (scalar cache) for every element rather than held
-    // across the loop, which would need far more SGPRs than there are
-    const double *bp = a.B;
-    asm volatile("" : "+s"(bp));
-    cdouble *Ba = (cdouble *)bp, *Bb = Ba + NM * Q, *Bc = Bb + NM * Q;
+  fetch(first);
+  for (long long e = first; e < a.ne; e += step) {
     double *ue = a.u + e * QT;
-    const double *w = a.wJ + e * a.wj_stride;
+    const double *w = a.wJ + e * a.wj_stride, *Ba = a.B, *Bb = Ba + NM * Q, *Bc = Bb + NM * Q;
 #pragma unroll
     for (int r = 0; r < NPL; ++r) {
       const int i = lane + 64 * r;
-      if (i < QT) X[i] = pre[r] * w[i];
+      const int b = W::el(i, QT);
+      if (i < ET && e + b < a.ne) X[i] = pre[r] * w[b * a.wj_stride + i - b * QT];
     }
     fetch(e + step);
     wave_lds_sync();
-    for (int r = lane; r < BC; r += 64) {          // pencils along a: H[i][r]
-      double x[Q];
-#pragma unroll
-      for (int k = 0; k < Q; ++k) x[k] = X[k * BC + r];
-#pragma unroll 2
-      for (int i = 0; i < NM; ++i) {
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < Q; ++k) s = s + Ba[i * Q + k] * x[k];
-        H[i * BC + r] = s;
-      }
+    hb_pencils<Q, NM, BC, BC, EPW, QT>(X, Ba, lane, [](int r) { return r; });                        // along a
+    hb_pencils<Q, NM, NM * Q, Q, EPW, QT>(X, Bb, lane, [](int r) { return r / Q * BC + r % Q; });    // along b
+    hb_pencils<Q, NM, W::N2, 1, EPW, QT>(X, Bc, lane, [](int r) { return r / NM * BC + r % NM * Q; });   // along c
+    for (int t = lane; t < EPW * W::N3; t += 64) {
+      const int b = W::el(t, W::N3), o = t - b * W::N3;
+      if (e + b < a.ne) ue[b * QT + o] = X[b * QT + W::box(o)];
     }
-    wave_lds_sync();
-    for (int p = lane; p < NM * Q; p += 64) {      // pencils along b: Ha[i][j][c] into X
-      const int i = p / Q, c = p - i * Q;
-      double h[Q];
-#pragma unroll
-      for (int k = 0; k < Q; ++k) h[k] = H[i * BC + k * Q + c];
-#pragma unroll 2
-      for (int j = 0; j < NM; ++j) {
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < Q; ++k) s = s + Bb[j * Q + k] * h[k];
-        X[(i * NM + j) * Q + c] = s;
-      }
-    }
-    wave_lds_sync();
-    for (int ij = lane; ij < W::N2; ij += 64) {    // pencils along c: fh[i][j][k] staged in H
-      double h[Q];
-#pragma unroll
-      for (int c = 0; c < Q; ++c) h[c] = X[ij * Q + c];
-#pragma unroll 2
-      for (int k = 0; k < NM; ++k) {
-        double s = 0.0;
-#pragma unroll
-        for (int c = 0; c < Q; ++c) s = s + h[c] * Bc[k * Q + c];
-        H[ij * NM + k] = s;
-      }
-    }
-    wave_lds_sync();
-    for (int i = lane; i < W::N3; i += 64) ue[i] = H[i];
     wave_lds_sync();
   }
 }
 
 template <int NM, int Q>
-__global__ void __launch_bounds__(kHbWaveThreads) k_hb_backward_w(HbArgs a) {
+__global__ void __launch_bounds__(kHbWaveThreads) __attribute__((amdgpu_waves_per_eu(HbW<NM, Q>::waves)))
+k_hb_backward_w(HbArgs a) {
 #pragma clang fp contract(off)
   using W = HbW<NM, Q>;
-  constexpr int QT = W::QT, N2 = W::N2, N3 = W::N3;
+  constexpr int QT = W::QT, BC = W::BC, N3 = W::N3, EPW = W::EPW, ET = EPW * N3;
   extern __shared__ double sm[];
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6, nw = kHbWaveThreads / 64;
-  double *X = sm + wv * 2 * W::XS, *H = X + W::XS;
-  constexpr int NPL = (N3 + 63) / 64;
-  const long long step = (long long)gridDim.x * nw;
+  double *X = sm + wv * EPW * QT;
+  constexpr int NPL = (ET + 63) / 64;
+  const long long step = (long long)gridDim.x * nw * EPW, first = ((long long)blockIdx.x * nw + wv) * EPW;
   double pre[NPL];
   auto fetch = [&](long long e) {
     const double *ue = a.u + e * QT;
 #pragma unroll
     for (int r = 0; r < NPL; ++r) {
       const int i = lane + 64 * r;
-      pre[r] = (e < a.ne && i < N3) ? ue[i] : 0.0;
+      const int b = W::el(i, N3);
+      pre[r] = i < ET && e + b < a.ne ? ue[i + b * (QT - N3)] : 0.0;
     }
   };
-  fetch((long long)blockIdx.x * nw + wv);
-  for (long long e = (long long)blockIdx.x * nw + wv; e < a.ne; e += step) {
-    // the basis is reloaded (scalar cache) for every element rather than held
-    // across the loop, which would need far more SGPRs than there are
-    const double *bp = a.B;
-    asm volatile("" : "+s"(bp));
+  fetch(first);
+  for (long long e = first; e < a.ne; e += step) {
     // transposed copies (rows of Q x NM), so that each output reads a
     // contiguous run of the basis
-    cdouble *BaT = (cdouble *)bp + 3 * NM * Q, *BbT = BaT + NM * Q, *BcT = BbT + NM * Q;
+    const double *BaT = a.B + 3 * NM * Q, *BbT = BaT + NM * Q, *BcT = BbT + NM * Q;
     double *ue = a.u + e * QT;
 #pragma unroll
     for (int r = 0; r < NPL; ++r) {
       const int i = lane + 64 * r;
-      if (i < N3) X[i] = pre[r];
+      const int b = W::el(i, N3);
+      if (i < ET) X[b * QT + W::box(i - b * N3)] = pre[r];
     }
     fetch(e + step);
     wave_lds_sync();
-    for (int r = lane; r < N2; r += 64) {          // pencils along i: H[a][j][k]
-      double x[NM];
-#pragma unroll
-      for (int i = 0; i < NM; ++i) x[i] = X[i * N2 + r];
-#pragma unroll 2
-      for (int p = 0; p < Q; ++p) {
-        double s = 0.0;
-#pragma unroll
-        for (int i = 0; i < NM; ++i) s = s + BaT[p * NM + i] * x[i];
-        H[p * N2 + r] = s;
-      }
-    }
-    wave_lds_sync();
-    for (int pk = lane; pk < Q * NM; pk += 64) {   // pencils along j: Ha[a][b][k] into X
-      const int p = pk / NM, k = pk - p * NM;
-      double h[NM];
-#pragma unroll
-      for (int j = 0; j < NM; ++j) h[j] = H[p * N2 + j * NM + k];
-#pragma unroll 2
-      for (int b = 0; b < Q; ++b) {
-        double s = 0.0;
-#pragma unroll
-        for (int j = 0; j < NM; ++j) s = s + BbT[b * NM + j] * h[j];
-        X[(p * Q + b) * NM + k] = s;
-      }
-    }
-    wave_lds_sync();
-    for (int ab = lane; ab < Q * Q; ab += 64) {    // pencils along k: f[a][b][c] staged in H
-      double h[NM];
-#pragma unroll
-      for (int k = 0; k < NM; ++k) h[k] = X[ab * NM + k];
-#pragma unroll 2
-      for (int c = 0; c < Q; ++c) {
-        double s = 0.0;
-#pragma unroll
-        for (int k = 0; k < NM; ++k) s = s + h[k] * BcT[c * NM + k];
-        H[ab * Q + c] = s;
-      }
-    }
-    wave_lds_sync();
-    for (int i = lane; i < QT; i += 64) ue[i] = H[i];
+    hb_pencils<NM, Q, W::N2, BC, EPW, QT>(X, BaT, lane, [](int r) { return r / NM * Q + r % NM; });   // along i
+    hb_pencils<NM, Q, Q * NM, Q, EPW, QT>(X, BbT, lane, [](int r) { return r / NM * BC + r % NM; });  // along j
+    hb_pencils<NM, Q, BC, 1, EPW, QT>(X, BcT, lane, [](int r) { return r * Q; });                      // along k
+    for (int i = lane; i < EPW * QT; i += 64)
+      if (e + W::el(i, QT) < a.ne) ue[i] = X[i];
     wave_lds_sync();
   }
 }
@@ -426,8 +392,8 @@ int run(dgx_hexblock *h, double *u, int on_device, bool inner) {
 #define DGX_HB(NM)                                                                                   \
   case NM:                                                                                           \
     kern = inner ? dgx::k_hb_inner_w<NM, NM + 1> : dgx::k_hb_backward_w<NM, NM + 1>;                   \
-    per_wg = dgx::kHbWaveThreads / 64;                                                               \
-    lds = sizeof(double) * 2 * dgx::HbW<NM, NM + 1>::XS * per_wg;                                    \
+    per_wg = dgx::kHbWaveThreads / 64 * dgx::HbW<NM, NM + 1>::EPW;                                    \
+    lds = sizeof(double) * dgx::HbW<NM, NM + 1>::QT * per_wg;                                        \
     break;
         DGX_HB(2) DGX_HB(3) DGX_HB(4) DGX_HB(5) DGX_HB(6) DGX_HB(7) DGX_HB(8) DGX_HB(9) DGX_HB(10) DGX_HB(11)
 #undef DGX_HB
