@@ -46,7 +46,8 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 constexpr int mq_size(int no, int n) { return ((no + 3) / 4) * 4 * ((n + 3) / 4 * 4); }
 constexpr int mq_order_size(int p) {
   return mq_size(p + 2, p + 1) + 2 * mq_size(p + 1, p + 2) + mq_size(p + 1, p + 1) + mq_size(2, p + 1) +
-         mq_size(p + 1, p + 1) + mq_size(p + 1, p + 2) + mq_size(p + 1, p + 2);
+         mq_size(p + 1, p + 1) + mq_size(p + 1, p + 2) + mq_size(p + 1, p + 2) + mq_size(p + 2, p + 2) +
+         mq_size(2, p + 2);
 }
 constexpr int mq_order_offset(int p) {
   int s = 0;
@@ -67,6 +68,9 @@ template <int P> struct MT {
   static constexpr int oPW = oBend + mq_size(2, L);         // [L][QF]  Gauss inner product
   static constexpr int oIg = oPW + mq_size(L, QF);          // [QF][Q]  GLL -> Gauss
   static constexpr int oPI = oIg + mq_size(QF, Q);          // [L][Q]   GLL face layer -> modal face
+  static constexpr int oDN = oPI + mq_size(L, Q);           // [Q][Q]   GLL collocation derivative
+  static constexpr int oNV = oDN + mq_size(Q, Q);           // [2][Q]   order P + 1 mode, and weighted (CT::NV)
+  static constexpr int QPAD = (Q + 3) / 4 * 4;              // row pitch of DN and NV
 };
 
 // sqrt(1/2)^3: the constant normalized Legendre mode of a hex
@@ -74,6 +78,13 @@ constexpr double kPhi0 = 0.35355339059327376220;
 
 __device__ __forceinline__ f4 mfma4(float a, float b, f4 c) {
   return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, c, 0, 0, 0);
+}
+
+// uniform_const of a pointer that the compiler keeps per lane.
+template <typename T> __device__ __forceinline__ const T *first_const(const T *p) {
+  const uint64_t b = reinterpret_cast<uint64_t>(p);
+  const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+  return uniform_const(reinterpret_cast<const T *>((uint64_t)hi << 32 | lo));
 }
 
 // Per-lane coefficients of M[NO][N] at c_mq + off: cf[ob][k] = M[4*ob + lane%4][k].
@@ -183,22 +194,17 @@ template <int P, int NTH = kStageThreads> struct M3 {
   // its linearization H[3][3][5] (direction, reference dimension, field),
   // B_1 at the GLL points b1[Q]
   static constexpr int EC_CN = 0, EC_LIN = 5, EC_CF = 20, EC_H = 35, EC_B1 = 80, EC_N = 80 + Q;
-  static constexpr int lds_stage = (2 * NA + NG) * 4 + EC_N * 8 + 64;
-  static constexpr int lds_vterm = (2 * NA + 24 * QF * FP) * 4 + 64;
+  // FP64 face traces of the updated state, over the same LDS (face_traces3's two buffers)
+  static constexpr int TA = cmax(5 * L2 * LP, 10 * QF * cmax(LP, 3 * L) + 15 * QF2), TB = 20 * L * LP + 15 * L2;
+  static constexpr int lds_stage = cmax((2 * NA + NG) * 4 + EC_N * 8, (TA + TB) * 8) + 64;
+  // gradient kernel: its tensors also hold moment tables [4][Q][Q]
+  static constexpr int NAV = cmax(NA, cmax(24 * Q * QP, 4 * Q2 * QP + 8 * Q * QP));
+  static constexpr int lds_vterm = (2 * NAV + 24 * Q * QP) * 4 + 64;
   // BR2: face-lift nodal values, metric rows, end traces (+ layer velocity)
-  static constexpr bool br2_vel_in_b = 42 * Q * QP <= NA;
-  static constexpr int lds_vterm_br2 = (2 * NA + 24 * Q * QP + 16 + 2 * Q + (br2_vel_in_b ? 0 : 18 * Q * QP)) * 4 + 64;
+  static constexpr bool br2_vel_in_b = 42 * Q * QP <= NAV;
+  static constexpr int lds_vterm_br2 = (2 * NAV + 24 * Q * QP + 16 + 2 * Q + (br2_vel_in_b ? 0 : 18 * Q * QP)) * 4 + 64;
   static constexpr int FS = Q * Q * QP;
   static __device__ __forceinline__ int nidx(int n) { return (n / Q) * QP + (n - (n / Q) * Q); }
-  // FP64 face traces of the updated state, in batches of TB fields over the
-  // LDS of the stage kernel (as doubles): per field the modal block (later
-  // reused for the Gauss-point passes W, O) and the three Bend collapses.
-  static constexpr int KP = 3;
-  static constexpr int TW = QF * cmax(2 * LP, KP * L), TO = cmax(2 * QF * FP, KP * QF2);
-  static constexpr int TM = cmax(L * L * LP, TW + TO);
-  static constexpr int TK = 2 * L * LP + 2 * L * LP + L2 * KP;
-  static constexpr int TB0 = ((2 * NA + NG) / 2) / (TM + TK);
-  static constexpr int TB = TB0 < 5 ? TB0 : 5;
 };
 
 // Final contraction of a chain over the first spatial dimension of
@@ -228,20 +234,76 @@ __device__ __forceinline__ void mchain_to_regs(int off, const float *in, f4 (&ac
   }
 }
 
-// Projected divergence chain for reference direction D of NF nodal fields in
-// A ([NF][Q][Q][Q], pitch QP); result accumulated into registers.
-template <int P, int NF, int NS, int D, int NTH = kStageThreads>
-__device__ __forceinline__ void mdiv_chain(float *A, float *B, f4 (&acc)[NS][M3<P>::NOB], int tid) {
+// Collocation derivative along reference direction D of NF nodal fields in A
+// ([NF][Q][Q][Q], pitch QP), written (c, which comes first) or added to B.
+template <int P, int NF, int D, int NTH = kStageThreads>
+__device__ __forceinline__ void mnodal_deriv(const float *A, float *B, int tid) {
   using S = M3<P, NTH>;
-  using T = MT<P>;
-  constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT;
-  constexpr int oc = D == 2 ? T::oQD : T::oBW, ob = D == 1 ? T::oQD : T::oBW, oa = D == 0 ? T::oQD : T::oBW;
-  mcon_last<NF * Q * Q, Q, L, QP, LP, NT>(oc, A, B, tid);        // [NF Q Q][L]
+  constexpr int Q = S::Q, QP = S::QP, NT = S::NT, o = MT<P>::oDN;
+  if constexpr (D == 2) mcon_last<NF * Q * Q, Q, Q, QP, QP, NT>(o, A, B, tid);
+  else if constexpr (D == 1) mcon_mid<NF * Q, Q, 1, Q, Q, QP, QP, NT, true>(o, A, B, tid);
+  else mcon_mid<NF, Q, Q, Q, Q, QP, QP, NT, true>(o, A, B, tid);
+}
+
+// Projection of NF nodal fields in B, accumulated into registers (the pencils
+// of mchain_to_regs); A is scratch.  Projecting the nodal divergence once
+// equals the three projected-derivative chains, with six contractions for nine.
+template <int P, int NF, int NS, int NTH = kStageThreads>
+__device__ __forceinline__ void mproj_to_regs(float *A, float *B, f4 (&acc)[NS][M3<P>::NOB], int tid) {
+  using S = M3<P, NTH>;
+  constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT, o = MT<P>::oBW;
+  mcon_last<NF * Q * Q, Q, L, QP, LP, NT>(o, B, A, tid);         // [NF Q Q][L]
   __syncthreads();
-  mcon_mid<NF * Q, Q, 1, L, L, LP, LP, NT>(ob, B, A, tid);       // [NF Q][L][L]
+  mcon_mid<NF * Q, Q, 1, L, L, LP, LP, NT>(o, A, B, tid);        // [NF Q][L][L]
   __syncthreads();
-  mchain_to_regs<P, NF, NS, NTH>(oa, A, acc, tid);               // [NF][L][L][L]
+  mchain_to_regs<P, NF, NS, NTH>(o, B, acc, tid);                // [NF][L][L][L]
   __syncthreads();
+}
+
+// Derivative along D of the 4 primitives' nodal values plus the face lifts
+// across D (lifted_dir of the FP64 kernels): out = DN x + clo KE_lo Hn[lo] +
+// chi KE_hi Hn[hi], and the pencil's moment w . x to mom[4][Q][Q].
+template <int P, int D, int NT>
+__device__ __forceinline__ void mlifted_dir(const float *in, float *out, float *mom, const float *Hn, float clo,
+                                            float chi, int tid) {
+  constexpr int Q = P + 2, QP = odd(Q), HB = Q * QP, NP = 4 * Q * Q, KP = (NP + NT - 1) / NT, NOB = (Q + 3) / 4;
+  constexpr int flo = D == 0 ? 4 : (D == 1 ? 1 : 0), fhi = D == 0 ? 2 : (D == 1 ? 3 : 5);
+  const double *KE = first_const(CT<P>::KE());
+  const float *w = first_const(c_mq + MT<P>::oNV) + MT<P>::QPAD;
+  float cf[NOB][Q];
+  load_coef<Q, Q>(MT<P>::oDN, tid, cf);
+#pragma unroll
+  for (int k = 0; k < KP; ++k) {
+    if (!wave_has(tid, k, NT, NP)) continue;
+    const int pc0 = tid + k * NT;
+    const bool ok = pc0 < NP;
+    const int pc = ok ? pc0 : 0, f = pc / (Q * Q), t = pc - f * Q * Q, t1 = t / Q, t2 = t - t1 * Q;
+    const int base = D == 0 ? (f * Q * Q + t1) * QP + t2
+                            : (D == 1 ? (f * Q * Q + t1 * Q) * QP + t2 : (f * Q * Q + t1 * Q + t2) * QP);
+    constexpr int st = D == 0 ? Q * QP : (D == 1 ? QP : 1);
+    float x[Q];
+#pragma unroll
+    for (int i = 0; i < Q; ++i) x[i] = in[base + i * st];
+    const float hl = clo * Hn[(f * 6 + flo) * HB + t1 * QP + t2];
+    const float hh = chi * Hn[(f * 6 + fhi) * HB + t1 * QP + t2];
+    float m = w[0] * x[0];
+#pragma unroll
+    for (int i = 1; i < Q; ++i) m = fmaf(w[i], x[i], m);
+    if (ok) mom[(f * Q + t1) * QP + t2] = m;
+#pragma unroll
+    for (int ob = 0; ob < NOB; ++ob) {
+      f4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int i = 0; i < Q; ++i) acc = mfma4(cf[ob][i], x[i], acc);
+      if (ok) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+          const int o = 4 * ob + q;
+          if (o < Q) out[base + o * st] = fmaf((float)KE[Q - 1 - o], hh, fmaf((float)KE[o], hl, acc[q]));
+        }
+      }
+    }
+  }
 }
 
 // modal [NF][L][L][L] (pitch LP) in A -> nodal [NF][Q][Q][Q] (pitch QP) in B
@@ -359,11 +421,18 @@ __device__ __forceinline__ void euler_flux_jvp(const double c[5], double n0, dou
 
 }  // namespace
 
-#ifndef DGX_VTERM_M_THREADS
-#define DGX_VTERM_M_THREADS 512
-#endif
-// Threads per element of the mixed viscous kernel.
-constexpr int kVterm3mThreads = DGX_VTERM_M_THREADS;
+// Threads per element, and the three wavefronts per SIMD that the registers are
+// allocated for: fewer threads keep more elements on a CU, whose phases fill
+// each other's waits, until a thread's several nodes no longer fit its
+// registers.  BR2 steps of 4 M modes per field against 256 threads for the
+// stage and 512 for the viscous kernel at every order, with three projected
+// chains per divergence: p = 2 80.3 -> 20.4 ms, p = 3 50.5 -> 16.7 (128 threads
+// 19.4), p = 4 27.6 -> 16.2 (64: 21.5, 256: 19.2), p = 5 21.1 -> 13.1 (128:
+// 14.3, 256: 14.9), p = 6 17.3 -> 12.5 (192: 14.9, 512: 15.6), p = 7 14.8 ->
+// 12.1 (192: 13.6, 512: 15.0), p = 8 21.1 -> 13.5 (256: 16.6, 448: 19.2).
+// Four, five and six wavefronts per SIMD at p = 7: 15.0, 18.8 and 19.3 (512 threads).
+constexpr int mixed_threads(int p) { return p <= 3 ? 64 : (p == 4 ? 128 : (p == 5 ? 192 : (p <= 7 ? 256 : 512))); }
+constexpr int kMixedWaves = 3;
 
 struct MixedArgs {
   const double *T;       // face traces of the input state (FP64)
@@ -380,9 +449,10 @@ struct MixedArgs {
 
 // Residual (or fused LSRK14 stage) of Euler3d / Navier_Stokes3d, mixed precision.
 template <int P, bool NS, bool UPDATE>
-__global__ void __launch_bounds__(kStageThreads)
+__global__ void __launch_bounds__(mixed_threads(P))
+__attribute__((amdgpu_waves_per_eu(lds_waves(M3<P, mixed_threads(P)>::lds_stage, mixed_threads(P), kMixedWaves))))
 k_stage3m(MixedArgs a, Geo geo, Phys ph) {
-  using S = M3<P>;
+  using S = M3<P, mixed_threads(P)>;
   constexpr int L = S::L, Q = S::Q, QF = S::QF, L2 = S::L2, L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2,
                 LP = S::LP, FP = S::FP, NT = S::NT, NPT = S::NPT, NSL = S::NSL, NOB = S::NOB, FS = S::FS;
   extern __shared__ __attribute__((aligned(16))) float smf[];
@@ -409,7 +479,10 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
       const int d = (tid - 16) / 3, x = (tid - 16) % 3;
       double dU[5], dF[5];
 #pragma unroll
-      for (int v = 0; v < 5; ++v) dU[v] = lin[v][x];
+      for (int v = 0; v < 5; ++v) {
+        const double l0 = lin[v][0], l1 = lin[v][1], l2 = lin[v][2];
+        dU[v] = x == 0 ? l0 : (x == 1 ? l1 : l2);
+      }
       const double *mg = geo.metric + 9 * (size_t)e + 3 * d;   // d varies by thread: not the register copy
       euler_flux_jvp(cn, mg[0], mg[1], mg[2], gm1, dU, dF);
 #pragma unroll
@@ -428,8 +501,8 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
       ec[S::EC_CF + 5 * d + 2] = cn[2] * vn + m1 * pc;
       ec[S::EC_CF + 5 * d + 3] = cn[3] * vn + m2 * pc;
       ec[S::EC_CF + 5 * d + 4] = (cn[4] + pc) * vn;
-    } else if (tid >= 64 && tid < 64 + Q) {
-      ec[S::EC_B1 + tid - 64] = CT<P>::BT()[(tid - 64) * L + 1];
+    } else if (tid >= 48 && tid < 48 + Q) {
+      ec[S::EC_B1 + tid - 48] = CT<P>::BT()[(tid - 48) * L + 1];
     }
   }
   // face corrections g = (J_side/J_vol) (Fhat - F(U-).n) [- BR1 viscous part], FP64
@@ -470,7 +543,7 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
   store_split<P, NT, true>(um, A, tid);
 
   __syncthreads();
-  mbackward<P, 5>(A, B, tid);
+  mbackward<P, 5, NT>(A, B, tid);
   // nodal state: constant and linear modes in FP64, the rest from the FP32 transform
   double un[NPT][5];
 #pragma unroll
@@ -527,11 +600,13 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
       }
     }
     __syncthreads();
-    mdiv_chain<P, 5, NSL, d>(A, B, acc, tid);
+    mnodal_deriv<P, 5, d, NT>(A, B, tid);
+    __syncthreads();
   };
-  vol_dir(IC<0>());
-  vol_dir(IC<1>());
   vol_dir(IC<2>());
+  vol_dir(IC<1>());
+  vol_dir(IC<0>());
+  mproj_to_regs<P, 5, NSL, NT>(A, B, acc, tid);
 
   // the update's HBM inputs (viscous volume term, RK register) are loaded
   // before the face projection, whose barriers then cover their latency
@@ -549,7 +624,7 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
   }
 
   // faces: H = (PW (x) PW) gF for 5 fields x 6 faces, in B
-  mface_project<P, 30>(gF, A, B, tid);
+  mface_project<P, 30, NT>(gF, A, B, tid);
   const float one6[6] = {1.f, 1.f, 1.f, 1.f, 1.f, 1.f};
   double unew[NSL][L];
 #pragma unroll
@@ -579,80 +654,20 @@ k_stage3m(MixedArgs a, Geo geo, Phys ph) {
   }
   if (!UPDATE) return;
 
-  // FP64 face traces of the updated state for the next stage, TB fields at a time
-  auto batch = [&](auto V0) {
-    constexpr int v0 = decltype(V0)::value;
-    constexpr int F = (5 - v0) < S::TB ? (5 - v0) : S::TB;
-    double *Md = reinterpret_cast<double *>(smf);
-    double *K0 = Md + F * S::TM, *K1 = K0 + F * 2 * L * LP, *K2 = K1 + F * 2 * L * LP;
-    __syncthreads();
+  // FP64 face traces of the updated state for the next stage
+  double *Md = reinterpret_cast<double *>(smf);
+  __syncthreads();
 #pragma unroll
-    for (int k = 0; k < NSL; ++k) {
-      const int G = tid + k * NT;
-      if (G < 5 * L2) {
-        const int v = G / L2, pp = G - v * L2, m = pp / L, nn = pp - m * L;
-        if (v >= v0 && v < v0 + F) {
+  for (int k = 0; k < NSL; ++k) {
+    const int G = tid + k * NT;
+    if (G < 5 * L2) {
+      const int v = G / L2, pp = G - v * L2, m = pp / L, nn = pp - m * L;
 #pragma unroll
-          for (int l = 0; l < L; ++l) Md[(((v - v0) * L + l) * L + m) * LP + nn] = unew[k][l];
-        }
-      }
+      for (int l = 0; l < L; ++l) Md[((v * L + l) * L + m) * LP + nn] = unew[k][l];
     }
-    __syncthreads();
-    constexpr int KP = S::KP;
-    con_mid<F, L, L, L, 2, LP, LP, NT>(EO<P>::Bend(), Md, K0, tid);       // [F][2][L][L]
-    con_mid<F * L, L, 1, L, 2, LP, LP, NT>(EO<P>::Bend(), Md, K1, tid);   // [F][L][2][L]
-    con_last<F * L2, L, 2, LP, KP, NT>(EO<P>::Bend(), Md, K2, tid);       // [F][L][L][2]
-    __syncthreads();
-    double *W = Md, *O = Md + F * S::TW;
-    double *Te = a.Tn + (size_t)e * 6 * 5 * QF2;
-    // faces 4 / 2: [F][2][QF][QF]
-    con_mid<2 * F, L, 1, L, QF, LP, LP, NT>(EO<P>::Bg(), K0, W, tid);     // [2F][QF][L]
-    __syncthreads();
-    con_last<2 * F * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);      // [2F][QF][QF]
-    __syncthreads();
-    for (int i = tid; i < 2 * F * QF2; i += NT) {
-      const int ve = i / QF2, q = i - ve * QF2, v = ve >> 1, end = ve & 1;
-      Te[((end ? 2 : 4) * 5 + v0 + v) * QF2 + q] = O[(ve * QF + q / QF) * FP + q % QF];
-    }
-    __syncthreads();
-    // faces 1 / 3: [F][QF][2][QF]
-    con_mid<F, L, 2, L, QF, LP, LP, NT>(EO<P>::Bg(), K1, W, tid);         // [F][QF][2][L]
-    __syncthreads();
-    con_last<2 * F * QF, L, QF, LP, FP, NT>(EO<P>::Bg(), W, O, tid);      // [F][QF][2][QF]
-    __syncthreads();
-    for (int i = tid; i < 2 * F * QF2; i += NT) {
-      const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
-      const int ia = q / QF, ic = q - ia * QF;
-      Te[((end ? 3 : 1) * 5 + v0 + v) * QF2 + q] = O[((v * QF + ia) * 2 + end) * FP + ic];
-    }
-    __syncthreads();
-    // faces 0 / 5: [F][QF][QF][2]
-    con_mid<F, L, L, 2, QF, KP, KP, NT>(EO<P>::Bg(), K2, W, tid);         // [F][QF][L][2]
-    __syncthreads();
-    con_mid<F * QF, L, 1, 2, QF, KP, KP, NT>(EO<P>::Bg(), W, O, tid);     // [F][QF][QF][2]
-    __syncthreads();
-    for (int i = tid; i < 2 * F * QF2; i += NT) {
-      const int v = i / (2 * QF2), r = i - v * 2 * QF2, end = r / QF2, q = r - end * QF2;
-      Te[((end ? 5 : 0) * 5 + v0 + v) * QF2 + q] = O[(v * QF2 + q) * KP + end];
-    }
-  };
-  batch(IC<0>());
-  if constexpr (S::TB < 5) batch(IC<S::TB>());
-  if constexpr (2 * S::TB < 5) batch(IC<2 * S::TB>());
-  if constexpr (3 * S::TB < 5) batch(IC<3 * S::TB>());
-  if constexpr (4 * S::TB < 5) batch(IC<4 * S::TB>());
-}
-
-// Face-lift contribution of the two faces normal to reference direction D at
-// modal (l, m, n) of block set H ([6][L][L], pitch LP), with weights clo, chi
-// for the face at -1 and +1 (faces 4/2 for a, 1/3 for b, 0/5 for c), FP32.
-template <int P, int D>
-__device__ __forceinline__ float mface_pair(const float *H, int l, int m, int n, float clo, float chi) {
-  constexpr int L = P + 1, LP = odd(L), HB = L * LP;
-  const double *B0 = CT<P>::Bend(), *B1 = CT<P>::Bend() + L;
-  if (D == 0) return fmaf(clo * (float)B0[l], H[4 * HB + m * LP + n], chi * (float)B1[l] * H[2 * HB + m * LP + n]);
-  if (D == 1) return fmaf(clo * (float)B0[m], H[1 * HB + l * LP + n], chi * (float)B1[m] * H[3 * HB + l * LP + n]);
-  return fmaf(clo * (float)B0[n], H[0 * HB + l * LP + m], chi * (float)B1[n] * H[5 * HB + l * LP + m]);
+  }
+  __syncthreads();
+  face_traces3<P, NT>(Md, Md + S::TA, a.Tn + (size_t)e * 6 * 5 * QF2, tid);
 }
 
 // Viscous flux of equation q contracted with (n0, n1, n2) from the stress
@@ -673,19 +688,19 @@ __device__ __forceinline__ float mvisc_flux(const float t[6], const float h[3], 
 // points of face s.  The lifted gradient is assembled one reference direction
 // at a time (affine faces: normals -+ grad xi_d / |grad xi_d|) straight into
 // the stress tensor and heat flux at the thread's nodes.
-// At p = 7 the BR2 variant needs a few registers more than the 128 that keep
-// two 512-thread workgroups per CU: capped there (4 registers spill).
 template <int P, bool BR2>
-__global__ void __launch_bounds__(kVterm3mThreads) __attribute__((amdgpu_waves_per_eu((BR2 && P == 7) ? 4 : 1)))
+__global__ void __launch_bounds__(mixed_threads(P))
+__attribute__((amdgpu_waves_per_eu(lds_waves(BR2 ? M3<P, mixed_threads(P)>::lds_vterm_br2 : M3<P, mixed_threads(P)>::lds_vterm,
+                                             mixed_threads(P), kMixedWaves))))
 k_vterm3m(const double *__restrict__ U, const double *__restrict__ Tr, float *__restrict__ V,
           float *__restrict__ TV, Geo geo, Phys ph, int ne) {
-  using S = M3<P, kVterm3mThreads>;
+  using S = M3<P, mixed_threads(P)>;
   using T = MT<P>;
   constexpr int L = S::L, Q = S::Q, QF = S::QF, L2 = S::L2, L3 = S::L3, Q3 = S::Q3, QF2 = S::QF2,
                 LP = S::LP, QP = S::QP, FP = S::FP, NT = S::NT, NPT = S::NPT, NSG = S::NSG, NOB = S::NOB,
                 FS = S::FS;
   extern __shared__ __attribute__((aligned(16))) float smf[];
-  float *A = smf, *B = A + S::NA, *Jq = B + S::NA;
+  float *A = smf, *B = A + S::NAV, *Jq = B + S::NAV;
   const int e = xcd_element(blockIdx.x, ne), tid = threadIdx.x;
 
   double cn[5];
@@ -744,12 +759,17 @@ k_vterm3m(const double *__restrict__ U, const double *__restrict__ Tr, float *__
     uw[r][0] = (float)u; uw[r][1] = (float)v; uw[r][2] = (float)w;
   }
   __syncthreads();
-  // face lift of the jumps: (PW (x) PW) Jq -> H[4][6][L][L], kept in the Jq region
+  // face lift of the jumps: (PW (x) PW) Jq -> H[4][6][L][L], then its values at
+  // each face's own GLL points Hn[4][6][Q][Q], kept in the Jq region
   mcon_mid<24, QF, 1, QF, L, FP, FP, NT>(T::oPW, Jq, A, tid);     // [24][L][QF]
   __syncthreads();
   mcon_last<24 * L, QF, L, FP, LP, NT>(T::oPW, A, Jq, tid);     // [24][L][L]
   __syncthreads();
-  const float *H = Jq;
+  mcon_mid<24, L, 1, L, Q, LP, LP, NT>(T::oBT, Jq, A, tid);     // [24][Q][L]
+  __syncthreads();
+  mcon_last<24 * Q, L, Q, LP, QP, NT>(T::oBT, A, Jq, tid);      // [24][Q][Q]
+  __syncthreads();
+  const float *Hn = Jq;
 
   const double *mt = geo.metric + 9 * (size_t)e;
   const float mu = (float)ph.vis, kap = (float)(ph.vis * ph.gamma / ph.Pr);
@@ -758,64 +778,119 @@ k_vterm3m(const double *__restrict__ U, const double *__restrict__ Tr, float *__
   for (int r = 0; r < NPT; ++r)
 #pragma unroll
     for (int j = 0; j < 9; ++j) tq[r][j] = 0.f;
+  // The lifted gradient from nodal derivatives and face-sized moments, as in the
+  // FP64 kernel: D_a N_b N_c q = D_a q - v_k D_a N_b c_c - v_j D_a c_b, ...
+  constexpr int TB = 4 * Q * QP;   // one [4][Q][Q] table
+  static_assert(4 * FS + 2 * TB <= S::NAV && 6 * TB <= S::NAV, "moment tables");
+  float *cA = A + S::NAV - TB, *cB = B + S::NAV - TB, *cC = B + 4 * FS;
+  const float c43 = mu * (4.f / 3.f), c23 = mu * (2.f / 3.f);
+  // physical gradients g[c][x] of (u, v, w, e) -> stress and heat flux
+  auto add_stress = [&](float (&t)[9], const float (&g)[4][3]) {
+    t[0] += c43 * g[0][0] - c23 * (g[1][1] + g[2][2]);
+    t[1] += mu * (g[0][1] + g[1][0]);
+    t[2] += mu * (g[0][2] + g[2][0]);
+    t[3] += c43 * g[1][1] - c23 * (g[0][0] + g[2][2]);
+    t[4] += mu * (g[1][2] + g[2][1]);
+    t[5] += c43 * g[2][2] - c23 * (g[0][0] + g[1][1]);
+#pragma unroll
+    for (int x = 0; x < 3; ++x) t[6 + x] += kap * g[3][x];
+    // formed here: put off, the sums keep every direction's terms in registers
+#pragma unroll
+    for (int j = 0; j < 9; ++j) asm volatile("" : "+v"(t[j]));
+  };
+#pragma unroll
+  for (int r = 0; r < NPT; ++r) {
+    const int n = tid + r * NT;
+    if (n < Q3) {
+      const int pn = S::nidx(n);
+#pragma unroll
+      for (int c = 0; c < 4; ++c) A[c * FS + pn] = pv[r][c];
+    }
+  }
+  __syncthreads();
   auto grad_dir = [&](auto Dc) {
     constexpr int d = decltype(Dc)::value;
-#pragma unroll
-    for (int r = 0; r < NPT; ++r) {
-      const int n = tid + r * NT;
-      if (n < Q3) {
-        const int pn = S::nidx(n);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) A[c * FS + pn] = pv[r][c];
-      }
-    }
-    __syncthreads();
-    f4 D[NSG][NOB];
-#pragma unroll
-    for (int k = 0; k < NSG; ++k)
-#pragma unroll
-      for (int ob = 0; ob < NOB; ++ob) D[k][ob] = f4{0.f, 0.f, 0.f, 0.f};
-    mdiv_chain<P, 4, NSG, d, NT>(A, B, D, tid);
-    const double g0d = mt[3 * d], g1d = mt[3 * d + 1], g2d = mt[3 * d + 2];
+    const double *m = first_const(mt) + 3 * d, g0d = m[0], g1d = m[1], g2d = m[2];
     const float inv = (float)(1.0 / sqrt(g0d * g0d + g1d * g1d + g2d * g2d));
-#pragma unroll
-    for (int k = 0; k < NSG; ++k) {
-      const int Gi = tid + k * NT;
-      if (Gi < 4 * L2) {
-        const int c = Gi / L2, pp = Gi - c * L2, m = pp / L, nn = pp - m * L;
-#pragma unroll
-        for (int l = 0; l < L; ++l)
-          A[((c * L + l) * L + m) * LP + nn] =
-              D[k][l / 4][l % 4] + mface_pair<P, d>(H + c * 6 * L * LP, l, m, nn, -inv, inv);
-      }
-    }
+    mlifted_dir<P, d, NT>(A, B, d == 0 ? cA : (d == 1 ? cB : cC), Hn, -inv, inv, again(tid));
     __syncthreads();
-    mbackward<P, 4, NT>(A, B, tid);
+    if constexpr (d == 2) return;   // c's part is added with the moments'
     const float g0 = (float)g0d, g1 = (float)g1d, g2 = (float)g2d;
-    const float c43 = mu * (4.f / 3.f), c23 = mu * (2.f / 3.f);
 #pragma unroll
     for (int r = 0; r < NPT; ++r) {
-      const int n = tid + r * NT;
+      const int n = again(tid) + r * NT;
       const int pn = S::nidx(n < Q3 ? n : 0);
-      const float au = B[pn], av = B[FS + pn], aw = B[2 * FS + pn], ae = B[3 * FS + pn];
-      const float ux = g0 * au, uy = g1 * au, uz = g2 * au;
-      const float vx = g0 * av, vy = g1 * av, vz = g2 * av;
-      const float wx = g0 * aw, wy = g1 * aw, wz = g2 * aw;
-      tq[r][0] += c43 * ux - c23 * (vy + wz);
-      tq[r][1] += mu * (uy + vx);
-      tq[r][2] += mu * (uz + wx);
-      tq[r][3] += c43 * vy - c23 * (ux + wz);
-      tq[r][4] += mu * (vz + wy);
-      tq[r][5] += c43 * wz - c23 * (ux + vy);
-      tq[r][6] += kap * (g0 * ae);
-      tq[r][7] += kap * (g1 * ae);
-      tq[r][8] += kap * (g2 * ae);
+      float g[4][3];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        const float a = B[c * FS + pn];
+        g[c][0] = g0 * a; g[c][1] = g1 * a; g[c][2] = g2 * a;
+      }
+      add_stress(tq[r], g);
     }
     __syncthreads();
   };
   grad_dir(IC<0>());
   grad_dir(IC<1>());
   grad_dir(IC<2>());
+  // N_b c_c, N_a c_c [i][j] and N_a c_b [i][k], to A
+  for (int t = tid; t < 12 * Q; t += NT) {
+    const int tb = t / (4 * Q), fx = t - tb * 4 * Q, f = fx / Q, x1 = fx - f * Q;
+    const int base = f * Q * QP + (tb == 0 ? x1 * QP : x1), st = tb == 0 ? 1 : QP;
+    const float *src = tb == 2 ? cB : cC, *v = first_const(c_mq + T::oNV), *w = v + T::QPAD;
+    float x[Q], s = 0.f;
+#pragma unroll
+    for (int m = 0; m < Q; ++m) { x[m] = src[base + m * st]; s = fmaf(w[m], x[m], s); }
+#pragma unroll
+    for (int m = 0; m < Q; ++m) A[tb * TB + base + m * st] = fmaf(-v[m], s, x[m]);
+  }
+  float vn[NPT][3];   // -v at the thread's nodes
+#pragma unroll
+  for (int r = 0; r < NPT; ++r) {
+    const int n = again(tid) + r * NT, nn = n < Q3 ? n : 0;
+    const float *v = c_mq + T::oNV;
+    vn[r][0] = -v[nn / (Q * Q)]; vn[r][1] = -v[(nn / Q) % Q]; vn[r][2] = -v[nn % Q];
+  }
+  __syncthreads();
+  // the derivatives, in place but for c_a's two: D_a N_b c_c, D_b N_a c_c [i][j],
+  // D_c N_a c_b [i][k], D_b c_a, D_c c_a [j][k] in A, D_a c_b [i][k] in B
+  for (int t = tid; t < 24 * Q; t += NT) {
+    const int tb = t / (4 * Q), fx = t - tb * 4 * Q, f = fx / Q, x1 = fx - f * Q;
+    const bool row = tb == 1 || tb == 2 || tb == 4;   // along the table's last index
+    const int base = f * Q * QP + (row ? x1 * QP : x1), st = row ? 1 : QP;
+    const float *src = tb < 3 ? A + tb * TB : (tb == 5 ? cB : cA), *D = first_const(c_mq + T::oDN);
+    float *dst = tb == 5 ? cB : A + tb * TB;
+    float x[Q];
+#pragma unroll
+    for (int m = 0; m < Q; ++m) x[m] = src[base + m * st];
+#pragma unroll
+    for (int o = 0; o < Q; ++o) {
+      float y = 0.f;
+#pragma unroll
+      for (int m = 0; m < Q; ++m) y = fmaf(D[o * T::QPAD + m], x[m], y);
+      dst[base + o * st] = y;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < NPT; ++r) {
+    const int n = again(tid) + r * NT, nn = n < Q3 ? n : 0, pn = S::nidx(nn);
+    const int i = nn / (Q * Q), j = (nn / Q) % Q, k = nn % Q;
+    const double *md = first_const(mt);
+    float g[4][3];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+      const float *ij = A + (c * Q + i) * QP + j, *ik = A + 2 * TB + (c * Q + i) * QP + k,
+                  *jk = A + 3 * TB + (c * Q + j) * QP + k;
+      const float a = fmaf(vn[r][2], ij[0], vn[r][1] * cB[(c * Q + i) * QP + k]);
+      const float b = fmaf(vn[r][2], ij[TB], vn[r][0] * jk[0]);
+      const float d = B[c * FS + pn] + fmaf(vn[r][1], ik[0], vn[r][0] * jk[TB]);
+#pragma unroll
+      for (int x = 0; x < 3; ++x) g[c][x] = fmaf((float)md[x], a, fmaf((float)md[3 + x], b, (float)md[6 + x] * d));
+    }
+    add_stress(tq[r], g);
+  }
+  __syncthreads();
 
   f4 acc[NSG][NOB];   // modal viscous volume term of the 4 equations
   // BR2 scratch: Hn [24][Q][Q] and gs[9], KE[2][Q] in the Jq region; the
@@ -824,16 +899,14 @@ k_vterm3m(const double *__restrict__ U, const double *__restrict__ Tr, float *__
   constexpr int HN = 24 * Q * QP, VOFF = S::br2_vel_in_b ? 0 : HN + 16 + 2 * Q;
   float *Df = B, *Vel = S::br2_vel_in_b ? B + HN : Jq + VOFF;
   if constexpr (BR2) {
-    // nodal values of the face lifts at each face's own GLL points: Hn[24][Q][Q]
-    mcon_mid<24, L, 1, L, Q, LP, LP, NT>(T::oBT, Jq, A, tid);   // [24][Q][L]
-    if (tid < 9) {   // unit rows of the metric
+    // the face lifts' nodal values Hn[24][Q][Q] are in place; after them the
+    // unit rows of the metric and the end-trace table
+    if (tid < 9) {
       const int d = tid / 3;
       Jq[HN + tid] = (float)(mt[tid] / sqrt(mt[3 * d] * mt[3 * d] + mt[3 * d + 1] * mt[3 * d + 1] +
                                             mt[3 * d + 2] * mt[3 * d + 2]));
     }
     if (tid >= 16 && tid < 16 + 2 * Q) Jq[HN + tid] = (float)CT<P>::KE()[tid - 16];
-    __syncthreads();
-    mcon_last<24 * Q, L, Q, LP, QP, NT>(T::oBT, A, Jq, tid);    // [24][Q][Q]
     __syncthreads();
   }
 
@@ -942,11 +1015,13 @@ k_vterm3m(const double *__restrict__ U, const double *__restrict__ Tr, float *__
       }
     }
     __syncthreads();
-    mdiv_chain<P, 4, NSG, d, NT>(A, B, acc, tid);
+    mnodal_deriv<P, 4, d, NT>(A, B, tid);
+    __syncthreads();
   };
-  visc_dir(IC<0>());
-  visc_dir(IC<1>());
   visc_dir(IC<2>());
+  visc_dir(IC<1>());
+  visc_dir(IC<0>());
+  mproj_to_regs<P, 4, NSG, NT>(A, B, acc, tid);
 #pragma unroll
   for (int k = 0; k < NSG; ++k) {
     const int Gi = tid + k * NT;
@@ -976,17 +1051,17 @@ void pack_mq(const double *M, int no, int n, float *out) {
 
 template <int P>
 hipError_t launch_mixed3_p(const StageLaunch &s) {
-  using S = M3<P>;
+  using S = M3<P, mixed_threads(P)>;
   if (s.op == 0) {
     if (s.phys.visc == 1) {
-      const int sh = M3<P, kVterm3mThreads>::lds_vterm_br2;
+      const int sh = M3<P, mixed_threads(P)>::lds_vterm_br2;
       (void)hipFuncSetAttribute((const void *)k_vterm3m<P, true>, hipFuncAttributeMaxDynamicSharedMemorySize, sh);
-      hipLaunchKernelGGL((k_vterm3m<P, true>), dim3(s.ne), dim3(kVterm3mThreads), sh, s.stream, s.U, s.T, s.Vfw,
+      hipLaunchKernelGGL((k_vterm3m<P, true>), dim3(s.ne), dim3(mixed_threads(P)), sh, s.stream, s.U, s.T, s.Vfw,
                          s.TVfw, s.geo, s.phys, s.ne);
     } else {
-      const int sh = M3<P, kVterm3mThreads>::lds_vterm;
+      const int sh = M3<P, mixed_threads(P)>::lds_vterm;
       (void)hipFuncSetAttribute((const void *)k_vterm3m<P, false>, hipFuncAttributeMaxDynamicSharedMemorySize, sh);
-      hipLaunchKernelGGL((k_vterm3m<P, false>), dim3(s.ne), dim3(kVterm3mThreads), sh, s.stream, s.U, s.T, s.Vfw,
+      hipLaunchKernelGGL((k_vterm3m<P, false>), dim3(s.ne), dim3(mixed_threads(P)), sh, s.stream, s.U, s.T, s.Vfw,
                          s.TVfw, s.geo, s.phys, s.ne);
     }
     return hipGetLastError();
@@ -999,7 +1074,7 @@ hipError_t launch_mixed3_p(const StageLaunch &s) {
   do {                                                                                               \
     (void)hipFuncSetAttribute((const void *)k_stage3m<P, NSV, UPD>,                                  \
                               hipFuncAttributeMaxDynamicSharedMemorySize, sh);                       \
-    hipLaunchKernelGGL((k_stage3m<P, NSV, UPD>), dim3(s.ne), dim3(kStageThreads), sh, s.stream, a, s.geo,      \
+    hipLaunchKernelGGL((k_stage3m<P, NSV, UPD>), dim3(s.ne), dim3(mixed_threads(P)), sh, s.stream, a, s.geo,  \
                        s.phys);                                                                      \
   } while (0)
   if (s.ns) { if (s.update) DGX_MSTAGE(true, true); else DGX_MSTAGE(true, false); }
@@ -1046,7 +1121,10 @@ hipError_t upload_tables_m3d(const double *h) {
     pack_mq(Bend, 2, L, o); o += mq_size(2, L);
     pack_mq(PW, L, QF, o); o += mq_size(L, QF);
     pack_mq(Ig, QF, Q, o); o += mq_size(QF, Q);
-    pack_mq(Ig + QF * Q, L, Q, o); o += mq_size(L, Q);   // PI follows Ig in the FP64 tables
+    const double *PI = Ig + QF * Q, *DN = PI + L * Q + 2 * Q + L * Q + Q * QF;
+    pack_mq(PI, L, Q, o); o += mq_size(L, Q);
+    pack_mq(DN, Q, Q, o); o += mq_size(Q, Q);
+    pack_mq(DN + Q * Q, 2, Q, o); o += mq_size(2, Q);    // NV
     if (o != mq.data() + mq_order_offset(p + 1)) return hipErrorInvalidValue;
   }
   return hipMemcpyToSymbol(HIP_SYMBOL(c_mq), mq.data(), sizeof(float) * kMqTotal);

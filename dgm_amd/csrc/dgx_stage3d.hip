@@ -160,21 +160,23 @@ struct StageArgs {
 
 // Threads per element: up to p = 5 one per pencil of 5 fields, so that every
 // contraction phase is a single pass whose lanes are nearly all busy (p = 4:
-// also one per node); from p = 6 on, where the LDS holds two workgroups per
+// also one per node; p = 2: one wavefront for the 80 pencils, whose barriers
+// cost nothing, took a BR2 step of 4 M modes from 25.5 to 23.6 ms and an Euler
+// step from 8.1 to 7.3, where p = 3 lost 20 %); from p = 6 on, where the LDS holds two workgroups per
 // CU, 512, for four wavefronts per SIMD (320 at p = 6 were 10 % slower).  512
 // for all orders left 76 % of the lanes idle at p = 3: an Euler LSRK14 step of
 // 1.2 M modes per field 8.31 -> 2.76 ms at p = 2, 4.27 -> 1.83 at p = 3,
 // 2.67 -> 1.70 at p = 4, 2.18 -> 1.62 at p = 5; with BR2 viscous terms 26.9 ->
 // 7.4, 13.8 -> 5.1, 8.0 -> 4.7, 6.2 -> 4.7.
-constexpr int hex_threads(int p) { return p >= 6 ? 512 : (p == 4 ? 256 : round64(5 * (p + 2) * (p + 2))); }
+constexpr int hex_threads(int p) { return p >= 6 ? 512 : p == 2 ? 64 : (p == 4 ? 256 : round64(5 * (p + 2) * (p + 2))); }
 // Wavefronts per SIMD that the register allocation leaves room for, where the
 // LDS does: five at the lowest orders, whose kernels spill eight registers at most
 // for it.  Against four, Euler steps of 4 M modes per field went from 9.48 to 8.10
-// ms at p = 2, 5.86 to 5.52 at p = 3, 5.83 to 5.52 at p = 4, and with BR2 27.8
-// to 25.7 at p = 2; but the Navier-Stokes stage at p = 3 lost 3 % and k_vterm3
-// from p = 3 on gained nothing.
+// ms at p = 2, 5.86 to 5.52 at p = 3, 5.83 to 5.52 at p = 4, and with BR2 43.3
+// to 39.4 at p = 1; but the Navier-Stokes stage at p = 3 lost 3 % and k_vterm3
+// from p = 2 on gained nothing.
 constexpr int stage_waves(int p, bool ns) { return p > 4 || (ns && p == 3) ? 4 : 5; }
-constexpr int vterm_waves(int p) { return p > 2 ? 4 : 5; }
+constexpr int vterm_waves(int p) { return p > 1 ? 4 : 5; }
 
 template <int P, bool NS, bool UPDATE>
 __global__ void __launch_bounds__(hex_threads(P))
