@@ -76,7 +76,8 @@ FP32_MFMA_PEAK_TFLOPS = 157.3
 ARITHMETIC = {"fp64": "FP64 VALU (MI355X FP64 vector and matrix peaks are both 78.6 TFLOP/s)",
               "mixed": "FP32 MFMA contractions with FP64 pointwise work; peak is the FP32 matrix rate"}
 BYTES_PER_DOF_STAGE = 32.0
-# algorithmic flops per DOF-stage by kernel kind, per order (3D NS, BR1); BR2
+# algorithmic flops per DOF-stage by kernel kind, per order (3D NS, BR1), of the
+# plain sums; the kernels' even-odd contractions and moments execute fewer.  BR2
 # adds its face pass to the viscous kernel: nodal face lifts (2 x 29,376 FMA),
 # the per-face-node correction (486 nodes x ~154 flops), the lift of the flux
 # difference (29,376 FMA) and its face sum (12,288 FMA) per element of 2,560 DOF

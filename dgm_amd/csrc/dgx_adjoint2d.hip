@@ -1,6 +1,6 @@
 // Backward kernels of the 2D Euler residual (quads, Lax-Friedrichs, affine,
 // periodic): the vector-Jacobian product out = (dR/dU)^T lam of the residual
-// R = -dU/dt that k_traces2 + k_rhs2 compute (Euler::convection,
+// R = -dU/dt that k_traces2 + k_quad2 compute (Euler::convection,
 // convective_flux, lift and project, src/Euler.cpp:296-757,
 // src/Quad.cpp:1971-2038), and the pressure observation at receiver points
 // with its adjoint.  They drive the discrete adjoint of LSRK14 time stepping
