@@ -5,18 +5,15 @@
 #pragma once
 #include "dgx_device.hpp"
 
-#ifndef DGX_STAGE_THREADS
-#define DGX_STAGE_THREADS 256
-#endif
-
 namespace dgx {
 
-// Threads per workgroup (one element per workgroup) of the fused hex kernels.
-constexpr int kStageThreads = DGX_STAGE_THREADS;
+// Default thread count of the fused hex kernels' templates, for sizes that do not
+// depend on it; the kernels name their own (hex_threads, mixed_threads).
+constexpr int kStageThreads = 256;
 
 constexpr int round64(int n) { return (n + 63) / 64 * 64; }
 // Wavefronts per SIMD that the LDS of workgroups of nt threads allows, at
-// most 4: the register budget to ask the compiler for.
+// most `most`: the register budget to ask the compiler for.
 constexpr int lds_waves(int lds, int nt, int most = 4) {
   const int w = (160 * 1024 / lds) * (nt / 64) / 4;
   return w < 1 ? 1 : (w > most ? most : w);
