@@ -78,8 +78,8 @@ template <int P> struct CT {
 // and half the coefficients, which are scalar loads and mostly stay in scalar
 // registers (41 instead of 81 for a 9-point derivative).  The sums differ from
 // the plain ones by rounding only.  Against plain sums, a Navier-Stokes LSRK14
-// step on 32^3 hexes at p = 7 went from 52.6 to 48.8 ms, ten TVD-RK3 steps of
-// four quads at p = 10 from 1.01 to 0.71 ms.  Kinds:
+// step on 32^3 hexes at p = 7 went from 52.6 to 48.8 ms.  Affine Navier-Stokes
+// quads keep the plain sums (k_quad2).  Kinds:
 //   EO_MN   modes -> points          M[rev o][l] = (-1)^l M[o][l]
 //   EO_NM   points -> modes          M[l][rev i] = (-1)^l M[l][i]
 //   EO_NMA  points -> modes, odd     M[l][rev i] = -(-1)^l M[l][i]   (a derivative)

@@ -51,14 +51,14 @@ template <int P>
 __device__ __forceinline__ void backward2(const Tab &tb, const double *m, double *s1, double *out,
                                           int tid) {
   constexpr int L = H2<P>::L, Q = H2<P>::Q, NT = H2<P>::NT;
-  contract<1, L, L, 1, Q, NT>(EO<P>::BT(), m, s1, tid);
+  contract<1, L, L, 1, Q, NT>(CT<P>::BT(), m, s1, tid);
   __syncthreads();
-  contract<1, Q, L, 2, Q, NT>(EO<P>::BT(), s1, out, tid);
+  contract<1, Q, L, 2, Q, NT>(CT<P>::BT(), s1, out, tid);
   __syncthreads();
 }
 
 // Gauss-point traces of a state's NF fields on the elements' edges.
-template <int P, int NF, int EPW, typename R>
+template <int P, int NF, int EPW, class TT, typename R>
 __device__ __forceinline__ void load_traces2(const double *__restrict__ U, double *__restrict__ T, int ne, int e0,
                                              R *sm) {
   using S = Q2S<P, NF, EPW>;
@@ -71,25 +71,32 @@ __device__ __forceinline__ void load_traces2(const double *__restrict__ U, doubl
     if (i < S::NM) M[i] = (R)U[((size_t)v * ne + min(e0 + el, ne - 1)) * L2 + (r - v * L2)];
   }
   __syncthreads();
-  quad_traces<P, NF, EPW, R, TE<R, P>>(M, K, T, e0, ne, tid);
+  quad_traces<P, NF, EPW, R, TT>(M, K, T, e0, ne, tid);
 }
 
-template <int P, typename R = double>
+// TT: the tables (CT<P> for Navier-Stokes, see k_quad2).
+template <int P, class TT, typename R = double>
 __global__ void __launch_bounds__(64)
 k_traces2(const double *__restrict__ U, double *__restrict__ T, int ne, int nf) {
   if (nf == 3) {
     constexpr int E = quad_epw(P, 3);
     __shared__ R sm[Q2S<P, 3, E>::size];
-    load_traces2<P, 3, E, R>(U, T, ne, blockIdx.x * E, sm);
+    load_traces2<P, 3, E, TT, R>(U, T, ne, blockIdx.x * E, sm);
   } else {
     constexpr int E = quad_epw(P, 4);
     __shared__ R sm[Q2S<P, 4, E>::size];
-    load_traces2<P, 4, E, R>(U, T, ne, blockIdx.x * E, sm);
+    load_traces2<P, 4, E, TT, R>(U, T, ne, blockIdx.x * E, sm);
   }
 }
 
 // One stage of an affine domain (quad_stage): EQ 0 Euler, 1 Navier-Stokes with
-// the BR1 viscous terms V, TV, 2 shallow water.
+// the BR1 viscous terms V, TV, 2 shallow water.  Navier-Stokes takes the plain
+// tables, like its traces, k_grad2 and k_visc2: explicit steps may exceed the
+// viscous limit dt ~ h^2 / (nu (p + 1)^4) for a while, and there each step
+// multiplies a difference in the last bit by ten and more (p = 10, 134^2
+// quads, five RK4 steps: a million times), so that the even-odd sums' other
+// rounding shows in the eleventh digit.  It costs time: ten TVD-RK3 steps of
+// four quads at p = 10 take 0.94 ms, with even-odd sums 0.63 ms.
 template <int P, int EPW, typename R, int EQ>
 __global__ void __launch_bounds__(64)
 k_quad2(const double *X, const double *__restrict__ T, const double *__restrict__ V, const double *__restrict__ TV,
@@ -102,7 +109,8 @@ k_quad2(const double *X, const double *__restrict__ T, const double *__restrict_
     quad_stage<P, EPW, R, TE<R, P>, false>(X, T, V, TV, geo, ne, e0, flag, QuadShallow{ph}, QuadBalanced{up, Bal, bal},
                                            Tn, sm);
   else
-    quad_stage<P, EPW, R, TE<R, P>, EQ == 1>(X, T, V, TV, geo, ne, e0, flag, QuadEuler{ph}, up, Tn, sm);
+    quad_stage<P, EPW, R, std::conditional_t<EQ == 1, CT<P>, TE<R, P>>, EQ == 1>(X, T, V, TV, geo, ne, e0, flag,
+                                                                                QuadEuler{ph}, up, Tn, sm);
 }
 
 // lifted, projected gradients of (u, v, e): G[e][2*prim + dir][L2]
@@ -159,12 +167,12 @@ k_grad2(const double *__restrict__ U, const double *__restrict__ T, double *__re
       Fb[k] = val;
     }
     __syncthreads();
-    contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), Fb, Xa, tid);
-    contract<1, Q, Q, 2, L, NT>(EO<P>::QD(), Fb, Xc, tid);
+    contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), Fb, Xa, tid);
+    contract<1, Q, Q, 2, L, NT>(CT<P>::QD(), Fb, Xc, tid);
     contract<1, 4, QF, 2, L, NT>(CT<P>::PW(), Jq + q * 4 * QF, H, tid);
     __syncthreads();
-    contract<1, Q, L, 1, L, NT>(EO<P>::QD(), Xa, D2, tid);
-    contract<1, Q, L, 1, L, NT>(EO<P>::BW(), Xc, D2 + L2, tid);
+    contract<1, Q, L, 1, L, NT>(CT<P>::QD(), Xa, D2, tid);
+    contract<1, Q, L, 1, L, NT>(CT<P>::BW(), Xc, D2 + L2, tid);
     __syncthreads();
     for (int k = tid; k < L2; k += NT) {
       const int l = k / L, m = k - l * L;
@@ -226,7 +234,7 @@ k_visc2(const double *__restrict__ U, const double *__restrict__ G, double *__re
     for (int q = 0; q < 3; ++q) Lay[(s * 3 + q) * Q + j] = f[q][0] * nn[0] + f[q][1] * nn[1];
   }
   __syncthreads();
-  contract<1, 12, Q, 2, QF, NT>(EO<P>::Ig(), Lay, Wf, tid);
+  contract<1, 12, Q, 2, QF, NT>(CT<P>::Ig(), Lay, Wf, tid);
   __syncthreads();
   copy_block<NT>(Wf, TV + (size_t)e * 12 * QF, 12 * QF, tid);
   const double *mt = geo.metric + 9 * (size_t)e;
@@ -241,12 +249,12 @@ k_visc2(const double *__restrict__ U, const double *__restrict__ G, double *__re
   }
   __syncthreads();
   for (int q = 0; q < 3; ++q) {
-    contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), Gn + 2 * q * Q2, X1, tid);
-    contract<1, Q, Q, 2, L, NT>(EO<P>::QD(), Gn + (2 * q + 1) * Q2, X2, tid);
+    contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), Gn + 2 * q * Q2, X1, tid);
+    contract<1, Q, Q, 2, L, NT>(CT<P>::QD(), Gn + (2 * q + 1) * Q2, X2, tid);
     __syncthreads();
-    contract<1, Q, L, 1, L, NT>(EO<P>::QD(), X1, Vo, tid);
+    contract<1, Q, L, 1, L, NT>(CT<P>::QD(), X1, Vo, tid);
     __syncthreads();
-    contract<1, Q, L, 1, L, NT, true>(EO<P>::BW(), X2, Vo, tid);
+    contract<1, Q, L, 1, L, NT, true>(CT<P>::BW(), X2, Vo, tid);
     __syncthreads();
     copy_block<NT>(Vo, V + ((size_t)e * 3 + q) * L2, L2, tid);
     __syncthreads();
@@ -262,9 +270,9 @@ k_forward2(const double *__restrict__ Fn, double *__restrict__ Fm, Tab tb, int n
   const int e = blockIdx.x % ne, v = blockIdx.x / ne, tid = threadIdx.x;
   copy_block<NT>(Fn + ((size_t)v * ne + e) * Q2, A, Q2, tid);
   __syncthreads();
-  contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), A, X, tid);
+  contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), A, X, tid);
   __syncthreads();
-  contract<1, Q, L, 1, L, NT>(EO<P>::BW(), X, O, tid);
+  contract<1, Q, L, 1, L, NT>(CT<P>::BW(), X, O, tid);
   __syncthreads();
   copy_block<NT>(O, Fm + ((size_t)v * ne + e) * L2, L2, tid);
 }
@@ -371,7 +379,7 @@ k_batch_traces2(const Batch2 *__restrict__ b, int nreq, int nwork) {
   int r = 0;
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
     while (r + 1 < nreq && b[r + 1].off <= w) ++r;
-    load_traces2<P, NF, E, R>(b[r].U, b[r].T, b[r].ne, (w - b[r].off) * E, sm);
+    load_traces2<P, NF, E, TE<R, P>, R>(b[r].U, b[r].T, b[r].ne, (w - b[r].off) * E, sm);
     __syncthreads();
   }
 }
@@ -434,7 +442,7 @@ k_batch_persist2(const Batch2 *__restrict__ b, int nreq, int nwork, int nsteps, 
     int r = 0;
     for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
       while (r + 1 < nreq && b[r + 1].off <= w) ++r;
-      load_traces2<P, NF, E, R>(b[r].U, b[r].T, b[r].ne, (w - b[r].off) * E, sm);
+      load_traces2<P, NF, E, TE<R, P>, R>(b[r].U, b[r].T, b[r].ne, (w - b[r].off) * E, sm);
       __syncthreads();
     }
   }
@@ -580,9 +588,12 @@ static hipError_t launch2(const LaunchArgs &a) {
     case OP_TRACES: {
       const int E = quad_epw(P, a.nfield), grid = (ne + E - 1) / E;
       if (a.mixed)
-        hipLaunchKernelGGL((k_traces2<P, float>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
+        hipLaunchKernelGGL((k_traces2<P, TE<float, P>, float>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne,
+                           a.nfield);
+      else if (a.ns)
+        hipLaunchKernelGGL((k_traces2<P, CT<P>>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
       else
-        hipLaunchKernelGGL(k_traces2<P>, dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
+        hipLaunchKernelGGL((k_traces2<P, EO<P>>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
       break;
     }
     case OP_RHS: {

@@ -199,6 +199,26 @@ struct LinearAdjoint {
   }
 };
 
+// y = M x of one pencil, for the two forms of a table: even-odd, or the plain
+// rows M [NO][NI] with sums in ascending order.
+template <int K, int NI, int NO, typename T>
+__device__ __forceinline__ void table_apply(EoMat<K, T> M, const T (&x)[NI], T (&y)[NO]) {
+  eo_apply<K, NI, NO>(M.h, x, y);
+}
+template <int NI, int NO, typename T>
+__device__ __forceinline__ void table_apply(const T *__restrict__ M, const T (&x)[NI], T (&y)[NO]) {
+#pragma unroll
+  for (int o = 0; o < NO; ++o) {
+    T s = 0;
+#pragma unroll
+    for (int i = 0; i < NI; ++i) s = fma(M[o * NI + i], x[i], s);
+    y[o] = s;
+  }
+}
+// the full rows of a table whose even-odd form holds them (EO_MN), or of a plain one
+template <typename T> __device__ __forceinline__ const T *table_rows(EoMat<EO_MN, T> M) { return M.h; }
+template <typename T> __device__ __forceinline__ const T *table_rows(const T *M) { return M; }
+
 // The state's end values [EF][4][L] on the four edges from M, then its values
 // at their Gauss points, into T of elements e0 .. (those below ne).
 template <int P, int NF, int EPW, typename R, class TE>
@@ -217,7 +237,7 @@ __device__ __forceinline__ void quad_traces(const R *M, R *K, double *__restrict
     R x[L], y[QF];
 #pragma unroll
     for (int l = 0; l < L; ++l) x[l] = k[l * st];
-    eo_apply<EO_MN, L, QF>(TE::Bg().h, x, y);
+    table_apply(TE::Bg(), x, y);
     if (e0 + el < ne) {
 #pragma unroll
       for (int q = 0; q < QF; ++q) Te[pc * QF + q] = y[q];
@@ -351,8 +371,8 @@ __device__ __forceinline__ void quad_stage(const double *X, const double *__rest
     R a[Q], b[Q], y[L], z[L];
 #pragma unroll
     for (int i = 0; i < Q; ++i) { a[i] = X1[(f * Q + i) * L + c]; b[i] = X2[(f * Q + i) * L + c]; }
-    eo_apply<EO_NMA, Q, L>(TE::QD().h, a, y);
-    eo_apply<EO_NM, Q, L>(TE::BW().h, b, z);
+    table_apply(TE::QD(), a, y);
+    table_apply(TE::BW(), b, z);
 #pragma unroll
     for (int l = 0; l < L; ++l) M[(f * L + l) * L + c] = y[l] + z[l];
   }
@@ -362,7 +382,7 @@ __device__ __forceinline__ void quad_stage(const double *X, const double *__rest
   for (int k = 0; k < S::NU; ++k) {
     const int i = tid + k * NT, el = i / (NF * L2), rr = i - el * NF * L2, v = rr / L2, m = rr - v * L2, l = m / L;
     if (i >= S::NM) continue;
-    double r = M[i] + face_add2<P, R>(TE::Bend().h, H + (el * NF + v) * 4 * L, l, m - l * L, cw);
+    double r = M[i] + face_add2<P, R>(table_rows(TE::Bend()), H + (el * NF + v) * 4 * L, l, m - l * L, cw);
     if constexpr (NS) r -= vv[k];
     const int e = e0 + el;
     const size_t o = ((size_t)v * ne + e) * L2 + m;

@@ -185,9 +185,9 @@ __global__ void __launch_bounds__(64) k_vforward2(VarpArgs a) {
   const double *src = a.X + ((size_t)v * a.ne + e) * a.QM;
   for (int i = tid; i < Q2; i += NT) A[i] = src[i];
   __syncthreads();
-  contract<1, Q, Q, 2, L, NT>(EO<P>::BW(), A, X, tid);
+  contract<1, Q, Q, 2, L, NT>(CT<P>::BW(), A, X, tid);
   __syncthreads();
-  contract<1, Q, L, 1, L, NT>(EO<P>::BW(), X, O, tid);
+  contract<1, Q, L, 1, L, NT>(CT<P>::BW(), X, O, tid);
   __syncthreads();
   double *dst = a.Y + ((size_t)v * a.ne + e) * a.NM;
   for (int i = tid; i < a.NM; i += NT) dst[i] = i < L2 ? O[i] : 0.0;
@@ -201,9 +201,9 @@ __global__ void __launch_bounds__(64) k_vbackward2(VarpArgs a) {
   const double *src = a.X + ((size_t)v * a.ne + e) * a.NM;
   for (int i = tid; i < L2; i += NT) A[i] = src[i];
   __syncthreads();
-  contract<1, L, L, 1, Q, NT>(EO<P>::BT(), A, X, tid);
+  contract<1, L, L, 1, Q, NT>(CT<P>::BT(), A, X, tid);
   __syncthreads();
-  contract<1, Q, L, 2, Q, NT>(EO<P>::BT(), X, O, tid);
+  contract<1, Q, L, 2, Q, NT>(CT<P>::BT(), X, O, tid);
   __syncthreads();
   double *dst = a.Y + ((size_t)v * a.ne + e) * a.QM;
   for (int i = tid; i < a.QM; i += NT) dst[i] = i < Q2 ? O[i] : 0.0;
