@@ -1623,6 +1623,7 @@ int dgx_coordinates(dgx_handle h, double *xyz) {
 int dgx_state_device_ptr(dgx_handle h, double **U) {
   if (!h || !U) return fail(DGX_ERR_ARGUMENT, "null argument");
   *U = h->U;
+  h->u_shared = true;
   return DGX_OK;
 }
 
@@ -1680,8 +1681,9 @@ int nstages(int inttype) {
 // Stage `st` of one step of integrator `inttype`, as the reference's
 // TimeInt::advance runs it (RungeKutta src/TimeInt.cpp:267-302, TVD :824-856,
 // LSRK14 :1989-2013); the step starts at the domain time of stage 0.
-// `traces_ready`: the fused LSRK14 path may take the face traces the previous
-// stage wrote instead of evaluating them.
+// `traces_ready`: nobody else wrote the stage's state since the stage before, so
+// that affine elements (any integrator) and curved hexes (LSRK14) may take the
+// face traces that stage left instead of evaluating them.
 int run_stage(dgx_domain *h, int inttype, int st, double dt, bool traces_ready) {
   const size_t n = h->state_len();
   hipStream_t s = h->stream;
@@ -1807,7 +1809,10 @@ int dgx_stage(dgx_handle h, int inttype, int stage, double dt) {
   if (stage != h->next_stage || (stage > 0 && inttype != h->stage_int))
     return fail(DGX_ERR_ARGUMENT, "stages run in order 0 .. " + std::to_string(ns - 1) +
                                       " of one integrator; expected stage " + std::to_string(h->next_stage));
-  int rc = run_stage(h, inttype, stage, dt, stage > 0);
+  // LSRK14's stages run on the state itself, which the caller may write between
+  // them once it has the pointer; the other integrators' intermediate states
+  // are the domain's own
+  int rc = run_stage(h, inttype, stage, dt, stage > 0 && !(h->u_shared && inttype == DGX_LSRK14));
   if (rc) return rc;
   h->stage_int = inttype;
   h->next_stage = stage + 1 == ns ? 0 : stage + 1;

@@ -51,6 +51,7 @@ struct dgx_domain {
   double *G = nullptr, *V = nullptr, *TV = nullptr, *nodal = nullptr, *T2 = nullptr;
   float *Vf = nullptr, *TVf = nullptr;   // viscous terms of the mixed path
   const double *t_of = nullptr;          // the state whose face traces T holds, where a stage or launch put them
+  bool u_shared = false;                 // the caller has the pointer to U and may write it at any time
   bool fused = false;   // hex fused stage kernels available for this order
   bool curved = false;  // curved hexes (dgx_curved3d.hip): nodal metrics, mass-matrix projection
   double *d_gm = nullptr, *d_fgeo = nullptr, *d_jav = nullptr;

@@ -206,7 +206,9 @@ int dgx_coordinates(dgx_handle h, double *xyz);
 int dgx_state_upload(dgx_handle h, const double *U, int layout, int on_device);
 int dgx_state_download(dgx_handle h, double *U, int layout, int on_device);
 
-/* Device pointer of the modal state ([field][elem][mode], FP64). */
+/* Device pointer of the modal state ([field][elem][mode], FP64).  It may be
+ * written between calls, dgx_stage's included (ordered with the domain's
+ * stream): each call starts from the state it finds. */
 int dgx_state_device_ptr(dgx_handle h, double **U);
 
 /* Residual F = -dU/dt of the current state into the domain's residual
