@@ -308,10 +308,12 @@ template <int P, int NF, int NT> struct MassSolve {
 // Weighted divergence at the nodes, Out[v] += sum_d gm[d][X] D_d F_X of NV
 // fields for one Cartesian component X whose fluxes F holds ([NV][Q][Q][Q],
 // pitch QP): one pencil of each reference direction in turn, its outputs
-// scaled by the metric term at their nodes.  `first` writes Out.
+// scaled by the metric term at their nodes.  `first` writes Out.  The nine
+// terms of a node cancel to a large part, so they are summed in FP64 also where
+// the derivatives are FP32.
 // `beside(d)` is other work of the phase of direction d, on other buffers.
 template <int P, int NV, int NT, typename R, class F2>
-__device__ __forceinline__ void metric_deriv(EoMat<EO_NNA, R> D, const R *F, R *Out, const double *ge, int X, bool first,
+__device__ __forceinline__ void metric_deriv(EoMat<EO_NNA, R> D, const R *F, double *Out, const double *ge, int X, bool first,
                                              int tid, F2 beside) {
   using S = C3<P>;
   constexpr int Q = S::Q, Q2 = S::Q2, Q3 = S::Q3, QP = S::QP;
@@ -334,8 +336,8 @@ __device__ __forceinline__ void metric_deriv(EoMat<EO_NNA, R> D, const R *F, R *
 #pragma unroll
       for (int k = 0; k < Q; ++k) {
         const double val = m[k] * (double)y[k];
-        if (first && d == 0) Out[b + k * sl] = (R)val;
-        else Out[b + k * sl] = (R)((double)Out[b + k * sl] + val);
+        if (first && d == 0) Out[b + k * sl] = val;
+        else Out[b + k * sl] += val;
       }
     }
     beside(d);
@@ -352,8 +354,9 @@ __device__ __forceinline__ void metric_deriv(EoMat<EO_NNA, R> D, const R *F, R *
 // 1.76 ms (this kernel with conjugate gradients and one thread per node's
 // derivatives, and the traces' own kernel) to 0.65 ms.
 // R: arithmetic of the residual before the mass solve (its element tensors,
-// contractions and derivatives): double, or float on the mixed path, whose
-// LDS views alias the same memory as the FP64 buffers of the mass solve.
+// contractions and derivatives; the weighted divergence and the face terms are
+// summed in FP64): double, or float on the mixed path, whose LDS views alias
+// the same memory as the FP64 buffers of the mass solve.
 // NS: Navier-Stokes (BR1), adding the viscous terms k_grad3c and k_visc3c
 // wrote: the weighted nodal divergence V is subtracted before the projection,
 // and each interior side's correction gains J_side/J_vol (1/2)(F_v.n- + F_v+.n+)
@@ -474,7 +477,7 @@ k_rhs3c(CurvedArgs a, const double *__restrict__ gm, const double *__restrict__ 
         W1r[4 * FS + pn] = (R)((E + p) * u);
       }
       __syncthreads();
-      metric_deriv<P, 5, NT, R>(TR::DN(), W1r, W2r, ge, x, x == 0, tid, [](int) {});
+      metric_deriv<P, 5, NT, R>(TR::DN(), W1r, W2, ge, x, x == 0, tid, [](int) {});
     }
     double acc[NPT][5], wj[NPT];
 #pragma unroll
@@ -483,7 +486,7 @@ k_rhs3c(CurvedArgs a, const double *__restrict__ gm, const double *__restrict__ 
       wj[rr] = n < Q3 ? ge[9 * Q3 + n] : 0.0;
 #pragma unroll
       for (int v = 0; v < 5; ++v) {
-        acc[rr][v] = n < Q3 ? (double)W2r[v * FS + pn] : 0.0;
+        acc[rr][v] = n < Q3 ? W2[v * FS + pn] : 0.0;
         if (NS && v > 0 && n < Q3) acc[rr][v] -= a.V[((size_t)e * 4 + v - 1) * Q3 + n];
       }
     }

@@ -114,9 +114,16 @@ __device__ __forceinline__ void eo_apply(const T *__restrict__ h, const T (&x)[N
     }
   } else {
     T xe[HI], xo[FI > 0 ? FI : 1];
+    // a derivative takes no notice of a constant, but the FP32 sums would round
+    // relative to it: they act on the differences to the middle entry
+    constexpr bool diff = sizeof(T) == 4 && (K == EO_NMA || K == EO_NNA);
+    const T c = diff ? x[FI] : T(0);
 #pragma unroll
-    for (int i = 0; i < FI; ++i) { xe[i] = x[i] + x[NI - 1 - i]; xo[i] = x[i] - x[NI - 1 - i]; }
-    if constexpr (NI & 1) xe[FI] = x[FI];
+    for (int i = 0; i < FI; ++i) {
+      xe[i] = diff ? (x[i] - c) + (x[NI - 1 - i] - c) : x[i] + x[NI - 1 - i];
+      xo[i] = x[i] - x[NI - 1 - i];
+    }
+    if constexpr (NI & 1) xe[FI] = diff ? T(0) : x[FI];
     if constexpr (K == EO_NM || K == EO_NMA) {
 #pragma unroll
       for (int l = 0; l < NO; ++l) {

@@ -162,8 +162,8 @@ def test_mixed_curved_hexes_against_fp64(p):
     derivatives in FP32, the metric terms, Riemann fluxes, mass solve, state
     and registers FP64.  Stated errors against the FP64 path (measured
     maxima in brackets): one residual, relative L2 per field, <= 1e-5
-    [2.9e-6]; the state after 50 LSRK14 steps against the norm of the whole
-    state <= 5e-6 [1.2e-6], per field <= 1e-4 [2.5e-5] (the momenta that are
+    [2.3e-6]; the state after 50 LSRK14 steps against the norm of the whole
+    state <= 5e-6 [9.4e-7], per field <= 1e-4 [2.1e-5] (the momenta that are
     only the flow's deflection by the bump have small norms)."""
     from test_gpu_parity import _channel_state
     lo, hi = (0.0, 0.0, 0.0), (2.0, 2.0, 1.0)
@@ -190,3 +190,45 @@ def test_mixed_curved_hexes_against_fp64(p):
     assert np.all(e_w <= 5e-6) and np.all(e_f <= 1e-4), (e_f, e_w)
     g64.close()
     g32.close()
+
+
+# relative L2 error of the whole residual against the FP64 path on the folded
+# mesh below, per order, as plain FP32 derivatives summed in FP64 give it
+FOLDED = {1: 1.80e-7, 2: 4.97e-7, 3: 8.38e-7, 4: 1.29e-6, 5: 1.74e-6, 6: 2.29e-6, 7: 2.75e-6, 8: 3.48e-6}
+
+
+def _folded(p, precision):
+    """Thin hexes folded five times their width: the metric terms of a node
+    cancel to a large part."""
+    m = meshgen.periodic_hexes(3, 3, 3)
+    fold = lambda x, y, z: (x + 5 * np.sin(2 * np.pi * y), y, 0.01 * z + 0.05 * np.sin(2 * np.pi * x))   # noqa: E731
+    d = dgx.GPUDomain(m, p, dgx.DGX_EULER3D, xnodes=meshgen.mapped_nodes(m, p, fold), precision=precision)
+    return d, meshgen.hex_nodes(m, p)
+
+
+def _wave(x, amp):
+    s = [np.sin(2 * np.pi * (x[0] + 0.1 * k)) * np.cos(2 * np.pi * (x[1] - x[2] + 0.2 * k)) for k in range(5)]
+    return np.stack([1 + amp * s[0], 0.3 + amp * s[1], amp * s[2] - 0.1, amp * s[3], 2.5 + amp * s[4]])
+
+
+@pytest.mark.parametrize("p", range(1, 9))
+def test_mixed_curved_residual_of_every_order(p):
+    """DGX_MIXED on curved hexes is as exact as plain FP32 derivatives whose
+    nine weighted terms are summed in FP64 (FOLDED, and 5 %, the part of the
+    rounding that depends on the order of the sums; even-odd sums of the fluxes
+    themselves, which round relative to their constant part, exceed it by 9 % at
+    p = 1 and 6 % at p = 2); and a free stream, whose fluxes are the same FP32 value at every
+    node, has the FP64 path's rounding residual."""
+    print(f"[mixed] folded hexes p={p}", flush=True)
+    F, Z = [], []
+    for prec in (dgx.DGX_FP64, dgx.DGX_MIXED):
+        d, x = _folded(p, prec)
+        for out, amp in ((F, 0.1), (Z, 0.0)):
+            d.upload(_wave(x, amp))
+            out.append(d.rhs(dgx.DGX_MODAL))
+        d.close()
+    err = np.linalg.norm(F[1] - F[0]) / np.linalg.norm(F[0])
+    free = [np.linalg.norm(z) / np.linalg.norm(F[0]) for z in Z]
+    print(f"[mixed] folded hexes p={p}: residual rel L2 {err}, free stream {free}", flush=True)
+    assert err <= 1.05 * FOLDED[p], err
+    assert free[1] <= 1.5 * free[0], free
