@@ -59,3 +59,27 @@ def test_rhs_on_strongly_curved_hexes(eqn, p, a):
     assert np.all(err <= bar), err
     if a >= 0.05 and p >= 2:
         assert its > 8, its      # the slow path was taken
+
+
+@pytest.mark.parametrize("p,a", [(2, 0.004), (4, 0.004), (5, 0.002), (3, 0.1)])
+@pytest.mark.parametrize("power", [(-300, -400, -300, -400, -350), (300, 400, 300, 400, 350), (0, -300, 300, -400, 400)])
+def test_the_solve_does_not_depend_on_the_fields_scale(p, a, power):
+    """The projection of nodal data, its fields scaled by powers of two: scaling
+    is exact in every operation of the solve, so the modes are the unscaled ones
+    scaled, to the bit, if no stopping rule loses a field's squared norms (2^-800
+    to 2^800) to underflow or overflow.  By corrections alone at the small
+    twists, by conjugate gradients at the large one."""
+    print(f"[mass solve] scaled fields p={p} twist={a} powers {power}", flush=True)
+    m = meshgen.periodic_hexes(2, 2, 2)
+    gpu = dgx.GPUDomain(m, p, 8, xnodes=meshgen.mapped_nodes(m, p, _twist(a)))
+    U = _state(meshgen.hex_nodes(m, p))
+    scale = 2.0 ** np.array(power)[:, None, None]
+    gpu.upload(U)
+    ref = gpu.download(dgx.DGX_MODAL)
+    its = gpu.solver_iterations()
+    gpu.upload(U * scale)
+    got = gpu.download(dgx.DGX_MODAL)
+    print(f"[mass solve] {its} and {gpu.solver_iterations()} iterations", flush=True)
+    gpu.close()
+    assert np.array_equal(got / scale, ref), np.abs(got / scale - ref).max((1, 2))
+    assert (its <= 8) == (a < 0.1), its
