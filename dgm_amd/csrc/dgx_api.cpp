@@ -497,8 +497,8 @@ int stage3(dgx_domain *d, const double *X, const dgx::StageStep &st, bool traces
 // One LSRK stage of a curved hex domain: the traces (unless the previous stage
 // of this call wrote them), on Navier-Stokes the lifted gradients and viscous
 // terms, then k_rhs3c with the register update fused into its store (bitwise
-// the same as the residual followed by the axpby and axpy) and the traces of
-// the new state after it.
+// the same as the residual followed by the axpby and axpy) and, with a second
+// trace buffer, the traces of the new state after it.
 int step_curved3(dgx_domain *d, double A, double B, double dt, bool traces_ready) {
   int rc;
   if (!(traces_ready && d->t_of == d->U) && (rc = launch(d, dgx::OP_TRACES, d->U, nullptr))) return rc;
@@ -514,8 +514,8 @@ int step_curved3(dgx_domain *d, double A, double B, double dt, bool traces_ready
   ca.update = true; ca.Us = d->U; ca.Ut = d->Ut; ca.Tn = d->T2; ca.ca = A; ca.cb = B; ca.dt = dt;
   hipError_t e = timed(d, dgx::OP_RHS, [&] { return launch_curved(d, ca); });
   if (e != hipSuccess) return fail(DGX_ERR_DEVICE, std::string("curved stage: ") + hipGetErrorString(e));
-  std::swap(d->T, d->T2);        // the next stage's traces
-  d->t_of = d->U;
+  if (d->T2) std::swap(d->T, d->T2);   // the next stage's traces
+  d->t_of = d->T2 ? d->U : nullptr;
   ++d->stages;
   return DGX_OK;
 }
@@ -1076,7 +1076,7 @@ hipError_t launch_varp(const dgx_domain *d, int op, const double *in, double *ou
   return hipSuccess;
 }
 
-int build(dgx_domain *d, const dgx_domain_desc *desc) {
+int build(dgx_domain *d, const dgx_domain_desc *desc, bool spare) {
   const int nsd = desc->nsd, ne = desc->ne, p = desc->p;
   d->nsd = nsd; d->ne = ne; d->p = p;
   d->L = p + 1; d->Q = p + 2; d->QF = p + 1;
@@ -1383,9 +1383,9 @@ int build(dgx_domain *d, const dgx_domain_desc *desc) {
     if ((rc = alloc(&d->d_J, (size_t)ne + 3))) return rc;   // Jacobians, then the three means
     HIPCHK(hipMemcpy(d->d_J, d->J.data(), ne * sizeof(double), hipMemcpyHostToDevice));
   }
-  // a second trace buffer: the hex stages and those of affine quads write the
-  // next stage's traces into it
-  if ((d->fused || (d->nsd == 3 && d->curved) || (d->nsd == 2 && !d->curved && !desc->porder)) &&
+  // a second trace buffer: the stages of affine elements write the next stage's
+  // traces into it
+  if ((d->fused || (d->nsd == 2 && !d->curved && !desc->porder)) &&
       (rc = alloc(&d->T2, (size_t)ne * d->ns * d->nf * qs)))
     return rc;
   d->mixed = d->prec == DGX_MIXED;
@@ -1404,6 +1404,11 @@ int build(dgx_domain *d, const dgx_domain_desc *desc) {
     if ((rc = alloc(&d->TV, (size_t)ne * d->ns * (d->nf - 1) * qs))) return rc;
   }
   if (desc->porder && (rc = varp_setup(d, desc, sides))) return rc;
+  // curved hexes' stages too, where there is memory for it after all else
+  if (spare && dgx::spare_bytes(desc) && hipMalloc((void **)&d->T2, dgx::spare_bytes(desc) + 64) != hipSuccess) {
+    (void)hipGetLastError();
+    d->T2 = nullptr;
+  }
   return DGX_OK;
 }
 
@@ -1437,14 +1442,14 @@ int dgx_domain_bytes(const dgx_domain_desc *desc, size_t *bytes) {
   const bool fused = nsd == 3 && dgx::stage3_supported(desc->p) && !desc->xnodes;
   const bool mixed = desc->precision == DGX_MIXED;
   size_t b = 4 * nf * ne * nm * 8;                          // U, Ut, R0, R1
-  b += (fused || (nsd == 3 && desc->xnodes) || (nsd == 2 && !desc->porder) ? 2 : 1) * ne * ns * nf * qs * 8;   // face traces
+  b += (fused || (nsd == 2 && !desc->porder) ? 2 : 1) * ne * ns * nf * qs * 8 + dgx::spare_bytes(desc);   // face traces
   if (visc) {
     const size_t w = mixed ? 4 : 8;
     if (!fused && !mixed) b += ne * (nsd == 2 ? 6 : 12) * nm * 8;
     b += ne * (nf - 1) * (desc->xnodes ? nq : nm) * w + ne * ns * (nf - 1) * qs * w;
   }
   b += nf * ne * nq * 8;                                    // nodal transfer buffer
-  b += ne * (9 + 4 * ns) * 8 + ne * ns * (4 + 4 + 4 + 1);   // geometry and links
+  b += ne * (9 + 4 * ns) * 8 + ne * ns * (4 + 4 + (nsd == 2 ? 4 : 0) + 1);   // geometry and links
   b += 8 * qs * 2 + (size_t)(1 << 20);                      // orientation tables, tables, rounding
   const bool fns = desc->bc_function || desc->source;
   if (desc->xnodes || fns || !all_quads_affine(desc))   // curved: nodal metrics, face geometry
@@ -1465,6 +1470,19 @@ int dgx_domain_bytes(const dgx_domain_desc *desc, size_t *bytes) {
 }
 
 int dgx_domain_create(const dgx_domain_desc *desc, void *stream, dgx_handle *out) {
+  return dgx::domain_create(desc, stream, out, true);
+}
+
+}  // extern "C"
+
+namespace dgx {
+
+size_t spare_bytes(const dgx_domain_desc *desc) {
+  const size_t QF = desc->p + 1;
+  return desc->nsd == 3 && desc->xnodes ? (size_t)desc->ne * 30 * QF * QF * sizeof(double) : 0;
+}
+
+int domain_create(const dgx_domain_desc *desc, void *stream, dgx_handle *out, bool spare) {
   if (!desc || !out) return fail(DGX_ERR_ARGUMENT, "null argument");
   *out = nullptr;
   if (desc->nsd != 2 && desc->nsd != 3) return fail(DGX_ERR_ARGUMENT, "nsd must be 2 or 3");
@@ -1567,11 +1585,15 @@ int dgx_domain_create(const dgx_domain_desc *desc, void *stream, dgx_handle *out
     if (hipStreamCreate(&d->stream) != hipSuccess) { delete d; return fail(DGX_ERR_DEVICE, "hipStreamCreate failed"); }
     d->own_stream = true;
   }
-  int rc = build(d, desc);
+  int rc = build(d, desc, spare);
   if (rc) { release(d); delete d; return rc; }
   *out = d;
   return DGX_OK;
 }
+
+}  // namespace dgx
+
+extern "C" {
 
 int dgx_domain_destroy(dgx_handle h) {
   if (!h) return DGX_OK;

@@ -571,7 +571,7 @@ k_rhs3c(CurvedArgs a, const double *__restrict__ gm, const double *__restrict__ 
     }
   }
   if (tid == 0 && a.iters) atomicMax(a.iters, it);
-  if (PROJ || !a.update) return;
+  if (PROJ || !a.update || !a.Tn) return;
   // face traces of the updated state for the next stage
   static_assert(10 * QF * cmax(LP, 3 * L) + 15 * QF2 <= S::SZ && 20 * L * LP + 15 * L2 <= S::SZ, "trace buffers");
   __syncthreads();

@@ -94,6 +94,11 @@ struct dgx_domain {
 };
 
 namespace dgx {
+// dgx_domain_create; spare: with the memory a domain can do without
+// (spare_bytes: a curved hex domain's second trace buffer, without which each
+// stage evaluates its traces in a launch of its own), if there is enough.
+int domain_create(const dgx_domain_desc *desc, void *stream, dgx_handle *out, bool spare);
+size_t spare_bytes(const dgx_domain_desc *desc);
 // CFL evaluation of a 2D domain (dgx_api.cpp): the largest idt of
 // Euler::set_time_step with `part` (ne + 1 doubles of device memory) as the
 // kernels' scratch, waiting for the domain's stream; and the step rule.

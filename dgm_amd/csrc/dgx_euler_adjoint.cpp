@@ -51,7 +51,7 @@ struct dgx_euler_adjoint {
   double *lamU = nullptr, *lamT = nullptr, *Lt = nullptr, *SB = nullptr, *TB = nullptr;
   std::vector<double *> snaps;
   int rec_step = -1;       // the step whose stage states the next advance records
-  int have_step = -1;      // the step whose stage states SB and their traces TB hold
+  int have_step = -1;      // the step whose stage states SB and (where there is memory for them) traces TB hold
   long long fwd_steps = 0, adj_steps = 0;
   int snaps_used = 0;
 
@@ -126,24 +126,23 @@ int vjp(dgx_euler_adjoint *a, const double *U, const double *T, double *lam, dou
 
 // forward step k: state_k (in the domain's U) -> state_{k+1}.  The step to be
 // reversed next runs through the stage buffers, which then hold its stage
-// states and their traces.
+// states and, with TB, their traces.
 int step_forward(dgx_euler_adjoint *a, int k) {
   dgx_domain *d = a->dom;
   const size_t n = a->n(), nt = a->nt();
-  const bool record = k == a->rec_step;
+  const bool record = k == a->rec_step, keep = record && a->TB;
   int rc;
   if (record) HIPCHK(hipMemcpyAsync(a->SB, d->U, n * 8, hipMemcpyDeviceToDevice, d->stream));
-  if (record && a->t_valid) HIPCHK(hipMemcpyAsync(a->TB, d->T, nt * 8, hipMemcpyDeviceToDevice, d->stream));
-  else if (!a->t_valid && (rc = traces(a, d->U, record ? a->TB : d->T))) return rc;
+  if (keep && a->t_valid) HIPCHK(hipMemcpyAsync(a->TB, d->T, nt * 8, hipMemcpyDeviceToDevice, d->stream));
+  else if (!a->t_valid && (rc = traces(a, d->U, keep ? a->TB : d->T))) return rc;
   for (int s = 0; s < kStages; ++s) {
     const bool last = s == kStages - 1;
-    if (record)
-      rc = stage(a, s, a->SB + s * n, a->TB + s * nt, last ? d->U : a->SB + (s + 1) * n,
-                 last ? d->T : a->TB + (s + 1) * nt);
-    else
-      rc = stage(a, s, d->U, d->T, d->U, d->T2);
+    const double *X = record ? a->SB + s * n : d->U;
+    double *Xn = record && !last ? a->SB + (s + 1) * n : d->U;
+    if (keep) rc = stage(a, s, X, a->TB + s * nt, Xn, last ? d->T : a->TB + (s + 1) * nt);
+    else rc = stage(a, s, X, d->T, Xn, d->T2);
     if (rc) return rc;
-    if (!record) std::swap(d->T, d->T2);
+    if (!keep) std::swap(d->T, d->T2);
   }
   a->t_valid = true;
   if (record) a->have_step = k;
@@ -162,8 +161,11 @@ int step_adjoint(dgx_euler_adjoint *a, int k) {
     o.d = a->d_data + (size_t)k * a->nrec;
     HIPCHK(dgx::launch_pobs2_adj(o));
   }
+  if (!a->TB) a->t_valid = false;
   for (int s = kStages - 1; s >= 0; --s) {
-    int rc = vjp(a, a->SB + s * n, a->TB + s * a->nt(), a->lamT, a->lamU, s);
+    int rc;
+    if (!a->TB && (rc = traces(a, a->SB + s * n, a->dom->T))) return rc;
+    rc = vjp(a, a->SB + s * n, a->TB ? a->TB + s * a->nt() : a->dom->T, a->lamT, a->lamU, s);
     if (rc) return rc;
   }
   a->have_step = -1;
@@ -269,12 +271,15 @@ int dgx_euler_adjoint_create(const dgx_domain_desc *mesh, const dgx_euler_adjoin
       hipMalloc((void **)&a->d_y, nobs * 8) != hipSuccess || hipMalloc((void **)&a->d_data, nobs * 8) != hipSuccess ||
       hipMalloc((void **)&a->d_J, 8) != hipSuccess || hipMalloc((void **)&a->lamU, n * 8) != hipSuccess ||
       hipMalloc((void **)&a->lamT, n * 8) != hipSuccess || hipMalloc((void **)&a->Lt, nlt * 8) != hipSuccess ||
-      hipMalloc((void **)&a->SB, kStages * n * 8) != hipSuccess ||
-      hipMalloc((void **)&a->TB, kStages * nlt * 8) != hipSuccess)
+      hipMalloc((void **)&a->SB, kStages * n * 8) != hipSuccess)
     return fail_mem("Euler adjoint buffers");
   a->snaps.assign(a->nsnap, nullptr);
   for (int s = 0; s < a->nsnap; ++s)
     if (hipMalloc((void **)&a->snaps[s], n * 8) != hipSuccess) return fail_mem("checkpoint slots");
+  if (hipMalloc((void **)&a->TB, kStages * a->nt() * 8) != hipSuccess) {   // after all that is needed
+    (void)hipGetLastError();
+    a->TB = nullptr;
+  }
   hipStream_t st = d->stream;
   if (a->nrec > 0) {
     (void)hipMemcpyAsync(a->d_rec_e, rec_e.data(), a->nrec * sizeof(int), hipMemcpyHostToDevice, st);
@@ -291,6 +296,14 @@ int dgx_euler_adjoint_destroy(dgx_euler_adjoint_handle a) {
   (void)hipStreamSynchronize(a->dom->stream);
   release(a);
   delete a;
+  return DGX_OK;
+}
+
+int dgx_euler_adjoint_release_traces(dgx_euler_adjoint_handle a) {
+  if (!a) return fail(DGX_ERR_ARGUMENT, "null handle");
+  HIPCHK(hipStreamSynchronize(a->dom->stream));
+  if (a->TB) HIPCHK(hipFree(a->TB));
+  a->TB = nullptr;
   return DGX_OK;
 }
 

@@ -225,7 +225,7 @@ struct CurvedArgs {
   bool update = false;
   bool mixed = false;                        // hexes: FP32 residual arithmetic before the FP64 mass solve
   double *Us = nullptr, *Ut = nullptr;
-  double *Tn = nullptr;                      // update: the face traces of the new state
+  double *Tn = nullptr;                      // update: if set, the face traces of the new state go here
   double ca = 0.0, cb = 0.0, dt = 0.0;
   hipStream_t stream = nullptr;
 };

@@ -54,6 +54,7 @@ struct Request {
   int done_steps = 0, inflight_steps = 0, slices = 0;
   bool inflight = false;
   size_t bytes = 0, state_len = 0;
+  bool spare = true;           // dgx::domain_create
   dgx_handle h = nullptr;
   hipStream_t stream = nullptr;
   hipEvent_t ev = nullptr;
@@ -125,7 +126,7 @@ int admit(dgx_server *s, Request *r) {
   if (hipStreamCreate(&r->stream) != hipSuccess) return sfail(DGX_ERR_DEVICE, "hipStreamCreate failed");
   if (hipEventCreateWithFlags(&r->ev, hipEventDisableTiming) != hipSuccess)
     return sfail(DGX_ERR_DEVICE, "hipEventCreate failed");
-  int rc = dgx_domain_create(&r->desc, r->stream, &r->h);
+  int rc = dgx::domain_create(&r->desc, r->stream, &r->h, r->spare);
   if (rc) return sfail(rc, dgx_last_error());
   int qtot, nm, nf, ne;
   if ((rc = dgx_sizes(r->h, &qtot, &nm, &nf, &ne))) return sfail(rc, dgx_last_error());
@@ -344,6 +345,10 @@ int dgx_server_submit(dgx_server_handle s, const dgx_domain_desc *desc, const do
   auto r = std::make_unique<Request>();
   int rc = dgx_domain_bytes(desc, &r->bytes);
   if (rc) return sfail(rc, dgx_last_error());
+  if (r->bytes > s->cfg.hbm_budget && dgx::spare_bytes(desc)) {   // fits without what it can do without?
+    r->spare = false;
+    r->bytes -= dgx::spare_bytes(desc);
+  }
   if (r->bytes > s->cfg.hbm_budget) return sfail(DGX_ERR_ARGUMENT, "request exceeds the memory budget on its own");
   const size_t nv = (size_t)desc->ne * desc->nsd * (desc->nsd == 2 ? 4 : 8);
   r->vert.assign(desc->vert, desc->vert + nv);

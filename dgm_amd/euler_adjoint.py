@@ -37,6 +37,7 @@ def _bind(lib):
         "dgx_euler_adjoint_create": ([ctypes.POINTER(dgx.DomainDesc), ctypes.POINTER(EulerAdjointDesc), h,
                                       ctypes.POINTER(h)], ctypes.c_int),
         "dgx_euler_adjoint_destroy": ([h], ctypes.c_int),
+        "dgx_euler_adjoint_release_traces": ([h], ctypes.c_int),
         "dgx_euler_adjoint_forward": ([h, dp, dp, dp], ctypes.c_int),
         "dgx_euler_adjoint_gradient": ([h, dp, dp, dp, dp], ctypes.c_int),
         "dgx_euler_adjoint_vjp": ([h, dp, dp, dp], ctypes.c_int),
@@ -91,6 +92,10 @@ class EulerAdjointProblem:
             self.close()
         except Exception:
             pass
+
+    def release_traces(self):
+        """Gives the memory of the stage states' face traces back."""
+        _check(self.lib, self.lib.dgx_euler_adjoint_release_traces(self.h))
 
     def _state(self, U, what="state"):
         u = np.ascontiguousarray(U, dtype=np.float64)

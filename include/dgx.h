@@ -295,7 +295,10 @@ int dgx_profile(dgx_handle h, int inttype, double dt, int nsteps, double *ms, in
 
 /* Device bytes a domain built from `desc` holds (state, RK registers,
  * traces, viscous terms, nodal transfer buffer, geometry), without building
- * it.  Used for admission against a memory budget. */
+ * it.  Used for admission against a memory budget.  Counted in them is the
+ * second trace buffer of curved hexes (30 ne (p+1)^2 doubles), which such a
+ * domain does without where it does not fit the device or a server's budget
+ * (the same results, one launch more a stage). */
 int dgx_domain_bytes(const dgx_domain_desc *desc, size_t *bytes);
 
 /* ---------------------------------------------------------------------------
@@ -453,10 +456,16 @@ typedef struct {
  * Jacobian; the Roe flux's is assembled from forward-mode derivatives of the
  * same formula), DGX_FP64, periodic parallelogram quads (no boundary rows,
  * xnodes, functions or porder).  Allocates nsnap + 20 states of
- * 4 x ne x (p+1)^2 doubles. */
+ * 4 x ne x (p+1)^2 doubles and, where the device has them left after that,
+ * 14 x 16 x ne x (p+1) for the face traces of a reversed step's stage states. */
 int dgx_euler_adjoint_create(const dgx_domain_desc *mesh, const dgx_euler_adjoint_desc *ad, void *stream,
                              dgx_euler_adjoint_handle *out);
 int dgx_euler_adjoint_destroy(dgx_euler_adjoint_handle a);
+
+/* Gives the memory of the stage states' face traces back (as after a create
+ * that did not get it): gradients keep their bits, and a reversed stage takes
+ * one launch more. */
+int dgx_euler_adjoint_release_traces(dgx_euler_adjoint_handle a);
 
 /* Forward solve from U0 (host); y[nsteps][nrec] receives the observations and
  * UT the final modal state (host memory, each may be NULL).  Returns

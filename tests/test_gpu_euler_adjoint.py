@@ -255,3 +255,16 @@ def test_reo_opt_problem_descends():
     print(f"[euler-adjoint] descent: J {J0:.6e} -> {J:.6e}", flush=True)
     assert J < J0
     prob.close()
+
+
+def test_gradient_without_the_stage_traces_has_the_same_bits():
+    """Where the device has no memory for the stage states' face traces, each
+    reversed stage evaluates them again."""
+    mesh, orc, Uh, rec, prob = _setup()
+    data = prob.forward(Uh * (1.0 + 0.01 * np.random.default_rng(5).standard_normal(Uh.shape)))[0]
+    J, g = prob.gradient(Uh, data)
+    prob.release_traces()
+    for _ in range(2):
+        J2, g2 = prob.gradient(Uh, data)
+        assert J2 == J and np.array_equal(g2, g)
+    prob.close()

@@ -227,3 +227,42 @@ def test_oversized_request_rejected():
     with pytest.raises(dgx.DgxError):
         srv.submit(**job)
     srv.close()
+
+
+def test_curved_hexes_are_served_within_the_memory_they_need():
+    """A curved request that fits the budget only without its second trace
+    buffer is accepted, keeps to the budget and has the same bits; without more
+    than that it is refused."""
+    import ctypes
+    p, steps = 3, 6
+    m = meshgen.periodic_hexes(3, 3, 3, (0.0,) * 3, (2 * np.pi,) * 3)
+    xn = np.ascontiguousarray(meshgen.mapped_nodes(
+        m, p, lambda x, y, z: (x, y + 0.1 * np.sin(x), z + 0.1 * np.sin(y))))
+    U = np.ascontiguousarray(ic.taylor_green(*xn))
+    lib = serve._bind(dgx.load())
+    desc, keep = serve._desc(m, p, dgx.DGX_EULER3D, 1.4, 0.0, 0.72, 0, dgx.DGX_FP64)
+    desc.xnodes = xn.ctypes.data_as(ctypes.POINTER(ctypes.c_double))
+    need = ctypes.c_size_t()
+    assert lib.dgx_domain_bytes(ctypes.byref(desc), ctypes.byref(need)) == 0
+    spare = 30 * m.ne * (p + 1) ** 2 * 8
+
+    def submit(srv):
+        rid = ctypes.c_longlong()
+        rc = lib.dgx_server_submit(srv.h, ctypes.byref(desc), U.ctypes.data_as(ctypes.POINTER(ctypes.c_double)),
+                                   dgx.DGX_NODAL, dgx.DGX_LSRK14, 1e-3, steps, ctypes.byref(rid))
+        return rc, rid.value
+
+    got = []
+    for budget in (need.value, need.value - spare):
+        srv = serve.Server(hbm_budget=budget, max_active=1, steps_per_slice=4)
+        rc, rid = submit(srv)
+        assert rc == 0, lib.dgx_last_error()
+        srv.requests[rid] = serve.Request(rid, 5, m.ne, (p + 2) ** 3, dgx.DGX_NODAL)
+        srv.run_until_done(timeout_s=60.0)
+        got.append(srv.result(rid)[0])
+        assert srv.peak()[0] == budget
+        srv.close()
+    assert np.array_equal(got[0], got[1])
+    srv = serve.Server(hbm_budget=need.value - spare - 1, max_active=1)
+    assert submit(srv)[0] == -1   # DGX_ERR_ARGUMENT
+    srv.close()
