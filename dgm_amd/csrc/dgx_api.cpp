@@ -229,6 +229,40 @@ HostBasis make_basis(int p) {
     b.NV[i] = (double)(normleg(L, z[i]) / sqrtl(nn));
     b.NV[Q + i] = (double)(w[i] * normleg(L, z[i]) / sqrtl(nn));
   }
+  // halves of the symmetric matrices (dgx_device.hpp: EOx), rounded once
+  auto rows = [&](int nr, int ni, int odd, auto M) {     // points -> modes
+    for (int l = 0; l < nr; ++l) {
+      const ld s = (l + odd) % 2 ? -1 : 1;
+      for (int i = 0; i < dgx::half_up(ni); ++i) b.half.push_back((double)((M(l, i) + s * M(l, ni - 1 - i)) / 2));
+    }
+  };
+  auto square = [&](int no, int ni, auto M) {            // points -> points
+    for (int o = 0; o < dgx::half_up(no); ++o) {
+      for (int i = 0; i < dgx::half_up(ni); ++i)
+        b.half.push_back((double)(2 * i + 1 == ni ? M(o, i) : (M(o, i) + M(o, ni - 1 - i)) / 2));
+      for (int i = 0; i < ni / 2; ++i) b.half.push_back((double)((M(o, i) - M(o, ni - 1 - i)) / 2));
+    }
+  };
+  rows(L, Q, 0, [&](int l, int i) { return normleg(l, z[i]) * w[i]; });                  // BW
+  rows(L, Q, 1, [&](int l, int k) {                                                       // QD
+    ld s = 0;
+    for (int i = 0; i < Q; ++i) s += normleg(l, z[i]) * w[i] * Dl[i * Q + k];
+    return s;
+  });
+  rows(L, Q, 0, [&](int l, int i) {                                                       // PI
+    ld s = 0;
+    for (int a = 0; a < QF; ++a) s += wg[a] * normleg(l, zg[a]) * lagrange(z, i, zg[a]);
+    return s;
+  });
+  rows(L, Q, 0, [&](int l, int i) { return normleg(l, z[i]); });                          // BL
+  rows(L, QF, 0, [&](int l, int a) { return wg[a] * normleg(l, zg[a]); });                // PW
+  square(QF, Q, [&](int a, int i) { return lagrange(z, i, zg[a]); });                     // Ig
+  square(Q, QF, [&](int i, int a) {                                                       // GL
+    ld s = 0;
+    for (int l = 0; l < L; ++l) s += normleg(l, z[i]) * wg[a] * normleg(l, zg[a]);
+    return s;
+  });
+  square(Q, Q, [&](int i, int j) { return Dl[i * Q + j]; });                              // D
   return b;
 }
 
@@ -246,24 +280,8 @@ int upload_all_tables() {
       std::copy(t->begin(), t->end(), packed.begin() + off);
       off += t->size();
     }
-    // halves of the symmetric matrices (dgx_device.hpp: EOx)
-    auto rows = [&](const std::vector<double> &M, int nr, int ni, int odd) {   // points -> modes
-      for (int l = 0; l < nr; ++l) {
-        const double s = (l + odd) % 2 ? -1.0 : 1.0;
-        for (int i = 0; i < dgx::half_up(ni); ++i)
-          packed[off++] = 0.5 * (M[l * ni + i] + s * M[l * ni + ni - 1 - i]);
-      }
-    };
-    auto square = [&](const std::vector<double> &M, int no, int ni) {          // points -> points
-      for (int o = 0; o < dgx::half_up(no); ++o) {
-        for (int i = 0; i < dgx::half_up(ni); ++i)
-          packed[off++] = 2 * i + 1 == ni ? M[o * ni + i] : 0.5 * (M[o * ni + i] + M[o * ni + ni - 1 - i]);
-        for (int i = 0; i < ni / 2; ++i) packed[off++] = 0.5 * (M[o * ni + i] - M[o * ni + ni - 1 - i]);
-      }
-    };
-    const int L = b.L, Q = b.Q, QF = b.QF;
-    rows(b.BW, L, Q, 0); rows(b.QD, L, Q, 1); rows(b.PI, L, Q, 0); rows(b.BL, L, Q, 0); rows(b.PW, L, QF, 0);
-    square(b.Ig, QF, Q); square(b.GL, Q, QF); square(b.D, Q, Q);
+    std::copy(b.half.begin(), b.half.end(), packed.begin() + off);
+    off += b.half.size();
     if (off != (size_t)dgx::tab_offset(p) + dgx::tab_size(p)) return fail(DGX_ERR_ARGUMENT, "table layout");
   }
   hipError_t e;
