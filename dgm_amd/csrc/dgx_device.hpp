@@ -114,9 +114,10 @@ __device__ __forceinline__ void eo_apply(const T *__restrict__ h, const T (&x)[N
     }
   } else {
     T xe[HI], xo[FI > 0 ? FI : 1];
-    // a derivative takes no notice of a constant, but the FP32 sums would round
-    // relative to it: they act on the differences to the middle entry
-    constexpr bool diff = sizeof(T) == 4 && (K == EO_NMA || K == EO_NNA);
+    // a derivative takes no notice of a constant, but FP32 sums would round
+    // relative to it: the nodal derivatives of the mixed curved hexes act on the
+    // differences to the middle entry
+    constexpr bool diff = sizeof(T) == 4 && K == EO_NNA;
     const T c = diff ? x[FI] : T(0);
 #pragma unroll
     for (int i = 0; i < FI; ++i) {
