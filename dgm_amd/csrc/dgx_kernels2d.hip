@@ -74,19 +74,16 @@ __device__ __forceinline__ void load_traces2(const double *__restrict__ U, doubl
   quad_traces<P, NF, EPW, R, TT>(M, K, T, e0, ne, tid);
 }
 
-// TT: the tables (CT<P> for Navier-Stokes, see k_quad2).
-template <int P, class TT, typename R = double>
+// TT: the tables (CT<P> for Navier-Stokes, see k_quad2).  EPW as for the stage;
+// LDS for the traces alone.  With every mesh packed and the whole stage's block
+// (42 KB at p = 10, three wavefronts a CU) a residual of Euler quads took 6.84 us
+// on 32^2 at p = 2, 47.6 us on 256^2 at p = 2, 58.9 us on 64^2 at p = 10; now
+// 6.57, 38.8 and 45.5.
+template <int P, int EPW, int NF, class TT, typename R>
 __global__ void __launch_bounds__(64)
-k_traces2(const double *__restrict__ U, double *__restrict__ T, int ne, int nf) {
-  if (nf == 3) {
-    constexpr int E = quad_epw(P, 3);
-    __shared__ R sm[Q2S<P, 3, E>::size];
-    load_traces2<P, 3, E, TT, R>(U, T, ne, blockIdx.x * E, sm);
-  } else {
-    constexpr int E = quad_epw(P, 4);
-    __shared__ R sm[Q2S<P, 4, E>::size];
-    load_traces2<P, 4, E, TT, R>(U, T, ne, blockIdx.x * E, sm);
-  }
+k_traces2(const double *__restrict__ U, double *__restrict__ T, int ne) {
+  __shared__ R sm[Q2S<P, NF, EPW>::traces];
+  load_traces2<P, NF, EPW, TT, R>(U, T, ne, blockIdx.x * EPW, sm);
 }
 
 // One stage of an affine domain (quad_stage): EQ 0 Euler, 1 Navier-Stokes with
@@ -375,7 +372,7 @@ k_observe_adjoint(const double *__restrict__ U, double *__restrict__ Ubar, const
 template <int P, int E, int NF, typename R = double>
 __global__ void __launch_bounds__(64)
 k_batch_traces2(const Batch2 *__restrict__ b, int nreq, int nwork) {
-  __shared__ R sm[Q2S<P, NF, E>::size];
+  __shared__ R sm[Q2S<P, NF, E>::traces];
   int r = 0;
   for (int w = blockIdx.x; w < nwork; w += gridDim.x) {
     while (r + 1 < nreq && b[r + 1].off <= w) ++r;
@@ -581,21 +578,28 @@ static hipError_t launch_quad2(const LaunchArgs &a, const StageStep &s, double *
   return a.ns ? launch_quad2_e<P, double, 1>(a, s, Tn) : launch_quad2_e<P, double, 0>(a, s, Tn);
 }
 
+template <int P, int EPW, int NF, class TT, typename R>
+static hipError_t launch_traces2_k(const LaunchArgs &a) {
+  hipLaunchKernelGGL((k_traces2<P, EPW, NF, TT, R>), dim3((a.ne + EPW - 1) / EPW), dim3(64), 0, a.stream, a.U, a.T,
+                     a.ne);
+  return hipGetLastError();
+}
+
+template <int P, int NF, class TT, typename R>
+static hipError_t launch_traces2(const LaunchArgs &a) {
+  constexpr int E = quad_epw(P, NF);
+  return quad_packed(P, a.ne) ? launch_traces2_k<P, E, NF, TT, R>(a) : launch_traces2_k<P, 1, NF, TT, R>(a);
+}
+
 template <int P>
 static hipError_t launch2(const LaunchArgs &a) {
   const int ne = a.ne;
   switch (a.op) {
-    case OP_TRACES: {
-      const int E = quad_epw(P, a.nfield), grid = (ne + E - 1) / E;
+    case OP_TRACES:
       if (a.mixed)
-        hipLaunchKernelGGL((k_traces2<P, TE<float, P>, float>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne,
-                           a.nfield);
-      else if (a.ns)
-        hipLaunchKernelGGL((k_traces2<P, CT<P>>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
-      else
-        hipLaunchKernelGGL((k_traces2<P, EO<P>>), dim3(grid), dim3(64), 0, a.stream, a.U, a.T, ne, a.nfield);
-      break;
-    }
+        return a.nfield == 3 ? launch_traces2<P, 3, TE<float, P>, float>(a) : launch_traces2<P, 4, TE<float, P>, float>(a);
+      if (a.ns) return launch_traces2<P, 4, CT<P>, double>(a);
+      return a.nfield == 3 ? launch_traces2<P, 3, EO<P>, double>(a) : launch_traces2<P, 4, EO<P>, double>(a);
     case OP_RHS: {
       StageStep s;
       s.Xn = a.R;

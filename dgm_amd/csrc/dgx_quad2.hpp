@@ -28,6 +28,7 @@ template <int P, int NF, int EPW> struct Q2S {
   // M [EF][L2] modal; X1, X2 [EF][Q][L]; N1, N2 [EF][Q2] nodal state, fluxes
   // (N1 later the traces' end values [EF][4][L]); gF [EF][4][QF]; H [EF][4][L]
   static constexpr int size = NM + 2 * NX + 2 * NN + EF * 4 * QF + EF * 4 * L;
+  static constexpr int traces = NM + EF * 4 * L;         // of which the traces alone need M and the end values
   static_assert(NFP <= NT, "one face point per lane");
   static_assert(4 * L <= Q2, "the end values fit in N1");
 };
