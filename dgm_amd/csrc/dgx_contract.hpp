@@ -7,10 +7,6 @@
 
 namespace dgx {
 
-// Default thread count of the fused hex kernels' templates, for sizes that do not
-// depend on it; the kernels name their own (hex_threads, mixed_threads).
-constexpr int kStageThreads = 256;
-
 constexpr int round64(int n) { return (n + 63) / 64 * 64; }
 // Wavefronts per SIMD that the LDS of workgroups of nt threads allows, at
 // most `most`: the register budget to ask the compiler for.

@@ -27,19 +27,14 @@ namespace dgx {
 
 // Float copies of the basis tables for the mixed residual (FP32 contractions
 // and derivatives; FP64 metrics, fluxes, state and the mass solve), filled
-// beside c_tab at upload.  TE3<R, P> and TB3<R, P> give the tables of
-// arithmetic type R.
+// beside c_tab at upload.  TE3<R, P> gives the even-odd tables of arithmetic
+// type R.
 static __constant__ float c_tabf3[kTabTotal];
 struct EoBaseF3 {
   using R = float;
   __device__ static __forceinline__ const float *base() { return c_tabf3; }
 };
 template <typename R, int P> using TE3 = EOx<std::conditional_t<std::is_same<R, double>::value, EoBaseD, EoBaseF3>, P>;
-template <typename R, int P> struct TB3;
-template <int P> struct TB3<double, P> : CT<P> {};
-template <int P> struct TB3<float, P> {
-  __device__ static __forceinline__ const float *DN() { return c_tabf3 + (CT<P>::DN() - c_tab); }
-};
 
 template <int P> struct C3 {
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1;

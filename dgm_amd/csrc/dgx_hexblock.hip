@@ -15,12 +15,13 @@
 // LDS before it writes any of it.
 //
 // The sums run in ascending index order with separate multiplies and adds, so
-// the results are the same bits as a plain loop in that order.  The work is
-// HBM-bound: per element qtot doubles in and nm^3 out (or the reverse) against
-// qtot + 2 (nm qtot + nm^2 qb qc + nm^3 qc) flops, 3.2 flop/B at nm = 8,
-// q = 9, below MI355X's FP64 ridge of 9.8 flop/B.  The kernels stream elements
-// through a grid of resident workgroups (as many as fit on the chip), each
-// holding the three basis matrices in LDS for all of its elements.
+// the results are the same bits as a plain loop in that order.  Per element the
+// work is qtot doubles in and nm^3 out (or the reverse) and qtot + 2 (nm qtot +
+// nm^2 qb qc + nm^3 qc) flops, 3.2 flop/B at nm = 8, q = 9, below MI355X's FP64
+// ridge of 9.8 flop/B, so memory is the floor; what the wavefront kernels wait
+// for is the chain of one element's phases (HbW).  The kernels stream elements
+// through a grid of resident workgroups (as many as fit on the chip); the
+// generic ones hold the three basis matrices in LDS for all of their elements.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

@@ -21,20 +21,8 @@ namespace dgx {
 // Float copies of the basis tables for the mixed quad kernels, which hold
 // their LDS tensors and run their contractions in FP32 while the state, face
 // traces, LSRK registers and pointwise physics stay FP64; filled beside c_tab
-// at upload.  TB<R, P> gives the tables of arithmetic type R.
+// at upload.  TE<R, P> gives the even-odd tables of arithmetic type R.
 static __constant__ float c_tabf[kTabTotal];
-template <typename R, int P> struct TB;
-template <int P> struct TB<double, P> : CT<P> {};
-template <int P> struct TB<float, P> {
-  static constexpr int L = P + 1, Q = P + 2, QF = P + 1, b = tab_offset(P);
-  __device__ static __forceinline__ const float *BT() { return c_tabf + b; }
-  __device__ static __forceinline__ const float *BW() { return c_tabf + b + Q * L; }
-  __device__ static __forceinline__ const float *QD() { return c_tabf + b + 2 * Q * L; }
-  __device__ static __forceinline__ const float *Bg() { return c_tabf + b + 3 * Q * L; }
-  __device__ static __forceinline__ const float *Bend() { return c_tabf + b + 3 * Q * L + QF * L; }
-  __device__ static __forceinline__ const float *PW() { return c_tabf + b + 3 * Q * L + QF * L + 2 * L; }
-};
-
 struct EoBaseF {
   using R = float;
   __device__ static __forceinline__ const float *base() { return c_tabf; }

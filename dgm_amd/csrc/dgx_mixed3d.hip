@@ -45,8 +45,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 // ---------------------------------------------------------------------------
 constexpr int mq_size(int no, int n) { return ((no + 3) / 4) * 4 * ((n + 3) / 4 * 4); }
 constexpr int mq_order_size(int p) {
-  return mq_size(p + 2, p + 1) + 2 * mq_size(p + 1, p + 2) + mq_size(p + 1, p + 1) + mq_size(2, p + 1) +
-         mq_size(p + 1, p + 1) + mq_size(p + 1, p + 2) + mq_size(p + 1, p + 2) + mq_size(p + 2, p + 2) +
+  return mq_size(p + 2, p + 1) + mq_size(p + 1, p + 1) + 3 * mq_size(p + 1, p + 2) + mq_size(p + 2, p + 2) +
          mq_size(2, p + 2);
 }
 constexpr int mq_order_offset(int p) {
@@ -62,10 +61,7 @@ template <int P> struct MT {
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1;
   static constexpr int oBT = mq_order_offset(P);            // [Q][L]   modal -> GLL
   static constexpr int oBW = oBT + mq_size(Q, L);           // [L][Q]   GLL inner product
-  static constexpr int oQD = oBW + mq_size(L, Q);           // [L][Q]   inner product of D
-  static constexpr int oBg = oQD + mq_size(L, Q);           // [QF][L]  modal -> Gauss
-  static constexpr int oBend = oBg + mq_size(QF, L);        // [2][L]   modal -> +-1
-  static constexpr int oPW = oBend + mq_size(2, L);         // [L][QF]  Gauss inner product
+  static constexpr int oPW = oBW + mq_size(L, Q);           // [L][QF]  Gauss inner product
   static constexpr int oIg = oPW + mq_size(L, QF);          // [QF][Q]  GLL -> Gauss
   static constexpr int oPI = oIg + mq_size(QF, Q);          // [L][Q]   GLL face layer -> modal face
   static constexpr int oDN = oPI + mq_size(L, Q);           // [Q][Q]   GLL collocation derivative
@@ -175,7 +171,7 @@ __device__ __forceinline__ void mcon_last(int off, const float *in, float *out, 
   }
 }
 
-template <int P, int NTH = kStageThreads> struct M3 {
+template <int P, int NTH> struct M3 {
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1;
   static constexpr int L2 = L * L, L3 = L * L * L, Q2 = Q * Q, Q3 = Q * Q * Q, QF2 = QF * QF;
   static constexpr int LP = odd(L), QP = odd(Q), FP = odd(QF);
@@ -211,8 +207,8 @@ template <int P, int NTH = kStageThreads> struct M3 {
 // [NF][Q][L][L] (pitch LP), accumulated into the MFMA result registers:
 // acc[k][ob][r] += sum_i M[4ob+r][i] in[f][i][m][n] for the pencils
 // G = tid + k*NT = f*L2 + m*L + n.
-template <int P, int NF, int NS, int NTH = kStageThreads>
-__device__ __forceinline__ void mchain_to_regs(int off, const float *in, f4 (&acc)[NS][M3<P>::NOB],
+template <int P, int NF, int NS, int NTH>
+__device__ __forceinline__ void mchain_to_regs(int off, const float *in, f4 (&acc)[NS][M3<P, NTH>::NOB],
                                                int tid) {
   using S = M3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, L2 = S::L2, LP = S::LP, NT = S::NT, NOB = S::NOB;
@@ -236,7 +232,7 @@ __device__ __forceinline__ void mchain_to_regs(int off, const float *in, f4 (&ac
 
 // Collocation derivative along reference direction D of NF nodal fields in A
 // ([NF][Q][Q][Q], pitch QP), written (c, which comes first) or added to B.
-template <int P, int NF, int D, int NTH = kStageThreads>
+template <int P, int NF, int D, int NTH>
 __device__ __forceinline__ void mnodal_deriv(const float *A, float *B, int tid) {
   using S = M3<P, NTH>;
   constexpr int Q = S::Q, QP = S::QP, NT = S::NT, o = MT<P>::oDN;
@@ -248,8 +244,8 @@ __device__ __forceinline__ void mnodal_deriv(const float *A, float *B, int tid) 
 // Projection of NF nodal fields in B, accumulated into registers (the pencils
 // of mchain_to_regs); A is scratch.  Projecting the nodal divergence once
 // equals the three projected-derivative chains, with six contractions for nine.
-template <int P, int NF, int NS, int NTH = kStageThreads>
-__device__ __forceinline__ void mproj_to_regs(float *A, float *B, f4 (&acc)[NS][M3<P>::NOB], int tid) {
+template <int P, int NF, int NS, int NTH>
+__device__ __forceinline__ void mproj_to_regs(float *A, float *B, f4 (&acc)[NS][M3<P, NTH>::NOB], int tid) {
   using S = M3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT, o = MT<P>::oBW;
   mcon_last<NF * Q * Q, Q, L, QP, LP, NT>(o, B, A, tid);         // [NF Q Q][L]
@@ -307,7 +303,7 @@ __device__ __forceinline__ void mlifted_dir(const float *in, float *out, float *
 }
 
 // modal [NF][L][L][L] (pitch LP) in A -> nodal [NF][Q][Q][Q] (pitch QP) in B
-template <int P, int NF, int NTH = kStageThreads>
+template <int P, int NF, int NTH>
 __device__ __forceinline__ void mbackward(float *A, float *B, int tid) {
   using S = M3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT, o = MT<P>::oBT;
@@ -320,7 +316,7 @@ __device__ __forceinline__ void mbackward(float *A, float *B, int tid) {
 }
 
 // Face blocks g[NFB][QF][QF] (pitch FP) -> H[NFB][L][L] (pitch LP) in B, via A.
-template <int P, int NFB, int NTH = kStageThreads>
+template <int P, int NFB, int NTH>
 __device__ __forceinline__ void mface_project(const float *g, float *A, float *B, int tid) {
   using S = M3<P, NTH>;
   constexpr int L = S::L, QF = S::QF, LP = S::LP, FP = S::FP, NT = S::NT, o = MT<P>::oPW;
@@ -1111,14 +1107,10 @@ hipError_t upload_tables_m3d(const double *h) {
   for (int p = 1; p <= kMaxMixed; ++p) {
     const int L = p + 1, Q = p + 2, QF = p + 1;
     const double *t = h + tab_offset(p);
-    const double *BT = t, *BW = BT + Q * L, *QD = BW + L * Q, *Bg = QD + L * Q, *Bend = Bg + QF * L;
-    const double *PW = Bend + 2 * L, *Ig = PW + L * QF;
+    const double *BT = t, *BW = BT + Q * L, *PW = BW + 2 * L * Q + QF * L + 2 * L, *Ig = PW + L * QF;
     float *o = mq.data() + mq_order_offset(p);
     pack_mq(BT, Q, L, o); o += mq_size(Q, L);
     pack_mq(BW, L, Q, o); o += mq_size(L, Q);
-    pack_mq(QD, L, Q, o); o += mq_size(L, Q);
-    pack_mq(Bg, QF, L, o); o += mq_size(QF, L);
-    pack_mq(Bend, 2, L, o); o += mq_size(2, L);
     pack_mq(PW, L, QF, o); o += mq_size(L, QF);
     pack_mq(Ig, QF, Q, o); o += mq_size(QF, Q);
     const double *PI = Ig + QF * Q, *DN = PI + L * Q + 2 * Q + L * Q + Q * QF;

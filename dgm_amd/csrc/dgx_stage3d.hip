@@ -26,7 +26,7 @@
 
 namespace dgx {
 
-template <int P, int NTH = kStageThreads> struct S3 {
+template <int P, int NTH> struct S3 {
   static constexpr int L = P + 1, Q = P + 2, QF = P + 1;
   static constexpr int L2 = L * L, L3 = L * L * L, Q2 = Q * Q, Q3 = Q * Q * Q, QF2 = QF * QF;
   static constexpr int LP = odd(L), QP = odd(Q), FP = odd(QF);   // padded pitches
@@ -57,7 +57,7 @@ template <int P, int NTH = kStageThreads> struct S3 {
 // [NF][Q][L][L] (pitch LP), accumulated into registers:
 // acc[k][l] += sum_i M[l][i] in[f][i][m][n] for the thread's pencils
 // G = tid + k*NT = f*L2 + m*L + n.
-template <int P, int NF, int NS, int NTH = kStageThreads>
+template <int P, int NF, int NS, int NTH>
 __device__ __forceinline__ void chain_to_regs(EoMat<EO_NM, double> M, const double *in, double (&acc)[NS][P + 1],
                                               int tid) {
   using S = S3<P, NTH>;
@@ -83,7 +83,7 @@ __device__ __forceinline__ void chain_to_regs(EoMat<EO_NM, double> M, const doub
 // directions of the contravariant fluxes, B holds the nodal divergence, and
 // projecting it once (proj_to_regs) equals the three projected-derivative
 // chains: (BW D)_d (x) BW (x) BW = (BW (x) BW (x) BW)(D along d).
-template <int P, int NF, int D, bool ACC, int NTH = kStageThreads>
+template <int P, int NF, int D, bool ACC, int NTH>
 __device__ __forceinline__ void nodal_deriv(const double *A, double *B, int tid) {
   using S = S3<P, NTH>;
   constexpr int Q = S::Q, QP = S::QP, NT = S::NT;
@@ -95,7 +95,7 @@ __device__ __forceinline__ void nodal_deriv(const double *A, double *B, int tid)
 
 // Projection BW (x) BW (x) BW of NF nodal fields in B, accumulated into the
 // modal registers acc (the pencils of chain_to_regs); A is scratch.
-template <int P, int NF, int NS, int NTH = kStageThreads>
+template <int P, int NF, int NS, int NTH>
 __device__ __forceinline__ void proj_to_regs(double *A, double *B, double (&acc)[NS][P + 1], int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT;
@@ -108,7 +108,7 @@ __device__ __forceinline__ void proj_to_regs(double *A, double *B, double (&acc)
 }
 
 // modal [NF][L][L][L] (pitch LP) in A -> nodal [NF][Q][Q][Q] (pitch QP) in B
-template <int P, int NF, int NTH = kStageThreads>
+template <int P, int NF, int NTH>
 __device__ __forceinline__ void backward_batch(double *A, double *B, int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, Q = S::Q, LP = S::LP, QP = S::QP, NT = S::NT;
@@ -121,7 +121,7 @@ __device__ __forceinline__ void backward_batch(double *A, double *B, int tid) {
 }
 
 // Face blocks g[NFB][QF][QF] (pitch FP) -> H[NFB][L][L] (pitch LP) in B, via W in A.
-template <int P, int NFB, int NTH = kStageThreads>
+template <int P, int NFB, int NTH>
 __device__ __forceinline__ void face_project(const double *g, double *A, double *B, int tid) {
   using S = S3<P, NTH>;
   constexpr int L = S::L, QF = S::QF, LP = S::LP, FP = S::FP, NT = S::NT;
