@@ -427,7 +427,7 @@ def curved_sample(args, seed=5):
                         f"on top, periodic sides), p={p}, Mach 0.5 + 1e-3 seeded density noise, LSRK14, FP64",
             "value": value, "unit": "DOF-stage/s", "dofs": dofs, "steps": args.cv_steps, "dt": dt,
             "ms_per_step": el / args.cv_steps * 1e3, "setup_s": t_setup, "state_finite": finite,
-            "mass_solve_cg_iterations_max": cg_iters,
+            "mass_solve_applications_max": cg_iters,
             "mixed": {"value": dofs * 14 * args.cv_steps / elm, "speedup_vs_fp64": el / elm, "state_finite": finite_m,
                       "rel_l2_per_field_vs_fp64": err_f, "rel_l2_per_field_of_state_vs_fp64": err_w,
                       "after_steps": args.cv_steps + 1},
@@ -478,7 +478,7 @@ def curved_ns_sample(args, seed=6):
                         f"noise, LSRK14, FP64",
             "value": dofs * 14 * args.cvns_steps / el, "unit": "DOF-stage/s", "dofs": dofs,
             "steps": args.cvns_steps, "dt": dt, "ms_per_step": el / args.cvns_steps * 1e3, "setup_s": t_setup,
-            "state_finite": finite, "mass_solve_cg_iterations_max": cg}
+            "state_finite": finite, "mass_solve_applications_max": cg}
 
 
 def element_block_sample(args, seed=11):

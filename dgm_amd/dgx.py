@@ -226,7 +226,7 @@ class GPUDomain:
         return F
 
     def solver_iterations(self):
-        """Most conjugate-gradient iterations of a curved hex mass solve so far."""
+        """Most applications of the mass matrix in one solve of a curved hex so far."""
         it = ctypes.c_int()
         _check(self.lib.dgx_solver_iterations(self.h, ctypes.byref(it)))
         return it.value

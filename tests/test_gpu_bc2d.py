@@ -1,4 +1,4 @@
-"""Slip-wall and state boundaries of 2D Euler on the GPU (ghost2 in k_rhs2 and
+"""Slip-wall and state boundaries of 2D Euler on the GPU (ghost2 in k_quad2 and
 k_rhs2c) against the oracle's restatement of Euler::WallBC
 (src/EulerBC.hpp:43-62) and StateBC (src/BC.cpp:17-28).
 

@@ -187,7 +187,7 @@ def test_forward_matches_oracle_and_advance():
     dom.advance(dgx.DGX_LSRK14, prob.dt, prob.nsteps)
     ref = dom.download(dgx.DGX_MODAL)
     print(f"[euler-adjoint] final state vs dgx_advance: max abs diff {np.abs(UT - ref).max()}", flush=True)
-    assert np.array_equal(UT, ref)   # the same stage kernel (k_step2) in both
+    assert np.array_equal(UT, ref)   # the same stage kernel (k_quad2) in both
     dom.close()
     prob.close()
 

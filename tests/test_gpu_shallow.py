@@ -1,4 +1,4 @@
-"""Shallow water on the GPU (k_shallow2 behind the C ABI, eqntype 30) against
+"""Shallow water on the GPU (k_quad2 behind the C ABI, eqntype 30) against
 the oracle's restatement of Shallow::time_derivative (src/Shallow.cpp:251-525).
 
 Bar: relative L2 per field <= 1e-12 for one residual, <= 1e-11 after steps;
