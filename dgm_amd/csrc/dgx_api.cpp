@@ -155,7 +155,8 @@ ld normleg(int l, ld x) { ld P, dP; leg(l, x, P, dP); return P * sqrtl((2 * l + 
 
 using dgx::HostBasis;
 
-HostBasis make_basis(int p) {
+// halves: also the even-odd halves, which only the upload needs.
+HostBasis make_basis(int p, bool halves = false) {
   HostBasis b;
   b.p = p; b.L = p + 1; b.Q = p + 2; b.QF = p + 1;
   const int L = b.L, Q = b.Q, QF = b.QF;
@@ -229,6 +230,7 @@ HostBasis make_basis(int p) {
     b.NV[i] = (double)(normleg(L, z[i]) / sqrtl(nn));
     b.NV[Q + i] = (double)(w[i] * normleg(L, z[i]) / sqrtl(nn));
   }
+  if (!halves) return b;
   // halves of the symmetric matrices (dgx_device.hpp: EOx), rounded once
   auto rows = [&](int nr, int ni, int odd, auto M) {     // points -> modes
     for (int l = 0; l < nr; ++l) {
@@ -273,7 +275,7 @@ int upload_all_tables() {
   if (status == 0) return DGX_OK;
   std::vector<double> packed(dgx::kTabTotal, 0.0);
   for (int p = 1; p <= dgx::kMaxOrder; ++p) {
-    HostBasis b = make_basis(p);
+    HostBasis b = make_basis(p, true);
     size_t off = dgx::tab_offset(p);
     for (const std::vector<double> *t : {&b.BT, &b.BW, &b.QD, &b.Bg, &b.Bend, &b.PW, &b.Ig, &b.PI, &b.KE, &b.BL, &b.GL,
                                          &b.D, &b.NV}) {
