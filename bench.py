@@ -18,12 +18,11 @@ value = modal DOF x stages / wall time of the timed steps.
 Also printed in the same JSON line:
   roofline      the dominant kernel (largest share of a step's time, from HIP
                 events on the library's stream) against the compute roofline:
-                its algorithmic flops per launch / its mean launch time, against
-                MI355X's 78.6 TFLOP/s FP64 peak (157.3 TFLOP/s FP32 matrix for the
-                mixed path).  Algorithmic flops per DOF-stage at p = 7 (minimal
-                sum-factorized operator): 787 in all, 256 of them in the inviscid
-                residual kernel, the other 531 in the BR1 viscous kernel; BR2's
-                face pass adds 85 to the viscous kernel.
+                the flops it executes per launch (counted on the device in a
+                separate run) / its mean launch time, against MI355X's 78.6 TFLOP/s
+                FP64 peak (157.3 TFLOP/s FP32 matrix for the mixed path).  At p = 7
+                the FP64 kernels execute 249 flops per DOF-stage in the inviscid
+                residual, 429 in the BR1 viscous kernel and 498 with BR2's face pass.
                 `bound` is "valu" for the FP64 kernels (every flop on the FP64
                 vector pipe) and "mfma" for the mixed ones.  `traffic` is the
                 kernel's HBM bytes per launch measured with rocprofv3 FETCH_SIZE
@@ -76,20 +75,21 @@ FP32_MFMA_PEAK_TFLOPS = 157.3
 ARITHMETIC = {"fp64": "FP64 VALU (MI355X FP64 vector and matrix peaks are both 78.6 TFLOP/s)",
               "mixed": "FP32 MFMA contractions with FP64 pointwise work; peak is the FP32 matrix rate"}
 BYTES_PER_DOF_STAGE = 32.0
-# algorithmic flops per DOF-stage by kernel kind, per order (3D NS, BR1), of the
-# plain sums; the kernels' even-odd contractions and moments execute fewer.  BR2
-# adds its face pass to the viscous kernel: nodal face lifts (2 x 29,376 FMA),
-# the per-face-node correction (486 nodes x ~154 flops), the lift of the flux
-# difference (29,376 FMA) and its face sum (12,288 FMA) per element of 2,560 DOF
-FLOPS_PER_DOF_STAGE = {7: {"residual": 256.0, "visc": 531.0}}
-BR2_VISC_FLOPS = {7: 85.0}
+# flops the kernels execute per DOF-stage of the 3D NS operator at p = 7, counted
+# on the device (SQ_INSTS_VALU_FMA/ADD/MUL of F64 and F32 times 64 lanes, MFMA
+# tiles with their padding; profiles/tgv_ns3d_32cubed_p7_roe_br2.md): the even-odd
+# sums and the gradient's moments execute fewer than the plain sums' 787 (BR1)
+# keys: path, p, kernel kind, viscous scheme
+FLOPS_PER_DOF_STAGE = {("fp64", 7, "residual", "br1"): 249.0, ("fp64", 7, "residual", "br2"): 249.0,
+                       ("fp64", 7, "visc", "br1"): 429.0, ("fp64", 7, "visc", "br2"): 498.0,
+                       ("mixed", 7, "residual", "br2"): 456.0, ("mixed", 7, "visc", "br2"): 712.0}
 # HBM bytes per launch measured with rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE on
 # the 32^3 p=7 workload, scaled by the counters of a plain copy of known size
 # (profiles/tgv_ns3d_32cubed_p7_roe_br2.md, profiles/tgv_ns3d_32cubed_p7_lf_br1.md)
 # keys: path, n, p, kernel, flux, viscous scheme
-MEASURED_TRAFFIC = {("fp64", 32, 7, "visc", "roe", "br2"): 2.308e9, ("fp64", 32, 7, "residual", "roe", "br2"): 5.789e9,
-                    ("mixed", 32, 7, "visc", "roe", "br2"): 1.836e9, ("mixed", 32, 7, "residual", "roe", "br2"): 5.197e9,
-                    ("fp64", 32, 7, "visc", "lf", "br1"): 2.308e9, ("fp64", 32, 7, "residual", "lf", "br1"): 5.789e9}
+MEASURED_TRAFFIC = {("fp64", 32, 7, "visc", "roe", "br2"): 2.302e9, ("fp64", 32, 7, "residual", "roe", "br2"): 5.789e9,
+                    ("mixed", 32, 7, "visc", "roe", "br2"): 1.833e9, ("mixed", 32, 7, "residual", "roe", "br2"): 5.194e9,
+                    ("fp64", 32, 7, "visc", "lf", "br1"): 2.302e9, ("fp64", 32, 7, "residual", "lf", "br1"): 5.789e9}
 KINDS = ["traces", "residual", "grad", "visc", "forward", "backward", "update"]
 FLUXES = {"lf": dgx.DGX_FLUX_LF, "roe": dgx.DGX_FLUX_ROE}
 VISCOUS = {"br1": dgx.DGX_VISCOUS_BR1, "br2": dgx.DGX_VISCOUS_BR2}
@@ -592,13 +592,11 @@ def run_path(m, n, p, mu, precision, args, flux=None, viscous=None, compare=True
                        "ms_mean": (ms[k] / cnt[k]) if cnt[k] else 0.0} for k in range(7)}
     dom = max(kern, key=lambda k: kern[k]["ms_total"])
     mean_s = kern[dom]["ms_mean"] / 1e3
-    flops = FLOPS_PER_DOF_STAGE.get(p, {}).get(dom)
-    if flops is not None and dom == "visc" and viscous == "br2":
-        flops += BR2_VISC_FLOPS[p]
+    flops = FLOPS_PER_DOF_STAGE.get((name, p, dom, viscous))
     roofline = None
     if flops is not None:
-        algo_flops = flops * dofs
-        achieved = algo_flops / mean_s / 1e12
+        done_flops = flops * dofs
+        achieved = done_flops / mean_s / 1e12
         peak = FP64_PEAK_TFLOPS if precision == dgx.DGX_FP64 else FP32_MFMA_PEAK_TFLOPS
         # the FP64 kernels run every flop on the FP64 vector pipe (no MFMA); the
         # mixed kernels run their contractions on MFMA
@@ -609,7 +607,7 @@ def run_path(m, n, p, mu, precision, args, flux=None, viscous=None, compare=True
                                       "workload, scaled by a plain copy (profiles/tgv_ns3d_32cubed_p7_*.md), "
                                       "not measured in this run",
                     "kernel": dom, "arithmetic": ARITHMETIC[name],
-                    "algorithmic_flops_per_launch": algo_flops, "ms_mean": kern[dom]["ms_mean"]}
+                    "executed_flops_per_launch": done_flops, "ms_mean": kern[dom]["ms_mean"]}
     stage_s = sum(kern[k]["ms_total"] for k in kern) / 1e3 / (14 * prof_steps)
     algo_bytes = BYTES_PER_DOF_STAGE * dofs
     hbm = algo_bytes / stage_s / 1e9
